@@ -13,6 +13,7 @@
 
 #include "../../include/hfmm.h"
 #include "common.h"
+#include "p2p_math.h"
 
 namespace hfmm {
 namespace {
@@ -45,10 +46,11 @@ __global__ __launch_bounds__(256) void scratch_clear_kernel(double2* acc, int64_
 
 // grid (target tiles of 256, source chunks): each block stages its chunk's sources 256 at
 // a time in LDS (from the interleaved x, y, z array) and adds its partial sums to the
-// scratch accumulators with FP64 atomics
-__global__ __launch_bounds__(256) void direct_aos_kernel(const double* xyz, const double2* q, int64_t n, double k,
-                                                         const int64_t* targets, int64_t nt, int64_t chunk,
-                                                         double2* acc) {
+// scratch accumulators with FP64 atomics; kp is |k| / pi, conj (k < 0) takes the conjugate of
+// the |k| sum of the conjugate charges
+__global__ __launch_bounds__(256) void direct_aos_kernel(const double* xyz, const double2* q, int64_t n,
+                                                         nearfield::HalfTurnK kp, int conj, const int64_t* targets,
+                                                         int64_t nt, int64_t chunk, double2* acc) {
     __shared__ double sx[256], sy[256], sz[256], sqr[256], sqi[256];
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const bool valid = t < nt;
@@ -59,6 +61,7 @@ __global__ __launch_bounds__(256) void direct_aos_kernel(const double* xyz, cons
     const double x = xyz[3 * ti], y = xyz[3 * ti + 1], z = xyz[3 * ti + 2];
     const int64_t s0 = (int64_t)blockIdx.y * chunk, s1 = min(n, s0 + chunk);
     double ar = 0.0, ai = 0.0;
+    const nearfield::SinCosPi64 sp = nearfield::SinCosPi64::pinned();
     for (int64_t base = s0; base < s1; base += 256) {
         const int64_t v = base + threadIdx.x;
         if (v < s1) {
@@ -67,27 +70,24 @@ __global__ __launch_bounds__(256) void direct_aos_kernel(const double* xyz, cons
             sz[threadIdx.x] = xyz[3 * v + 2];
             const double2 qq = q[v];
             sqr[threadIdx.x] = qq.x;
-            sqi[threadIdx.x] = qq.y;
+            sqi[threadIdx.x] = conj ? -qq.y : qq.y;
         }
         __syncthreads();
         const int nb = (int)min((int64_t)256, s1 - base);
+#pragma unroll 2
         for (int j = 0; j < nb; ++j) {
             const double dx = x - sx[j], dy = y - sy[j], dz = z - sz[j];
-            const double r = sqrt(dx * dx + dy * dy + dz * dz);
-            if (r > 0.0) {
-                double s, c;
-                sincos(k * r, &s, &c);
-                const double wr = c / r, wi = s / r;
-                ar += wr * sqr[j] - wi * sqi[j];
-                ai += wr * sqi[j] + wi * sqr[j];
-            }
+            double wr, wi;
+            nearfield::pair_weight64(dx * dx + dy * dy + dz * dz, 0.0, kp, sp, wr, wi);
+            ar = fma(wr, sqr[j], fma(-wi, sqi[j], ar));
+            ai = fma(wr, sqi[j], fma(wi, sqr[j], ai));
         }
         __syncthreads();
     }
     if (valid) {
         if (!in_range) ar = ai = __builtin_nan("");
         atomicAdd(&acc[t].x, ar);
-        atomicAdd(&acc[t].y, ai);
+        atomicAdd(&acc[t].y, conj ? -ai : ai);
     }
 }
 
@@ -132,7 +132,8 @@ extern "C" int hfmm_direct_noalloc(const double* xyz, int64_t n, const double* q
         hipLaunchKernelGGL(scratch_clear_kernel, dim3((unsigned)tiles), dim3(256), 0, s, acc, n_targets);
         check_launch("scratch clear");
         hipLaunchKernelGGL(direct_aos_kernel, dim3((unsigned)tiles, (unsigned)nchunk), dim3(256), 0, s, xyz,
-                           (const double2*)q, n, k, targets, n_targets, chunk, acc);
+                           (const double2*)q, n, nearfield::halfturn_k(std::fabs(k)), k < 0.0 ? 1 : 0, targets, n_targets,
+                           chunk, acc);
         check_launch("direct (no allocation)");
         hipLaunchKernelGGL(scratch_copy_kernel, dim3((unsigned)tiles), dim3(256), 0, s, acc, n_targets,
                            (double2*)out);

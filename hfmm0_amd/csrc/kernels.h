@@ -116,6 +116,7 @@ struct P2PArgs {
     const double *X, *Y, *Z;      // sorted points (FP64)
     const double2* q;             // sorted charges (complex FP64)
     double k;                     // |k|
+    double kp_hi, kp_lo;          // |k| / pi in two terms (FP64 near field)
     double scale;                 // coordinate scale of the mixed kernel (set by the launcher)
     double wscale;                // factor of the mixed kernel's sums (set by the launcher)
     const double2* far;           // far field per sorted point
@@ -263,6 +264,7 @@ void launch_m2l_block(const M2LBlockArgs& a, int tb, int g, int fp32, hipStream_
 int m2l_block_persistent_grid(int p, int tb, int g, int fp32, size_t shm);
 // near field of one problem in a persistent batch launch
 constexpr int kP2PBatchTargetsPerLane = 2;
+constexpr int kP2PFp64TargetsPerLane = 2;   // FP64 near field: two independent chains per lane
 struct P2PBatchArgs {
     P2PArgs a;                    // scale and wscale set (p2p_scaled)
 };

@@ -850,38 +850,30 @@ __global__ __launch_bounds__(kXlateThreads) void xlate_kernel(XlateArgs a) {
 // ---------------------------------------------------------------------------------
 // P2P near field.
 // ---------------------------------------------------------------------------------
+using nearfield::HalfTurnK;
 using nearfield::radian_weight;
 using nearfield::radian_weight_phase64;
 
-template <typename T>
-struct P2PMath;
-
-template <>
-struct P2PMath<float> {
-    __device__ static inline void kernel(float r2, float k, float& wr, float& wi) { radian_weight(r2, k, wr, wi); }
-};
-
-template <>
-struct P2PMath<double> {
-    __device__ static inline void kernel(double r2, double k, double& wr, double& wi) {
-        const double r = sqrt(r2);
-        const double rinv = 1.0 / r;
-        double s, c;
-        sincos(k * r, &s, &c);
-        wr = c * rinv;
-        wi = s * rinv;
-    }
-};
-
 // e^{ikr}/r and the field weight (1 - ikr) e^{ikr}/r^3, so that
 // -grad_x e^{ik|x-y|}/|x-y| = (x - y) * field weight (HFMM.py:29-37 in complex form)
-template <typename T>
-__device__ inline void field_weights(T r2, T k, T& wr, T& wi, T& fr, T& fi) {
-    P2PMath<T>::kernel(r2, k, wr, wi);
-    const T rinv2 = (T)1 / r2;
-    const T kr = k * sqrt(r2);
+__device__ inline void field_weights(float r2, float k, float& wr, float& wi, float& fr, float& fi) {
+    radian_weight(r2, k, wr, wi);
+    const float rinv2 = 1.0f / r2;
+    const float kr = k * sqrtf(r2);
     fr = (wr + kr * wi) * rinv2;
     fi = (wi - kr * wr) * rinv2;
+}
+__device__ inline void field_weights64(double r2, double fl2, double k, HalfTurnK kp,
+                                       const nearfield::SinCosPi64& sp, double& wr, double& wi, double& fr,
+                                       double& fi) {
+    double c, s, rs, rinv, r;
+    nearfield::halfturn64(r2, kp, sp, c, s, rs, rinv, r);
+    rs = r2 > fl2 ? rs : 0.0;
+    wr = c * rs;
+    wi = s * rs;
+    const double kr = k * r, rinv2 = rinv * rinv;
+    fr = fma(kr, wi, wr) * rinv2;
+    fi = fma(-kr, wr, wi) * rinv2;
 }
 
 // Source staging of the near-field kernels: lane `lane` of a batch starting at `base`
@@ -1148,13 +1140,13 @@ __global__ __launch_bounds__(64) void p2p_mixed_kernel(P2PArgs a) {
     p2p_mixed_body<PH, LOWK, R>(a, a.leaf0 + xcd_leaf(blockIdx.x, gridDim.x), st);
 }
 
-// FP64 near field (the plain form): one wave per target leaf; targets of a chunk of up to
-// 64 points are spread over lane groups: with T' = next power of two >= chunk size, lane
-// l holds target l % T' and scans the sources j == l / T' (mod 64/T') of each 64-point
-// source batch staged in LDS (coordinates relative to the target leaf centre).  Lane-group
-// partial sums are combined with wavefront shuffles.  Sources of a leaf are a list of
-// point ranges (adjacent leaves, and the W/X interactions evaluated directly); pairs at or
-// below the leaf's coincidence floor are skipped.
+// FP64 near field (the plain form): one wave per target leaf on the schedule of the mixed form
+// (R targets per lane, G = 64 / L groups of lanes over the staged sources; coordinates relative
+// to the target leaf centre).  Pairs at or below the leaf's coincidence floor get the weight
+// zero.  Bound by the issue of its FP64 instructions, about 50 per pair with a v_rsq_f64: 350 G
+// pairs/s at N = 400k (9.3e8 pairs, leaves of about 98) against 172 with the device library's
+// sincos, square root and division (5.41 -> 2.65 ms).
+template <int R>
 __device__ __forceinline__ void p2p_fp64_body(const P2PArgs& a, const int leaf, P2PStage& st) {
     double *sx = st.fp64.x, *sy = st.fp64.y, *sz = st.fp64.z, *sqr = st.fp64.qr, *sqi = st.fp64.qi;
     const int b = a.leaf_box[leaf];
@@ -1163,19 +1155,26 @@ __device__ __forceinline__ void p2p_fp64_body(const P2PArgs& a, const int leaf, 
     const int r0 = a.rng_ptr[leaf], r1 = a.rng_ptr[leaf + 1];
     const int S = a.leaf_src_total[leaf];
     const double fl2 = a.floor2[leaf];
+    const HalfTurnK kp{a.kp_hi, a.kp_lo};
+    const nearfield::SinCosPi64 sp = nearfield::SinCosPi64::pinned();
     const int lane = threadIdx.x;
-    // target chunks of 64; a remainder of 33..63 targets goes as 32 + the rest, so that the
-    // lanes are not left idle with T' = 64 (each lane then scans half or less of the sources)
     for (int t0 = 0, tc = 0; t0 < tcnt; t0 += tc) {
-        tc = tcnt - t0 >= 64 ? 64 : min(32, tcnt - t0);
-        int Tp = 1;
-        while (Tp < tc) Tp <<= 1;
-        const int G = 64 / Tp;
-        const int ti = lane & (Tp - 1), g = lane / Tp;
-        const bool has_t = ti < tc;
-        const int it = tstart + t0 + (has_t ? ti : 0);
-        const double xt = a.X[it] - cx, yt = a.Y[it] - cy, zt = a.Z[it] - cz;
-        double sr = 0.0, si = 0.0;
+        tc = p2p_chunk<R>(tcnt - t0);
+        const int need = (tc + R - 1) / R;
+        int L = 1;
+        while (L < need) L <<= 1;
+        const int G = 64 / L;
+        const int li = lane & (L - 1), g = lane / L;
+        double xt[R], yt[R], zt[R], sr[R], si[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int it = tstart + t0 + min(li + r * L, tc - 1);
+            xt[r] = a.X[it] - cx;
+            yt[r] = a.Y[it] - cy;
+            zt[r] = a.Z[it] - cz;
+            sr[r] = 0.0;
+            si[r] = 0.0;
+        }
         int ri = r0;
         for (int base = 0; base < S; base += 64) {
             const int v = base + lane;
@@ -1191,36 +1190,46 @@ __device__ __forceinline__ void p2p_fp64_body(const P2PArgs& a, const int leaf, 
             __syncthreads();
             const int nb = min(64, S - base);
             for (int j = g; j < nb; j += G) {
-                const double dx = xt - sx[j], dy = yt - sy[j], dz = zt - sz[j];
-                const double r2 = dx * dx + dy * dy + dz * dz;
-                if (r2 > fl2) {
+                const double xs = sx[j], ys = sy[j], zs = sz[j], qr = sqr[j], qi = sqi[j];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const double dx = xt[r] - xs, dy = yt[r] - ys, dz = zt[r] - zs;
+                    const double r2 = dx * dx + dy * dy + dz * dz;
                     double wr, wi;
-                    P2PMath<double>::kernel(r2, a.k, wr, wi);
-                    const double qr = sqr[j], qi = sqi[j];
-                    sr += wr * qr - wi * qi;
-                    si += wr * qi + wi * qr;
+                    nearfield::pair_weight64(r2, fl2, kp, sp, wr, wi);
+                    sr[r] = fma(wr, qr, fma(-wi, qi, sr[r]));
+                    si[r] = fma(wr, qi, fma(wi, qr, si[r]));
                 }
             }
             __syncthreads();
         }
-        for (int off = Tp; off < 64; off <<= 1) {
-            sr += __shfl_xor(sr, off);
-            si += __shfl_xor(si, off);
-        }
-        if (g == 0 && has_t) {
-            double2 f = a.far[it];
-            f.x += sr;
-            f.y += si;
-            if (a.out_mode & 1) f.y = -f.y;   // k < 0: conjugate of the |k| result
-            if (a.out_mode & 2) f.y = 0.0;    // k == 0 with real charges: the result is real
-            a.out[a.perm[it]] = f;
+        for (int off = L; off < 64; off <<= 1)
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                sr[r] += __shfl_xor(sr[r], off);
+                si[r] += __shfl_xor(si[r], off);
+            }
+        if (g == 0) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int ti = li + r * L;
+                if (ti < tc) {
+                    const int it = tstart + t0 + ti;
+                    double2 f = a.far[it];
+                    f.x += sr[r];
+                    f.y += si[r];
+                    if (a.out_mode & 1) f.y = -f.y;   // k < 0: conjugate of the |k| result
+                    if (a.out_mode & 2) f.y = 0.0;    // k == 0 with real charges: the result is real
+                    a.out[a.perm[it]] = f;
+                }
+            }
         }
     }
 }
 
 __global__ __launch_bounds__(64) void p2p_fp64_kernel(P2PArgs a) {
     __shared__ P2PStage st;
-    p2p_fp64_body(a, a.leaf0 + xcd_leaf(blockIdx.x, gridDim.x), st);
+    p2p_fp64_body<kP2PFp64TargetsPerLane>(a, a.leaf0 + xcd_leaf(blockIdx.x, gridDim.x), st);
 }
 
 // Persistent near field over the leaves of many problems (batches), one launch per leaf
@@ -1239,7 +1248,7 @@ __global__ __launch_bounds__(64) void p2p_persistent_kernel(const P2PBatchArgs* 
         const int prob = __builtin_amdgcn_readfirstlane(wk.x), leaf = __builtin_amdgcn_readfirstlane(wk.y);
         const P2PArgs a = args[prob].a;
         if constexpr (CLS == kP2PClassFp64)
-            p2p_fp64_body(a, leaf, st);
+            p2p_fp64_body<kP2PFp64TargetsPerLane>(a, leaf, st);
         else if constexpr (CLS == kP2PClassLowK)
             p2p_mixed_body<false, true, kP2PBatchTargetsPerLane>(a, leaf, st);
         else if constexpr (CLS == kP2PClassPhase32)
@@ -1258,7 +1267,7 @@ __global__ __launch_bounds__(64) void p2p_field_kernel(int leaf0, const int* lea
                                                        const int* rng_ptr, const int* rng_start, const int* rng_pref,
                                                        const int* leaf_src_total, const double* floor2,
                                                        const double* X, const double* Y, const double* Z,
-                                                       const double2* q, double k, const double2* far,
+                                                       const double2* q, double k, HalfTurnK kp, const double2* far,
                                                        const double2* far_e, const int* perm, int out_mode,
                                                        double2* out, double2* field) {
     // coordinates relative to the leaf centre and r^2 in FP64 at every precision: FP32
@@ -1277,6 +1286,7 @@ __global__ __launch_bounds__(64) void p2p_field_kernel(int leaf0, const int* lea
     const double fl2 = floor2[leaf];
     const int lane = threadIdx.x;
     const T kk = (T)k;
+    const nearfield::SinCosPi64 sp = nearfield::SinCosPi64::pinned();
     // target chunks of 64; a remainder of 33..63 targets goes as 32 + the rest, so that the
     // lanes are not left idle with T' = 64 (each lane then scans half or less of the sources)
     for (int t0 = 0, tc = 0; t0 < tcnt; t0 += tc) {
@@ -1314,16 +1324,18 @@ __global__ __launch_bounds__(64) void p2p_field_kernel(int leaf0, const int* lea
             for (int j = g; j < nb; j += G) {
                 const C dx = xt - sx[j], dy = yt - sy[j], dz = zt - sz[j];
                 const C r2 = dx * dx + dy * dy + dz * dz;
-                if (r2 > fl2) {
+                if (std::is_same<T, double>::value || r2 > fl2) {   // FP64: zero weights at the floor
                     T wr, wi, fr, fi;
-                    if constexpr (PH) {
+                    if constexpr (std::is_same<T, double>::value) {
+                        field_weights64(r2, fl2, k, kp, sp, wr, wi, fr, fi);
+                    } else if constexpr (PH) {
                         float rinv, kr;
                         radian_weight_phase64(r2, k, wr, wi, rinv, kr);
                         const float rinv2 = rinv * rinv;
                         fr = (wr + kr * wi) * rinv2;
                         fi = (wi - kr * wr) * rinv2;
                     } else {
-                        field_weights<T>((T)r2, kk, wr, wi, fr, fi);
+                        field_weights((T)r2, kk, wr, wi, fr, fi);
                     }
                     const T qr = sqr[j], qi = sqi[j];
                     acc[0] += wr * qr - wi * qi;
@@ -1366,46 +1378,48 @@ __global__ __launch_bounds__(64) void p2p_field_kernel(int leaf0, const int* lea
 }
 
 // ---------------------------------------------------------------------------------
-// FP64 direct sum at sampled targets: grid (target tiles of 64, source chunks);
-// partial sums combined with FP64 atomics into a zeroed output.
+// FP64 direct sum at sampled targets: grid (target tiles of 256, source chunks);
+// partial sums combined with FP64 atomics into a zeroed output.  kp is |k| / pi; conj
+// (k < 0) takes the conjugate of the |k| sum of the conjugate charges.  Bound by FP64 issue:
+// 500 G pairs/s at 1M sources x 4096 targets, against 234 with the device library's sincos, square
+// root and division (17.5 -> 8.2 ms).
 // ---------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void direct_kernel(const double* X, const double* Y, const double* Z,
-                                                     const double2* q, int64_t n, double k, const double* tx,
-                                                     const double* ty, const double* tz, int64_t nt,
-                                                     int64_t chunk, double2* out) {
+                                                     const double2* q, int64_t n, HalfTurnK kp, int conj,
+                                                     const double* tx, const double* ty, const double* tz,
+                                                     int64_t nt, int64_t chunk, double2* out) {
     __shared__ double sx[256], sy[256], sz[256], sqr[256], sqi[256];
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const bool valid = t < nt;
     const double x = valid ? tx[t] : 0.0, y = valid ? ty[t] : 0.0, z = valid ? tz[t] : 0.0;
     const int64_t s0 = (int64_t)blockIdx.y * chunk, s1 = min(n, s0 + chunk);
     double ar = 0.0, ai = 0.0;
+    const nearfield::SinCosPi64 sp = nearfield::SinCosPi64::pinned();
     for (int64_t base = s0; base < s1; base += 256) {
         const int64_t v = base + threadIdx.x;
         if (v < s1) {
             sx[threadIdx.x] = X[v];
             sy[threadIdx.x] = Y[v];
             sz[threadIdx.x] = Z[v];
-            sqr[threadIdx.x] = q[v].x;
-            sqi[threadIdx.x] = q[v].y;
+            const double2 qq = q[v];
+            sqr[threadIdx.x] = qq.x;
+            sqi[threadIdx.x] = conj ? -qq.y : qq.y;
         }
         __syncthreads();
         const int nb = (int)min((int64_t)256, s1 - base);
+#pragma unroll 2
         for (int j = 0; j < nb; ++j) {
             const double dx = x - sx[j], dy = y - sy[j], dz = z - sz[j];
-            const double r = sqrt(dx * dx + dy * dy + dz * dz);
-            if (r > 0.0) {
-                double s, c;
-                sincos(k * r, &s, &c);
-                const double wr = c / r, wi = s / r;
-                ar += wr * sqr[j] - wi * sqi[j];
-                ai += wr * sqi[j] + wi * sqr[j];
-            }
+            double wr, wi;
+            nearfield::pair_weight64(dx * dx + dy * dy + dz * dz, 0.0, kp, sp, wr, wi);
+            ar = fma(wr, sqr[j], fma(-wi, sqi[j], ar));
+            ai = fma(wr, sqi[j], fma(wi, sqr[j], ai));
         }
         __syncthreads();
     }
     if (valid) {
         atomicAdd(&out[t].x, ar);
-        atomicAdd(&out[t].y, ai);
+        atomicAdd(&out[t].y, conj ? -ai : ai);
     }
 }
 
@@ -1542,19 +1556,20 @@ void launch_p2p_field(int precision, int n_leaves, int n_fp32, const int* leaf_b
                       double k, const double2* far, const double2* far_e, const int* perm, int out_mode,
                       double2* out, double2* field, hipStream_t s) {
     if (n_leaves <= 0) return;
+    const HalfTurnK kp = nearfield::halfturn_k(k);
     if (precision == 0) {
         hipLaunchKernelGGL((p2p_field_kernel<double, false>), dim3(n_leaves), dim3(64), 0, s, 0, leaf_box, bx,
-                           rng_ptr, rng_start, rng_pref, leaf_src_total, floor2, X, Y, Z, q, k, far, far_e, perm,
+                           rng_ptr, rng_start, rng_pref, leaf_src_total, floor2, X, Y, Z, q, k, kp, far, far_e, perm,
                            out_mode, out, field);
     } else {
         if (n_fp32 > 0)
             hipLaunchKernelGGL((p2p_field_kernel<float, false>), dim3(n_fp32), dim3(64), 0, s, 0, leaf_box, bx,
-                               rng_ptr, rng_start, rng_pref, leaf_src_total, floor2, X, Y, Z, q, k, far, far_e,
+                               rng_ptr, rng_start, rng_pref, leaf_src_total, floor2, X, Y, Z, q, k, kp, far, far_e,
                                perm, out_mode, out, field);
         if (n_leaves > n_fp32)
             hipLaunchKernelGGL((p2p_field_kernel<float, true>), dim3(n_leaves - n_fp32), dim3(64), 0, s, n_fp32,
                                leaf_box, bx, rng_ptr, rng_start, rng_pref, leaf_src_total, floor2, X, Y, Z, q, k,
-                               far, far_e, perm, out_mode, out, field);
+                               kp, far, far_e, perm, out_mode, out, field);
     }
     check_launch("p2p_field");
 }
@@ -1711,8 +1726,8 @@ void launch_direct(const double* X, const double* Y, const double* Z, const doub
     const int64_t chunk = (n + nchunk - 1) / nchunk;
     nchunk = (n + chunk - 1) / chunk;
     launch_fill_zero(out, nt, s);
-    hipLaunchKernelGGL(direct_kernel, dim3((unsigned)tiles, (unsigned)nchunk), dim3(256), 0, s, X, Y, Z, q, n, k, tx,
-                       ty, tz, nt, chunk, out);
+    hipLaunchKernelGGL(direct_kernel, dim3((unsigned)tiles, (unsigned)nchunk), dim3(256), 0, s, X, Y, Z, q, n,
+                       nearfield::halfturn_k(std::fabs(k)), k < 0.0 ? 1 : 0, tx, ty, tz, nt, chunk, out);
     check_launch("direct");
 }
 

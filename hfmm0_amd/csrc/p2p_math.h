@@ -1,8 +1,9 @@
-// Near-field kernel arithmetic: e^{ikr}/r (and the field weight) in FP32 from an FP64 r^2.
-// Compiled for the GPU by hipcc and for the host by g++ (the host build is how the error
-// bounds of these functions are tested without a GPU); the only difference is the
-// reciprocal square root: the GPU's v_rsq_f32 (about 1 ulp) on the device, 1/sqrtf on the
-// host (correctly rounded square root, then a correctly rounded division).
+// Near-field kernel arithmetic: e^{ikr}/r (and the field weight) from an FP64 r^2, in FP32 for
+// mixed plans and in FP64 for FP64 plans and the direct sum.  Compiled for the GPU by hipcc
+// and for the host by g++ (the host build is how the error bounds of these functions are
+// tested without a GPU); the only difference is the reciprocal square root: the GPU's
+// v_rsq_f32 (about 1 ulp) on the device, 1/sqrtf on the host (correctly rounded square root,
+// then a correctly rounded division), and in FP64 the estimate that both refine.
 #pragma once
 
 #include <cmath>
@@ -110,6 +111,104 @@ HFMM_HD inline void pair_weight(double r2, double fl2, float& wr, float& wi) {
     else
         halfturn_parts(fmaxf((float)r2, 0x1p-120f), c, s, rs);
     rs = ok ? rs : 0.0f;
+    wr = c * rs;
+    wi = s * rs;
+}
+
+// ---------------------------------------------------------------------------------
+// FP64 half-turn form (FP64 plans and the direct sum).
+// ---------------------------------------------------------------------------------
+
+// k / pi as an unevaluated sum of two FP64 values (relative error about 2^-105)
+struct HalfTurnK {
+    double hi, lo;
+};
+inline HalfTurnK halfturn_k(double k) {
+    const double pi_hi = 3.1415926535897931160, pi_lo = 1.2246467991473532072e-16;
+    const double hi = k / pi_hi;
+    return HalfTurnK{hi, (std::fma(-hi, pi_hi, k) - hi * pi_lo) / pi_hi};
+}
+
+// an estimate of x^-1/2 with relative error below 1e-6 (v_rsq_f64: measured 5.2e-8)
+HFMM_HD inline double rsq64_estimate(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_rsq(x);
+#else
+    return (1.0 / std::sqrt(x)) * (1.0 - 6e-8);   // the device's error, so that host tests see the correction work
+#endif
+}
+
+// 1/r and r from r2 = r^2 (a normal number).  With y the estimate and e = 1 - r2 y^2,
+// r^-1 = y (1 - e)^-1/2 = y (1 + e/2 + 3 e^2/8) up to 5 e^3 / 16 (e <= 2e-6: below 1e-17); r is
+// r2 / r with one correction from its residual.
+HFMM_HD inline void rsqrt64(double r2, double& rinv, double& r) {
+    const double y = rsq64_estimate(r2);
+    const double e = fma(-(r2 * y), y, 1.0);
+    rinv = fma(y * e, fma(e, 0.375, 0.5), y);
+    const double t = r2 * rinv;
+    r = fma(0.5 * rinv, fma(-t, t, r2), t);
+}
+
+// sin(pi y) and cos(pi y) for |y| <= 1/2: minimax polynomials (Remez, absolute error) of
+// degree 17 (odd) and 16 (even), generated by hfmm0_amd/csrc/sincos_remez.py;
+// approximation error with the binary64 coefficients 5.4e-17 (sin) and 1.2e-16 (cos).
+// The kernels hold the coefficients in scalar registers (`pinned`): FP64 FMAs take a scalar
+// addend, while the compiler left to itself keeps them in vector registers and copies one
+// before every step, since its accumulating FMA overwrites the addend.
+struct SinCosPi64 {
+    double s[9] = {3.14159265358979312e+00,  -5.16771278004996848e+00, 2.55016403987724116e+00,
+                   -5.99264529317457884e-01, 8.21458865532826710e-02,  -7.37043035602404084e-03,
+                   4.66299170571231986e-04,  -2.19020215213132668e-05, 7.68394041277779699e-07};
+    double c[9] = {1.0,
+                   -4.93480220054467633e+00, 4.05871212641649759e+00, -1.33526276884346462e+00,
+                   2.35330630129808288e-01,  -2.58068887393525410e-02, 1.92955628359191256e-03,
+                   -1.04566580734636122e-04, 4.14959170019500732e-06};
+    HFMM_HD static inline SinCosPi64 pinned() {
+        SinCosPi64 p;
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+        for (int i = 0; i < 9; ++i) asm("" : "+s"(p.s[i]));
+#pragma unroll
+        for (int i = 1; i < 9; ++i) asm("" : "+s"(p.c[i]));
+#endif
+        return p;
+    }
+};
+
+HFMM_HD inline void sincospi_half64(double y, const SinCosPi64& p, double& s, double& c) {
+    const double t = y * y;
+    double ps = fma(t, p.s[8], p.s[7]), pc = fma(t, p.c[8], p.c[7]);
+#pragma unroll
+    for (int i = 6; i >= 0; --i) {
+        ps = fma(t, ps, p.s[i]);
+        pc = fma(t, pc, p.c[i]);
+    }
+    s = y * ps;
+    c = pc;
+}
+
+// e^{ikr} = (-1)^n (c + i s) from r2 = r^2 > 0 in FP64: c = cos(pi y), s = sin(pi y), and rs
+// the signed 1/r, so that e^{ikr}/r is (c rs, s rs); also 1/r and r.  The reduction
+// y = r k/pi - n takes k/pi in two terms, so only its own rounding (2^-53 of n) and r's enter
+// the phase.  r^2 below the smallest normal number counts as that number.  Beyond
+// k r / pi = 2^50, where an FP64 k r carries an error of a radian, the phase stays that of
+// 2^50 (the parity trick needs integers below 2^51).
+HFMM_HD inline void halfturn64(double r2, HalfTurnK k, const SinCosPi64& sp, double& c, double& s, double& rs, double& rinv, double& r) {
+    rsqrt64(fmax(r2, 0x1p-1022), rinv, r);
+    const double p = fmin(r * k.hi, 0x1p50);
+    const double m = p + 6755399441055744.0;  // 1.5 * 2^52
+    const double n = m - 6755399441055744.0;
+    const double y = fmin(fma(r, k.lo, fma(r, k.hi, -n)), 0.5);
+    sincospi_half64(y, sp, s, c);
+    rs = __builtin_bit_cast(double, dbits(rinv) | (dbits(m) << 63));
+}
+
+// Weight of one pair in FP64, e^{ikr}/r, exactly zero at or below the floor fl2.
+HFMM_HD inline void pair_weight64(double r2, double fl2, HalfTurnK k, const SinCosPi64& sp, double& wr,
+                                  double& wi) {
+    double c, s, rs, rinv, r;
+    halfturn64(r2, k, sp, c, s, rs, rinv, r);
+    rs = r2 > fl2 ? rs : 0.0;
     wr = c * rs;
     wi = s * rs;
 }

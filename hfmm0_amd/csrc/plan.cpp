@@ -19,6 +19,7 @@
 #include "../../include/hfmm.h"
 #include "common.h"
 #include "kernels.h"
+#include "p2p_math.h"
 
 namespace hfmm {
 
@@ -1207,6 +1208,9 @@ P2PArgs p2p_args(const hfmm_plan& P, int out_mode, double2* out) {
     pa.Z = P.dZ;
     pa.q = P.d_q;
     pa.k = P.k;
+    const nearfield::HalfTurnK kp = nearfield::halfturn_k(P.k);
+    pa.kp_hi = kp.hi;
+    pa.kp_lo = kp.lo;
     pa.far = P.d_far;
     pa.perm = P.d_perm;
     pa.out_mode = out_mode;

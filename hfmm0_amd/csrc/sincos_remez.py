@@ -6,11 +6,14 @@ The near field evaluates e^{i pi u} for u = k r / pi, reduced to y = u - rint(u)
     sin(pi y) ~= y * S(y^2),   S of degree 4 in y^2 (odd polynomial of degree 9 in y),
     cos(pi y) ~= C(y^2),       C of degree 5 in y^2 (even polynomial of degree 10 in y),
 
+and in binary64 (the FP64 near field and direct sum) with S of degree 8 (odd, degree 17 in
+y) and C of degree 8 (even, degree 16),
+
 chosen by the Remez exchange algorithm (E. Ya. Remez, 1934; the second algorithm as in
 Cheney, "Introduction to Approximation Theory", ch. 3) for the smallest maximum ABSOLUTE
 error of sin(pi y) and cos(pi y) over y in [0, 1/2] (the polynomials are odd / even, so
 the bound holds on [-1/2, 1/2]).  Arithmetic in mpmath at 50 digits; the coefficients are
-then rounded to binary32.
+then rounded to binary32 (binary64).
 
 Run:  python hfmm0_amd/csrc/sincos_remez.py   (prints the C initialisers and the errors)
 """
@@ -93,6 +96,13 @@ def main():
     es = max(abs(y * mp.polyval([mp.mpf(f32(c)) for c in cs][::-1], y * y) - mp.sin(mp.pi * y)) for y in ys)
     ec = max(abs(mp.polyval([mp.mpf(f32(c)) for c in cc][::-1], y * y) - mp.cos(mp.pi * y)) for y in ys)
     print("max |error| with binary32 coefficients, exact arithmetic: sin %.3e, cos %.3e" % (es, ec))
+    cs = remez(fs, ws, 9, a, b)
+    cc = remez(fc, wc, 9, a, b)
+    print("FP64 sin coefficients (y, y^3, ..., y^17):", ", ".join("%.17e" % float(c) for c in cs))
+    print("FP64 cos coefficients (1, y^2, ..., y^16):", ", ".join("%.17e" % float(c) for c in cc))
+    es = max(abs(y * mp.polyval([mp.mpf(float(c)) for c in cs][::-1], y * y) - mp.sin(mp.pi * y)) for y in ys)
+    ec = max(abs(mp.polyval([mp.mpf(float(c)) for c in cc][::-1], y * y) - mp.cos(mp.pi * y)) for y in ys)
+    print("max |error| with binary64 coefficients, exact arithmetic: sin %.3e, cos %.3e" % (es, ec))
 
 
 if __name__ == "__main__":
