@@ -262,6 +262,66 @@ void launch_m2l_block(const M2LBlockArgs& a, int tb, int g, int fp32, hipStream_
 // (p = larger table degree, tb, g, fp32) with `shm` bytes of LDS, and the launch over the
 // device descriptors d_args and the queues q of (descriptor, item) work.
 int m2l_block_persistent_grid(int p, int tb, int g, int fp32, size_t shm);
+// FP64 translations with one wave per work item (m2l_wave64.hip).  Operators are stored as MFMA
+// A fragments: element (row i, column k) of a block sits in register k / 4, lane 16 (k % 4) + i.
+// Rotations, per theta: for n = 0, 1, ... the u block ((n+1) x (n+1)), then the v block (rows
+// m = 1..n in the forward table; rows m = 0..n, the first zero, in the back table; columns
+// m = 1..n), two registers per lane side by side.  Coaxial tables, per distance: for m = 0..P
+// registers m / 4 .. P / 4 (rows and columns are degrees), Re and Im per lane side by side.
+constexpr int kWave64MaxP = 14;
+constexpr int kWave64Pairs = 16;              // pairs per group
+// accumulator registers (four orders each) of degrees 0..p
+__host__ __device__ constexpr int wave64_regs(int p) {
+    int k = 0;
+    for (int n = 0; n <= p; ++n) k += n / 4 + 1;
+    return k;
+}
+__host__ __device__ constexpr int wave64_rot_regs(int n, int h) {   // register pairs before (n, h)
+    return 2 * n + (n > 8 ? n - 8 : 0) + (n > 9 ? n - 9 : 0) + (h ? (n >= 8 ? 2 : 1) : 0);
+}
+__host__ __device__ constexpr int wave64_coax_regs(int P, int m) {   // registers before order m
+    return m * (P / 4 + 1) - (4 * ((m / 4) * (m / 4 - 1) / 2) + (m % 4) * (m / 4));
+}
+// (S, D) buffers start with a block of zeros, the source of absent pairs, and end with padding
+// that the last box's gather may read past its entries
+__host__ __device__ constexpr int wave_sd_pad(int pmax) { return (pmax + 1) * (pmax + 2) / 2 + 8; }
+struct M2LWaveArgs {
+    int ps, pt;                      // effective source and target degrees
+    int overwrite;                   // store instead of add (every block in one item)
+    int n_items;
+    const int4* items;               // (block, first group, end group, part): part 0 is the whole
+                                     // block, s > 0 leaves its sums in slot s - 1 of `part`
+    int n_blocks;
+    double4* part;                   // partial sums of split blocks (null: none), per slot and
+                                     // accumulator register 4 tb values
+    const int* part_ptr;             // n_blocks + 1: the slots of each block
+    int tb;                          // targets per block, a power of two up to the pairs per group
+    const int* blk_targets;          // blocks x tb target boxes (-1: empty slot)
+    const int* grp_class;            // per group: theta | dist << 16
+    const int* grp_src;              // per pair of a group: source offset in (S, D) entries (no
+                                     // pair: 0, a block of zeros)
+    const unsigned short* grp_dir;   // per pair: direction
+    const double* rot1;              // fragments of E_n^T per theta (forward)
+    const double* rot3;              // fragments of E_n per theta (back)
+    int rot_stride;
+    const double2* phase;            // e^{i m phi} per direction
+    int phase_stride;
+    const double* coax;
+    int coax_stride;
+    const void* M;                   // (S, D) entries
+    double2* L;                      // expansions added to (x basis)
+    const int64_t* exp_off;
+};
+void launch_m2l_wave64(const M2LWaveArgs& a, int p, hipStream_t s);
+// workgroups that add the parts of one split block of tb targets
+int wave64_sum_chunks(int p, int tb);
+// many translations of degree p: work[i] = (descriptor, item), n a multiple of kXcds; sums[i] =
+// (descriptor, split block, chunk, 0)
+void launch_m2l_wave64_batch(const M2LWaveArgs* d_args, const int2* work, int n, const int4* sums, int n_sums, int p,
+                             hipStream_t s);
+// the expansions of n_boxes consecutive boxes of degree p as (S_re, S_im, D_re, D_im) entries
+void launch_to_sd64(const double2* x, double4* sd, int64_t n_boxes, int p, hipStream_t s);
+
 // near field of one problem in a persistent batch launch
 constexpr int kP2PBatchTargetsPerLane = 2;
 constexpr int kP2PFp64TargetsPerLane = 2;   // FP64 near field: two independent chains per lane

@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <array>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <functional>
@@ -71,6 +72,32 @@ struct M2LBlockLevel {
     int* zero = nullptr;
 };
 
+// items an M2L launch of the wave kernel is split into (m2l_wave64.hip)
+constexpr int kWaveItems = 3072;
+
+// FP64 translation of one level with one wave per work item (m2l_wave64.hip)
+struct M2LWaveLevel {
+    bool use = false;
+    int tb = 0;                    // targets per block
+    int ps = 0, pt = 0;            // table degrees
+    int src_level = 0, tgt_level = 0;
+    int n_items = 0;
+    int4* items = nullptr;
+    int* targets = nullptr;
+    int* cls = nullptr;
+    int* src = nullptr;
+    unsigned short* dir = nullptr;
+    std::vector<double> tab;       // packed coaxial tables (host): fragments are made per degree
+    int n_dist = 0;
+    double* coax = nullptr;        // fragments for the effective degrees
+    int coax_stride = 0;
+    int n_blocks = 0, n_slots = 0;
+    int* part_ptr = nullptr;
+    double4* part = nullptr;       // partial sums of blocks split over items, shared by the levels
+    int n_groups = 0;
+    std::vector<int> host_targets, host_ptr;   // plans of a batch: blocks and their groups
+};
+
 struct XlateLaunch {
     int n_targets = 0;
     int* targets = nullptr;
@@ -129,6 +156,13 @@ struct hfmm_plan {
     M2LBlockLevel m2lb[kMaxLevels];
     bool m2l_fp32[kMaxLevels] = {};  // M2L of the level in FP32 (mixed precision)
     M2LBlockLevel m2mb[kMaxLevels], l2lb[kMaxLevels];   // M2M / L2L on matrix cores
+    M2LWaveLevel m2lc[kMaxLevels], m2mc[kMaxLevels], l2lc[kMaxLevels];   // FP64, one wave per item
+    bool in_batch = false;           // evaluated by a batch only
+    std::vector<int64_t> sd_off;     // offset of each box's (S, D) entries
+    int64_t n_sd = 0;
+    double *d_cr1 = nullptr, *d_cr3 = nullptr;   // rotation fragments of the wave kernel
+    int cr_stride = 0;
+    double4 *dMs = nullptr, *dLs = nullptr;      // multipoles / parents' locals in (S, D) form
     int m2l_kernel = 0;
     int p2p_tile = 2;               // targets per lane of the mixed near field
     double p2p_coord32_tol = 0.0;   // estimated error up to which a leaf takes FP32 coordinates (<= 0: none)
@@ -339,6 +373,31 @@ std::vector<int4> make_items(const Tree& t, const std::vector<int>& blk_targets,
         const int chunk = std::max(1, (e1 - e0 + nsplit - 1) / nsplit);
         for (int s = e0; s < e1; s += chunk)
             items.push_back(make_int4(b, s, std::min(e1, s + chunk), nsplit > 1 ? 1 : 0));
+    }
+    while (items.size() % kXcds) items.push_back(make_int4(0, 0, 0, 0));
+    return items;
+}
+
+// Work items of the wave kernel: blocks in space order, each split into equal items of at most
+// per_item groups; part_ptr[b] .. part_ptr[b + 1] are the partial sum slots of block b (none for
+// a whole block).  Padded to a multiple of the XCD count.
+std::vector<int4> wave_items(const Tree& t, const std::vector<int>& blk_targets, const std::vector<int>& blk_ptr, int tb,
+                             int per_item, std::vector<int>& part_ptr) {
+    const int nblk = (int)blk_ptr.size() - 1;
+    std::vector<int> border(nblk);
+    for (int b = 0; b < nblk; ++b) border[b] = b;
+    std::stable_sort(border.begin(), border.end(), [&](int x, int y) {
+        return t.code[blk_targets[(size_t)x * tb]] >> 3 < t.code[blk_targets[(size_t)y * tb]] >> 3;
+    });
+    auto parts = [&](int b) { return std::max(1, (blk_ptr[b + 1] - blk_ptr[b] + per_item - 1) / per_item); };
+    part_ptr.assign(nblk + 1, 0);
+    for (int b = 0; b < nblk; ++b) part_ptr[b + 1] = part_ptr[b] + (parts(b) > 1 ? parts(b) : 0);
+    std::vector<int4> items;
+    for (int b : border) {
+        const int e0 = blk_ptr[b], n = blk_ptr[b + 1] - e0, np = parts(b);
+        for (int i = 0; i < np; ++i)
+            items.push_back(make_int4(b, e0 + (int)((int64_t)n * i / np), e0 + (int)((int64_t)n * (i + 1) / np),
+                                      np > 1 ? part_ptr[b] + i + 1 : 0));
     }
     while (items.size() % kXcds) items.push_back(make_int4(0, 0, 0, 0));
     return items;
@@ -579,6 +638,149 @@ void build_tree_blocks(hfmm_plan& P, int L, int kind, const std::vector<double>&
     prepare_m2l_block(pm, tb, grp, fp32);
 }
 
+// Coaxial fragments of a level for its effective degrees (m2l_wave64.hip), into B.coax
+void pack_wave_coax(const hfmm_plan& P, M2LWaveLevel& B) {
+    const int ps = P.p_eff[B.src_level], pt = P.p_eff[B.tgt_level], pm = std::max(ps, pt);
+    const int regs = wave64_coax_regs(pm, pm + 1), csz = coax_size(B.pt, B.ps);
+    B.coax_stride = regs * 128;
+    std::vector<double> cf((size_t)B.n_dist * B.coax_stride, 0.0);
+    for (int d = 0; d < B.n_dist; ++d) {
+        size_t off = (size_t)d * csz;
+        for (int m = 0; m <= std::min(B.ps, B.pt); ++m) {
+            const int lens = B.ps + 1 - m;
+            for (int n2 = m; n2 <= pt; ++n2)
+                for (int n = m; n <= ps; ++n) {
+                    const size_t t = off + (size_t)(n2 - m) * lens + n - m;
+                    double* f = &cf[(size_t)d * B.coax_stride +
+                                    ((size_t)(wave64_coax_regs(pm, m) + n / 4 - m / 4) * 64 + 16 * (n % 4) + n2) * 2];
+                    f[0] = B.tab[2 * t];
+                    f[1] = B.tab[2 * t + 1];
+                }
+            off += (size_t)(B.pt + 1 - m) * lens;
+        }
+    }
+    HIPCHK(hipMemcpy(B.coax, cf.data(), cf.size() * sizeof(double), hipMemcpyHostToDevice));
+}
+
+// Translation of one level on the wave kernel: targets with their (source, direction) lists.
+// kind 0: M2L, 1: M2M, 2: L2L; coax: packed tables as X.coax (interleaved complex).
+void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt_level, const std::vector<int>& targets,
+                   const std::vector<int>& ptr, const std::vector<int>& src, const std::vector<unsigned short>& dir,
+                   const std::vector<double>& coax, int n_dist, const std::vector<DispInfo>& dinfo) {
+    const int ps = P.p_level[src_level], pt = P.p_level[tgt_level], pm = std::max(ps, pt);
+    if (P.m2l_kernel != 0 || pm > kWave64MaxP || !P.d_cr1) return;
+    if (P.n_sd > INT_MAX) return;   // 32-bit source offsets
+    const Tree& t = P.tree;
+    const int nt = (int)targets.size();
+    constexpr int pairs = kWave64Pairs;
+    // classes (theta, dist) present, and the targets ordered by the octant's z bit, then in
+    // space: V displacements of one z bit have the same classes
+    std::vector<int> cls_of(kNumDirs, -1), cls_key;
+    {
+        std::map<std::pair<int, int>, int> ids;
+        for (unsigned short d : dir) ids.emplace(std::make_pair(dinfo[d].theta, dinfo[d].dist), 0);
+        for (auto& kv : ids) {
+            kv.second = (int)cls_key.size();
+            cls_key.push_back(kv.first.first | kv.first.second << 16);
+        }
+        for (int d = 0; d < kNumDirs; ++d) {
+            auto it = ids.find(std::make_pair(dinfo[d].theta, dinfo[d].dist));
+            if (it != ids.end()) cls_of[d] = it->second;
+        }
+    }
+    const int nc = (int)cls_key.size();
+    std::vector<int> order(nt);
+    for (int i = 0; i < nt; ++i) order[i] = i;
+    if (kind != 1)
+        std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+            return ((t.code[targets[x]] >> 2) & 1) < ((t.code[targets[y]] >> 2) & 1);
+        });
+    std::vector<unsigned short> cnt((size_t)nt * nc, 0);
+    for (int i = 0; i < nt; ++i)
+        for (int e = ptr[i]; e < ptr[i + 1]; ++e) ++cnt[(size_t)i * nc + cls_of[dir[e]]];
+    // targets per block: the one with the fewest groups (each is 16 pairs of work); on a tie the
+    // smaller, whose blocks are more and end in fewer stores
+    int tb = 0;
+    int64_t best = 0;
+    for (int c : {2, 4, 8, 16}) {
+        const int slots = pairs / c;
+        int64_t g = 0;
+        for (int b0 = 0; b0 < nt; b0 += c)
+            for (int k = 0; k < nc; ++k) {
+                int mx = 0;
+                for (int j = b0; j < std::min(nt, b0 + c); ++j) mx = std::max<int>(mx, cnt[(size_t)order[j] * nc + k]);
+                g += (mx + slots - 1) / slots;
+            }
+        if (!tb || g < best) tb = c, best = g;
+    }
+    // The kernel's code for one group is straight-line, 15 to 40 KB, and every compute unit
+    // fetches it once: a launch of a group or two per wave spends most of its time on that (M2M
+    // of 512 children at p = 10: 42 us, against 20 for the block kernel; M2L of 3096 pairs: 28
+    // against 53).  M2M and L2L take it from 2 groups per SIMD on.
+    if (kind != 0 && best < 2048) return;
+    const int slots = pairs / tb, nblk = (nt + tb - 1) / tb;
+    std::vector<int> blk_targets((size_t)nblk * tb, -1), blk_ptr{0}, gcls, gsrc;
+    std::vector<unsigned short> gdir;
+    gsrc.reserve((size_t)best * pairs);
+    gdir.reserve((size_t)best * pairs);
+    std::vector<int> first(nc + 1), fill(nc);
+    for (int b = 0; b < nblk; ++b) {
+        const int j0 = b * tb, j1 = std::min(nt, j0 + tb);
+        first[0] = (int)gcls.size();
+        for (int k = 0; k < nc; ++k) {
+            int mx = 0;
+            for (int j = j0; j < j1; ++j) mx = std::max<int>(mx, cnt[(size_t)order[j] * nc + k]);
+            const int g = (mx + slots - 1) / slots;
+            for (int i = 0; i < g; ++i) gcls.push_back(cls_key[k]);
+            first[k + 1] = first[k] + g;
+        }
+        gsrc.resize(gcls.size() * pairs, 0);
+        gdir.resize(gcls.size() * pairs, 0);
+        for (int j = j0; j < j1; ++j) {
+            const int i = order[j];
+            blk_targets[j] = targets[i];
+            std::fill(fill.begin(), fill.end(), 0);
+            for (int e = ptr[i]; e < ptr[i + 1]; ++e) {
+                const int k = cls_of[dir[e]], f = fill[k]++;
+                const size_t o = (size_t)(first[k] + f / slots) * pairs + (f % slots) * tb + (j - j0);
+                gsrc[o] = (int)P.sd_off[src[e]];
+                gdir[o] = dir[e];
+            }
+        }
+        blk_ptr.push_back((int)gcls.size());
+    }
+    B.use = true;
+    B.tb = tb;
+    B.ps = ps;
+    B.pt = pt;
+    B.src_level = src_level;
+    B.tgt_level = tgt_level;
+    B.targets = P.upload(blk_targets);
+    B.cls = P.upload(gcls);
+    B.src = P.upload(gsrc);
+    B.dir = P.upload(gdir);
+    B.tab = coax;
+    B.n_dist = n_dist;
+    B.coax = P.alloc<double>((size_t)n_dist * wave64_coax_regs(pm, pm + 1) * 128);
+    pack_wave_coax(P, B);
+    B.n_blocks = nblk;
+    B.n_groups = blk_ptr[nblk];
+    if (P.in_batch && kind == 0) {   // split once the groups of all problems are known
+        B.host_targets = std::move(blk_targets);
+        B.host_ptr = std::move(blk_ptr);
+        return;
+    }
+    // M2L blocks are split into items whose sums meet in a second kernel: three items for each
+    // wave that runs at a time (1024 SIMDs)
+    std::vector<int> part_ptr;
+    const std::vector<int4> items = wave_items(
+        t, blk_targets, blk_ptr, tb, kind == 0 ? std::max(1, (B.n_groups + kWaveItems - 1) / kWaveItems) : B.n_groups, part_ptr);
+    B.n_items = (int)items.size();
+    B.items = P.upload(items);
+    B.n_slots = part_ptr[nblk];
+    B.part_ptr = P.upload(part_ptr);
+}
+
 void build_tables(hfmm_plan& P) {
     const Tree& t = P.tree;
     // directions
@@ -747,6 +949,27 @@ void build_tables(hfmm_plan& P) {
         }
         P.d_rf1 = P.upload(f1);   // FP64: M2L, M2M and L2L of FP64 levels
         P.d_rf3 = P.upload(f3);
+        if (P.m2l_kernel == 0) {   // the wave kernel's fragments
+            const int pc = std::min(pmax, kWave64MaxP);
+            P.cr_stride = wave64_rot_regs(pc + 1, 0) * 128;
+            std::vector<double> c1((size_t)thetas.size() * P.cr_stride, 0.0), c3(c1.size(), 0.0);
+            for (size_t th = 0; th < thetas.size(); ++th)
+                for (int n = 0; n <= pc; ++n)
+                    for (int st = 0; st < 2; ++st) {
+                        rotation_uv_blocks(&rot[th * rsz + rot_offset(n)], n, st == 0, Wu, Wv);
+                        double* base = &(st == 0 ? c1 : c3)[th * P.cr_stride];
+                        auto at = [&](int h, int i, int k) -> double& {
+                            const int j = k / 4;
+                            return base[((size_t)(wave64_rot_regs(n, h) + j / 2) * 64 + 16 * (k % 4) + i) * 2 + (j & 1)];
+                        };
+                        for (int i = 0; i <= n; ++i)
+                            for (int k = 0; k <= n; ++k) at(0, i, k) = Wu[(size_t)i * (n + 1) + k];
+                        for (int i = 0; i < n; ++i)   // the back table's v rows are the orders 0..n
+                            for (int k = 0; k < n; ++k) at(1, st == 0 ? i : i + 1, k) = Wv[(size_t)i * n + k];
+                    }
+            P.d_cr1 = P.upload(c1);
+            P.d_cr3 = P.upload(c3);
+        }
     }
     std::vector<double2> phase((size_t)kNumDirs * (pmax + 1));
     for (int d = 0; d < kNumDirs; ++d)
@@ -800,7 +1023,9 @@ void build_tables(hfmm_plan& P) {
                 coax_table(0, G, P.k, 2.0 * P.h[L] * std::sqrt((double)dist_d2[i]), P.R[L], P.R[L], X.ps, X.pt,
                            &cx[i * X.coax_stride * 2]);
             X.coax = (double2*)P.upload(cx);
-            build_m2l_blocks(P, L, targets, ptr, src, dir, cx, (int)dist_d2.size(), dinfo);
+            if (!P.m2l_fp32[L])
+                build_waves(P, P.m2lc[L], 0, L, L, targets, ptr, src, dir, cx, (int)dist_d2.size(), dinfo);
+            if (!P.m2lc[L].use) build_m2l_blocks(P, L, targets, ptr, src, dir, cx, (int)dist_d2.size(), dinfo);
         }
     }
     // M2M (parent level L <- children at L+1) and L2L (parent level L -> children at L+1)
@@ -839,6 +1064,7 @@ void build_tables(hfmm_plan& P) {
         coax_table(1, G, P.k, P.R[L + 1], P.R[L + 1], P.R[L], A.ps, A.pt, cx.data());
         A.coax = (double2*)P.upload(cx);
         build_tree_blocks(P, L, 1, cx);
+        if (!P.m2mb[L].fp32) build_waves(P, P.m2mc[L], 1, L + 1, L, targets, ptr, src, dir, cx, 1, dinfo);
         XlateLaunch& B = P.l2l[L];
         B.n_targets = (int)ctargets.size();
         B.targets = P.upload(ctargets);
@@ -854,6 +1080,7 @@ void build_tables(hfmm_plan& P) {
         coax_table(2, G, P.k, P.R[L + 1], P.R[L], P.R[L + 1], B.ps, B.pt, cy.data());
         B.coax = (double2*)P.upload(cy);
         build_tree_blocks(P, L, 2, cy);
+        if (!P.l2lb[L].fp32) build_waves(P, P.l2lc[L], 2, L, L + 1, ctargets, cptr, csrc, cdir, cy, 1, dinfo);
     }
 }
 
@@ -964,6 +1191,21 @@ void build_p2p(hfmm_plan& P) {
     }
 }
 
+size_t wave_part_size(const M2LWaveLevel& B, int n_slots) {
+    return (size_t)n_slots * wave64_regs(std::max(B.ps, B.pt)) * 4 * B.tb;
+}
+
+// The partial sums of the wave kernel's split blocks: one buffer for all levels, which run one
+// after another
+void alloc_wave_parts(hfmm_plan& P) {
+    size_t most = 0;
+    for (const M2LWaveLevel& B : P.m2lc) most = std::max(most, wave_part_size(B, B.n_slots));
+    if (!most) return;
+    double4* all = P.alloc<double4>(most);
+    for (M2LWaveLevel& B : P.m2lc)
+        if (B.n_slots) B.part = all;
+}
+
 void build_plan(hfmm_plan& P, const double* xyz, int64_t n, double k, const hfmm_opts& o) {
     if (!std::isfinite(k)) fail(HFMM_ERR_ARG, "k must be a finite real number");
     if (n <= 0 || n > (int64_t)1 << 30) fail(HFMM_ERR_ARG, "positions must be a nonempty finite (N,3) array");
@@ -1044,6 +1286,7 @@ void build_plan(hfmm_plan& P, const double* xyz, int64_t n, double k, const hfmm
     }
     std::vector<double> centre(3 * (size_t)nb);
     P.exp_off.assign(nb, 0);
+    P.sd_off.assign(nb, 0);
     int64_t off = 0;
     for (int b = 0; b < nb; ++b) {
         int gx, gy, gz;
@@ -1055,6 +1298,9 @@ void build_plan(hfmm_plan& P, const double* xyz, int64_t n, double k, const hfmm
         centre[3 * b + 2] = gz * s + half + t.pmin[2];
         P.exp_off[b] = off;
         off += ncoef(P.p_level[t.level[b]]);
+        if (b == 0) P.n_sd = wave_sd_pad(P.pmax);
+        P.sd_off[b] = P.n_sd;
+        P.n_sd += (P.p_level[t.level[b]] + 1) * (P.p_level[t.level[b]] + 2) / 2;
     }
     P.n_coef = off;
     P.d_centre = P.upload(centre);
@@ -1101,6 +1347,18 @@ void build_plan(hfmm_plan& P, const double* xyz, int64_t n, double k, const hfmm
     if (any_fp32) P.dM32 = P.alloc<float2>(P.n_coef);
     P.dL = P.alloc<double2>(P.n_coef);
     if (any_l2l32) P.dL32 = P.alloc<float2>(P.n_coef);
+    bool any_col = false, any_l2l_col = false;
+    for (int L = 0; L < kMaxLevels; ++L) {
+        any_col = any_col || P.m2lc[L].use || P.m2mc[L].use;
+        any_l2l_col = any_l2l_col || P.l2lc[L].use;
+    }
+    alloc_wave_parts(P);
+    const size_t n_sd = P.n_sd + wave_sd_pad(P.pmax);
+    for (double4** buf : {any_col ? &P.dMs : nullptr, any_l2l_col ? &P.dLs : nullptr})
+        if (buf) {
+            *buf = P.alloc<double4>(n_sd);
+            HIPCHK(hipMemset(*buf, 0, n_sd * sizeof(double4)));
+        }
     P.d_q = P.alloc<double2>(n);
     P.d_far = P.alloc<double2>(n);
     P.d_qin = P.alloc<double2>(n);
@@ -1172,6 +1430,40 @@ M2LBlockArgs block_args(const hfmm_plan& P, const M2LBlockLevel& B, bool fp32, c
     return a;
 }
 
+M2LWaveArgs wave_args(const hfmm_plan& P, const M2LWaveLevel& B, const double4* src, double2* dst, int overwrite) {
+    M2LWaveArgs a;
+    a.ps = P.p_eff[B.src_level];
+    a.pt = P.p_eff[B.tgt_level];
+    a.overwrite = overwrite;
+    a.n_items = B.n_items;
+    a.items = B.items;
+    a.n_blocks = B.n_blocks;
+    a.part = B.n_slots ? B.part : nullptr;
+    a.part_ptr = B.part_ptr;
+    a.tb = B.tb;
+    a.blk_targets = B.targets;
+    a.grp_class = B.cls;
+    a.grp_src = B.src;
+    a.grp_dir = B.dir;
+    a.rot1 = P.d_cr1;
+    a.rot3 = P.d_cr3;
+    a.rot_stride = P.cr_stride;
+    a.phase = P.d_phase;
+    a.phase_stride = P.pmax + 1;
+    a.coax = B.coax;
+    a.coax_stride = B.coax_stride;
+    a.M = src;
+    a.L = dst;
+    a.exp_off = P.d_expoff;
+    return a;
+}
+
+void launch_wave(const hfmm_plan& P, const M2LWaveLevel& B, const double4* src, double2* dst, int overwrite,
+                 hipStream_t s) {
+    const M2LWaveArgs a = wave_args(P, B, src, dst, overwrite);
+    launch_m2l_wave64(a, std::max(a.ps, a.pt), s);
+}
+
 // parts of one evaluate's device sequence (a batch runs them for all problems, with the
 // block M2L and the near field as persistent launches over every problem)
 constexpr int kSeqUp = 1;          // charges, clears, P2M, M2M
@@ -1188,6 +1480,13 @@ int64_t level_coef(const hfmm_plan& P, int l) {
     if (l > t.depth) return P.n_coef;
     const int b = t.level_start[l];
     return b < t.n_boxes() ? P.exp_off[b] : P.n_coef;
+}
+
+// the expansions of level l in (S, D) form, x basis buffer e to sd
+void level_to_sd(const hfmm_plan& P, int l, const double2* e, double4* sd, hipStream_t s) {
+    const Tree& t = P.tree;
+    const int b0 = t.level_start[l], b1 = t.level_start[l + 1];
+    if (b1 > b0) launch_to_sd64(e + P.exp_off[b0], sd + P.sd_off[b0], b1 - b0, P.p_level[l], s);
 }
 
 int out_mode_of(const hfmm_plan& P, int q_type) {
@@ -1238,8 +1537,14 @@ void run_sequence(hfmm_plan& P, const void* q, int q_type, double2* out, hipStre
         launch_p2m(P.d_leafdesc, P.n_far_leaves, P.p2m_chunk, lv, P.dX, P.dY, P.dZ, P.d_q, P.k, P.p_leafmax, P.dM, s);
         mark(2);
         bool conv[kMaxLevels + 1] = {};   // levels whose multipoles are in FP32 already
+        bool conv_sd[kMaxLevels + 1] = {};   // ... in (S, D) form
         for (int L = P.depth - 1; L >= 2; --L) {
-            if (P.m2mb[L].use) {
+            if (P.m2mc[L].use) {
+                const M2LWaveLevel& B = P.m2mc[L];
+                level_to_sd(P, L + 1, P.dM, P.dMs, s);
+                conv_sd[L + 1] = true;
+                launch_wave(P, B, P.dMs, P.dM, 1, s);
+            } else if (P.m2mb[L].use) {
                 const M2LBlockLevel& B = P.m2mb[L];
                 if (B.fp32) {   // the children's multipoles (complete now) in FP32
                     const int64_t c0 = level_coef(P, L + 1), c1 = level_coef(P, L + 2);
@@ -1257,6 +1562,8 @@ void run_sequence(hfmm_plan& P, const void* q, int q_type, double2* out, hipStre
         mark(3);
         // multipoles in FP32 for the FP32 block levels: every level not converted for an FP32
         // M2M (the converted ones need not be contiguous), one launch per run of levels
+        for (int L = 2; L <= P.depth; ++L)
+            if (P.m2lc[L].use && !conv_sd[L]) level_to_sd(P, L, P.dM, P.dMs, s);
         bool any_fp32 = false;
         for (int L = 2; L <= P.depth; ++L) any_fp32 |= P.m2l[L].n_targets && P.m2lb[L].use && P.m2lb[L].fp32;
         if (any_fp32)
@@ -1275,6 +1582,13 @@ void run_sequence(hfmm_plan& P, const void* q, int q_type, double2* out, hipStre
     for (int L = 2; L <= P.depth; ++L) {
         if (!P.m2l[L].n_targets) continue;
         const M2LBlockLevel& B = P.m2lb[L];
+        if (P.m2lc[L].use) {
+            if (!(parts & kSeqM2LBlock)) continue;
+            if (lev) HIPCHK(hipEventRecord(lev[2 * L], s));
+            launch_wave(P, P.m2lc[L], P.dMs, P.dL, 0, s);
+            if (lev) HIPCHK(hipEventRecord(lev[2 * L + 1], s));
+            continue;
+        }
         if (!B.use) {
             if (!(parts & kSeqM2LGeneric)) continue;
             if (lev) HIPCHK(hipEventRecord(lev[2 * L], s));
@@ -1299,7 +1613,10 @@ void run_sequence(hfmm_plan& P, const void* q, int q_type, double2* out, hipStre
     if (parts & kSeqDown) {
         for (int L = 2; L < P.depth; ++L) {
             const M2LBlockLevel& B = P.l2lb[L];
-            if (B.use && B.fp32) {   // the parents' locals (complete now) in FP32
+            if (P.l2lc[L].use) {
+                level_to_sd(P, L, P.dL, P.dLs, s);
+                launch_wave(P, P.l2lc[L], P.dLs, P.dL, 0, s);
+            } else if (B.use && B.fp32) {   // the parents' locals (complete now) in FP32
                 const int64_t c0 = level_coef(P, L), c1 = level_coef(P, L + 1);
                 launch_to_float(P.dL + c0, P.dL32 + c0, c1 - c0, s);
                 launch_m2l_block(block_args(P, B, true, P.dL32, P.dL, 0), B.tb, B.grp, 1, s);
@@ -1491,6 +1808,9 @@ int hfmm_plan_set_degrees(hfmm_plan* P, const int* p_level) {
         std::copy(eff, eff + kMaxLevels, P->p_eff);
         ++P->degree_version;
         HIPCHK(hipMemcpy(P->d_plevel, P->p_eff, sizeof(int) * kMaxLevels, hipMemcpyHostToDevice));
+        for (int L = 0; L < kMaxLevels; ++L)
+            for (M2LWaveLevel* B : {&P->m2lc[L], &P->m2mc[L], &P->l2lc[L]})
+                if (B->use) pack_wave_coax(*P, *B);
         if (P->gexec) {
             HIPCHK(hipGraphExecDestroy(P->gexec));
             P->gexec = nullptr;
@@ -1818,6 +2138,13 @@ struct hfmm_batch {
     int g_qtype = -1;
     // persistent launches over all problems (rebuilt with the graph): the block M2L, one
     // launch per kernel instance, and the near field
+    struct WaveInstance {                   // the FP64 wave kernel, one launch per degree
+        int p = 0, n = 0, n_sums = 0;
+        const int2* work = nullptr;
+        const int4* sums = nullptr;
+        const M2LWaveArgs* args = nullptr;
+    };
+    std::vector<WaveInstance> wave_inst;
     struct M2LInstance {
         int p = 0, tb = 0, g = 0, fp32 = 0, grid = 0;
         size_t shm = 0;
@@ -1836,15 +2163,21 @@ struct hfmm_batch {
         pallocs.clear();
         m2l_inst.clear();
         m2l_args.clear();
+        wave_inst.clear();
         d_p2p_args = nullptr;
         d_counters = nullptr;
     }
     template <typename T>
-    T* upload(const std::vector<T>& v) {
+    T* alloc(size_t n) {
         void* p = nullptr;
-        if (hipMalloc(&p, std::max<size_t>(1, v.size()) * sizeof(T)) != hipSuccess)
+        if (hipMalloc(&p, std::max<size_t>(1, n) * sizeof(T)) != hipSuccess)
             fail(HFMM_ERR_MEMORY, "hipMalloc failed (batch work lists)");
         pallocs.push_back(p);
+        return (T*)p;
+    }
+    template <typename T>
+    T* upload(const std::vector<T>& v) {
+        T* p = alloc<T>(v.size());
         if (!v.empty()) HIPCHK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
         return (T*)p;
     }
@@ -1899,6 +2232,19 @@ void build_persistent(hfmm_batch& B, void* const* out, int q_type) {
             pmax[key] = std::max(pmax[key], pk);
         }
     }
+    // wave kernel: one launch per degree over every problem and level, split to twice the items
+    // of a single level.  Split by level as for a plan alone, 16 problems of 2k to 20k points at
+    // p = 10 made 36128 items, of a group or two each: 2.67 ms, and 0.29 for the sums, against
+    // 1.37 and 0.05 for the 6016 items of this rule.
+    std::map<int, std::vector<std::pair<hfmm_plan*, const M2LWaveLevel*>>> waves;   // by degree
+    std::map<int, int64_t> wave_groups;
+    for (hfmm_plan* P : B.plans)
+        for (const M2LWaveLevel& c : P->m2lc) {
+            if (!c.use || !c.n_groups) continue;
+            const int pk = std::max(P->p_eff[c.src_level], P->p_eff[c.tgt_level]);
+            waves[pk].push_back({P, &c});
+            wave_groups[pk] += c.n_groups;
+        }
     B.n_counters = 16 * kXcds * ((int)groups.size() + 4);
     std::vector<int> zeros(B.n_counters, 0);
     B.d_counters = B.upload(zeros);
@@ -1918,6 +2264,35 @@ void build_persistent(hfmm_batch& B, void* const* out, int q_type) {
         in.grid = m2l_block_persistent_grid(in.p, in.tb, in.g, in.fp32, in.shm);
         B.m2l_inst.push_back(in);
         B.m2l_args.push_back(d_args);
+    }
+    for (auto& kv : waves) {   // every translation's items are a multiple of kXcds
+        hfmm_batch::WaveInstance in;
+        in.p = kv.first;
+        const int per_item = (int)std::max<int64_t>(1, (wave_groups[in.p] + 2 * kWaveItems - 1) / (2 * kWaveItems));
+        std::vector<M2LWaveArgs> args;
+        std::vector<int2> work;
+        std::vector<int4> sums;
+        for (auto& [P, c] : kv.second) {
+            std::vector<int> part_ptr;
+            const std::vector<int4> items = wave_items(P->tree, c->host_targets, c->host_ptr, c->tb, per_item, part_ptr);
+            const int n_slots = part_ptr[c->n_blocks], j = (int)args.size();
+            M2LWaveArgs w = wave_args(*P, *c, P->dMs, P->dL, 0);
+            w.n_items = (int)items.size();
+            w.items = B.upload(items);
+            w.part_ptr = B.upload(part_ptr);
+            w.part = n_slots ? B.alloc<double4>(wave_part_size(*c, n_slots)) : nullptr;
+            for (int t = 0; t < w.n_items; ++t) work.push_back(make_int2(j, t));
+            for (int b = 0; b < c->n_blocks; ++b)
+                if (part_ptr[b + 1] > part_ptr[b])
+                    for (int i = 0; i < wave64_sum_chunks(in.p, c->tb); ++i) sums.push_back(make_int4(j, b, i, 0));
+            args.push_back(w);
+        }
+        in.n = (int)work.size();
+        in.work = B.upload(work);
+        in.n_sums = (int)sums.size();
+        in.sums = B.upload(sums);
+        in.args = B.upload(args);
+        B.wave_inst.push_back(in);
     }
     std::vector<P2PBatchArgs> pa(np);
     std::vector<int2> work[4];
@@ -1963,6 +2338,9 @@ void batch_sequence(hfmm_batch& B, const void* const* q, int q_type, void* const
     for (size_t j = 0; j < B.m2l_inst.size(); ++j) {
         const auto& in = B.m2l_inst[j];
         launch_m2l_block_persistent(B.m2l_args[j], in.q, in.grid, in.p, in.tb, in.g, in.fp32, in.shm, s);
+    }
+    for (const auto& in : B.wave_inst) {
+        launch_m2l_wave64_batch(in.args, in.work, in.n, in.sums, in.n_sums, in.p, s);
     }
     mark(2);
     // downward passes
@@ -2025,6 +2403,7 @@ int hfmm_batch_create(int n_problems, const double* const* xyz, const int64_t* n
             if (!xyz[i]) fail(HFMM_ERR_ARG, "null positions of problem " + std::to_string(i));
             hfmm_plan* P = new hfmm_plan();
             try {
+                P->in_batch = true;
                 build_plan(*P, xyz[i], n[i], k[i], opts[i]);
             } catch (const Error& e) {
                 delete P;
