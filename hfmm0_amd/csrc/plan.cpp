@@ -95,7 +95,8 @@ struct M2LWaveLevel {
     int* part_ptr = nullptr;
     double4* part = nullptr;       // partial sums of blocks split over items, shared by the levels
     int n_groups = 0;
-    std::vector<int> host_targets, host_ptr;   // plans of a batch: blocks and their groups
+    std::vector<int> host_targets, host_ptr;   // plans of a batch: blocks and their groups,
+                                   // which the batch splits anew
 };
 
 struct XlateLaunch {
@@ -157,7 +158,7 @@ struct hfmm_plan {
     bool m2l_fp32[kMaxLevels] = {};  // M2L of the level in FP32 (mixed precision)
     M2LBlockLevel m2mb[kMaxLevels], l2lb[kMaxLevels];   // M2M / L2L on matrix cores
     M2LWaveLevel m2lc[kMaxLevels], m2mc[kMaxLevels], l2lc[kMaxLevels];   // FP64, one wave per item
-    bool in_batch = false;           // evaluated by a batch only
+    bool in_batch = false;           // one of a batch (also evaluated alone)
     std::vector<int64_t> sd_off;     // offset of each box's (S, D) entries
     int64_t n_sd = 0;
     double *d_cr1 = nullptr, *d_cr3 = nullptr;   // rotation fragments of the wave kernel
@@ -765,11 +766,6 @@ void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt
     pack_wave_coax(P, B);
     B.n_blocks = nblk;
     B.n_groups = blk_ptr[nblk];
-    if (P.in_batch && kind == 0) {   // split once the groups of all problems are known
-        B.host_targets = std::move(blk_targets);
-        B.host_ptr = std::move(blk_ptr);
-        return;
-    }
     // M2L blocks are split into items whose sums meet in a second kernel: three items for each
     // wave that runs at a time (1024 SIMDs)
     std::vector<int> part_ptr;
@@ -779,6 +775,10 @@ void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt
     B.items = P.upload(items);
     B.n_slots = part_ptr[nblk];
     B.part_ptr = P.upload(part_ptr);
+    if (P.in_batch && kind == 0) {
+        B.host_targets = std::move(blk_targets);
+        B.host_ptr = std::move(blk_ptr);
+    }
 }
 
 void build_tables(hfmm_plan& P) {

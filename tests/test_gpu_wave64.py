@@ -83,3 +83,16 @@ def test_batch(hf):
         for (x, q), k, pl, phi in zip(probs, ks, ps, out):
             alone = hf.evaluate(hf.setup(x, k, p=14, N_max=32, p_level=pl), q * (1 + rep))
             assert D.relative_error(phi, alone) < 1e-13
+
+
+def test_batch_plan_alone(hf):
+    """A problem of a batch evaluated by itself runs its own work items, before and after the batch."""
+    from hfmm0_amd.batch import Batch
+    print("case: wave64 batch, its plans alone", flush=True)
+    probs = [_points("cube", 3000, 1), _points("surface", 4100, 2)]
+    B = Batch([x for x, _ in probs], [5.0, 7.0], p=8, N_max=32)
+    for rep in range(2):
+        for i, (x, q) in enumerate(probs):
+            alone = hf.evaluate(hf.setup(x, [5.0, 7.0][i], p=8, N_max=32), q)
+            assert D.relative_error(hf.evaluate(B.plan(i), q), alone) < 1e-13
+        B.evaluate([q for _, q in probs])
