@@ -89,28 +89,35 @@ void launch_xlate(const XlateArgs& a, int n_targets, hipStream_t s);
 void launch_l2p_field(const int* leaves, int n_items, DevBoxes bx, DevLevels lv, const double* X, const double* Y,
                       const double* Z, const double2* L, double k, int pmax, double2* far, double2* far_e,
                       hipStream_t s);
-// Near field over the leaves in leaf_box order, coordinate differences and r^2 in FP64.
-// FP32 (precision != 0): FP32 weights; the first n_fp32 leaves with an FP32 phase k r, the
-// rest with the phase in FP64 (their pairs reach k r > kP2PFp32MaxKr).  FP64: every leaf
-// in FP64.  Pairs with r^2 <= floor2[leaf] (the coincidence floor of the leaf's pairs,
-// in unscaled coordinates) contribute nothing.
+// Near field (nearfield.hip) over work items, coordinate differences and r^2 in FP64.
+// FP32 (precision != 0): FP32 weights; the items of the first list with an FP32 phase k r, those
+// of the second with the phase in FP64 (their pairs reach k r > kP2PFp32MaxKr).  FP64: every leaf
+// in FP64 (first list).  Pairs with r^2 <= floor2[leaf] (the coincidence floor of the leaf's
+// pairs, in unscaled coordinates) contribute nothing.
 constexpr double kP2PFp32MaxKr = 8.0;
 // Largest k r over a plan's near pairs for which the mixed near field takes e^{ikr} as
 // 1 + ikr (relative error (kr)^2 / 2 <= 5e-9, below FP32 rounding).
 constexpr double kP2PLowKr = 1e-4;
-void launch_p2p_field(int precision, int n_leaves, int n_fp32, const int* leaf_box, DevBoxes bx,
-                      const int* rng_ptr, const int* rng_start, const int* rng_pref, const int* leaf_src_total,
-                      const double* floor2, const double* X, const double* Y, const double* Z, const double2* q,
-                      double k, const double2* far, const double2* far_e, const int* perm, int out_mode,
-                      double2* out, double2* field, hipStream_t s);
-
+// waves that share a work item's sources
+constexpr int kNearWaves = 4;
+struct NearItem {                 // targets [target, target + n_targets) of a leaf (0: padding)
+    int leaf, box, target, n_targets;
+};
+struct NearItems {
+    const NearItem* items = nullptr;
+    int n = 0;                    // a multiple of kXcds
+};
+struct NearBatch {                // 64 consecutive sources of a leaf's ranges
+    unsigned long long mask;      // bit i > 0: source i is the first of a range
+    int first;                    // range of source 0
+    int pad;
+};
 struct P2PArgs {
-    int leaf0;                    // first leaf of the launch (set by the launcher)
     const int* leaf_box;          // leaf -> box
     DevBoxes bx;
-    const int* rng_ptr;           // per leaf: its source point ranges [rng_ptr[l], rng_ptr[l+1])
-    const int* rng_start;         // first point of each range
-    const int* rng_pref;          // sources of the leaf before each range
+    const int* batch_ptr;         // per leaf: its first batch of 64 sources
+    const NearBatch* batches;
+    const int* rng_delta;         // per range: point of a source minus its number in the leaf
     const int* leaf_src_total;    // sources of each leaf
     const double* floor2;         // per leaf: coincidence floor on r^2 (unscaled coordinates)
     const double *X, *Y, *Z;      // sorted points (FP64)
@@ -118,17 +125,23 @@ struct P2PArgs {
     double k;                     // |k|
     double kp_hi, kp_lo;          // |k| / pi in two terms (FP64 near field)
     double scale;                 // coordinate scale of the mixed kernel (set by the launcher)
-    double wscale;                // factor of the mixed kernel's sums (set by the launcher)
+    double wscale;                // factor of the sums (set by the launcher)
     const double2* far;           // far field per sorted point
+    const double2* far_e;         // field: 3 values per sorted point
     const int* perm;              // sorted -> input order
     int out_mode;                 // bit 0: conjugate, bit 1: zero imaginary part
     double2* out;                 // input order
+    double2* field;               // 3 values per point, input order
     const unsigned char* coord32; // per leaf (mixed form, FP32 phase): 1 = coordinate differences
                                   // and r^2 in FP32 (null: FP64 at every leaf)
 };
+constexpr int kP2PFp64TargetsPerLane = 2;   // FP64 near field: two independent chains per lane
+constexpr int kP2PFieldTargetsPerLane = 1;
 // lowk: every near pair of the plan has k r <= kP2PLowKr (mixed form only); tile: targets
-// per lane of the mixed form (1, 2 or 4)
-void launch_p2p(const P2PArgs& a, int precision, int n_leaves, int n_fp32, bool lowk, int tile, hipStream_t s);
+// per lane of the mixed form (1, 2 or 4); items: the two lists
+void launch_p2p(const P2PArgs& a, const NearItems* items, int precision, bool lowk, int tile, hipStream_t s);
+// the potential and E = -grad phi (a.far_e, a.field set)
+void launch_p2p_field(const P2PArgs& a, const NearItems* items, int precision, hipStream_t s);
 // Per leaf l < n (leaf order of a): flag[l] = 1 where FP32 coordinates keep the estimated
 // relative near-field error of every target of the leaf at or below tol:
 //   2^-21 c_max sqrt(sum_j r_j^-4 / sum_j r_j^-2)  <= tol,
@@ -322,18 +335,13 @@ void launch_m2l_wave64_batch(const M2LWaveArgs* d_args, const int2* work, int n,
 // the expansions of n_boxes consecutive boxes of degree p as (S_re, S_im, D_re, D_im) entries
 void launch_to_sd64(const double2* x, double4* sd, int64_t n_boxes, int p, hipStream_t s);
 
-// near field of one problem in a persistent batch launch
+// near field of the problems of a batch: one launch per leaf class (FP64 plans; mixed plans with
+// k r <= kP2PLowKr; mixed, FP32 phase; mixed, FP64 phase) over items of all problems,
+// d_args[prob[i]] with scale and wscale set (p2p_scaled)
 constexpr int kP2PBatchTargetsPerLane = 2;
-constexpr int kP2PFp64TargetsPerLane = 2;   // FP64 near field: two independent chains per lane
-struct P2PBatchArgs {
-    P2PArgs a;                    // scale and wscale set (p2p_scaled)
-};
-// leaf classes of the persistent near field: FP64 plans; mixed plans with k r <= kP2PLowKr;
-// mixed, FP32 phase; mixed, FP64 phase
 constexpr int kP2PClassFp64 = 0, kP2PClassLowK = 1, kP2PClassPhase32 = 2, kP2PClassPhase64 = 3;
 P2PArgs p2p_scaled(P2PArgs a, int precision, bool lowk);
-int p2p_persistent_grid(int cls);
-void launch_p2p_persistent(int cls, const P2PBatchArgs* d_args, const WorkQueues& q, int grid, hipStream_t s);
+void launch_p2p_batch(int cls, const P2PArgs* d_args, const NearItem* items, const int* prob, int n, hipStream_t s);
 void launch_m2l_block_persistent(const M2LBlockArgs* d_args, const WorkQueues& q, int grid, int p, int tb, int g,
                                  int fp32, size_t shm, hipStream_t s);
 void launch_to_float(const double2* in, float2* out, int64_t n, hipStream_t s);

@@ -848,536 +848,6 @@ __global__ __launch_bounds__(kXlateThreads) void xlate_kernel(XlateArgs a) {
 }
 
 // ---------------------------------------------------------------------------------
-// P2P near field.
-// ---------------------------------------------------------------------------------
-using nearfield::HalfTurnK;
-using nearfield::radian_weight;
-using nearfield::radian_weight_phase64;
-
-// e^{ikr}/r and the field weight (1 - ikr) e^{ikr}/r^3, so that
-// -grad_x e^{ik|x-y|}/|x-y| = (x - y) * field weight (HFMM.py:29-37 in complex form)
-__device__ inline void field_weights(float r2, float k, float& wr, float& wi, float& fr, float& fi) {
-    radian_weight(r2, k, wr, wi);
-    const float rinv2 = 1.0f / r2;
-    const float kr = k * sqrtf(r2);
-    fr = (wr + kr * wi) * rinv2;
-    fi = (wi - kr * wr) * rinv2;
-}
-__device__ inline void field_weights64(double r2, double fl2, double k, HalfTurnK kp,
-                                       const nearfield::SinCosPi64& sp, double& wr, double& wi, double& fr,
-                                       double& fi) {
-    double c, s, rs, rinv, r;
-    nearfield::halfturn64(r2, kp, sp, c, s, rs, rinv, r);
-    rs = r2 > fl2 ? rs : 0.0;
-    wr = c * rs;
-    wi = s * rs;
-    const double kr = k * r, rinv2 = rinv * rinv;
-    fr = fma(kr, wi, wr) * rinv2;
-    fi = fma(-kr, wr, wi) * rinv2;
-}
-
-// Source staging of the near-field kernels: lane `lane` of a batch starting at `base`
-// walks the leaf's list of point ranges (prefix sums rng_pref over [r0, r1)) to the range
-// holding source v = base + lane; `ri` carries the range index from batch to batch (it
-// only grows), so the walk is a step or two per batch.
-__device__ inline int p2p_source_index(int v, int r1, const int* rng_start, const int* rng_pref, int& ri) {
-    while (ri + 1 < r1 && rng_pref[ri + 1] <= v) ++ri;
-    return rng_start[ri] + (v - rng_pref[ri]);
-}
-
-// Target chunk of a leaf: up to 64 R targets; a remainder that is not a power of two
-// (and above 4 R) goes as its largest power of two first, so that few target slots of
-// the R x L lanes are idle (each chunk stages the sources once more).
-template <int R>
-__device__ inline int p2p_chunk(int remaining) {
-    if (remaining >= 64 * R) return 64 * R;
-    if (remaining <= 4 * R) return remaining;
-    int p = 1;
-    while (2 * p <= remaining) p <<= 1;
-    return p;
-}
-
-// Mixed-precision near field: one wave per target leaf.  Each lane holds R targets of the
-// chunk (li, li + L, ..., with L lanes per group, L = next power of two >= chunk / R) and
-// scans every G-th source (G = 64 / L groups) of each 64-point batch staged in LDS, so
-// that every source read from LDS feeds R independent pair evaluations.  Coordinates are
-// relative to the target leaf centre and scaled by a.scale = k / pi, in FP64: the
-// coordinate differences and r^2 are FP64 (exact to rounding for close pairs; FP32 at the
-// FP32-phase leaves flagged in a.coord32, p2p_mixed_body_c32), the
-// weights e^{i pi u}/u (u = k r / pi) FP32 (halfturn_weight; PH: phase in FP64), the
-// 64-source batch sums FP32, added into FP64 sums per target.  LOWK (k r below 1e-4 over
-// every pair of the plan, k = 0 included): coordinates unscaled and the weights
-// 1/r + i k, exact to FP32 rounding.  Pairs with r^2 at or below the leaf's coincidence
-// floor contribute nothing.  The sums times a.wscale (k / pi; 1 for LOWK) are added to the
-// far field and written in input order.  The workgroup handles leaf a.leaf0 + blockIdx.x.
-// LDS of the near-field kernels: 64 staged sources
-union P2PStage {
-    struct {
-        double2 xy[64];
-        double2 zq[64];   // (z, charge as two FP32 bit-cast into one double)
-    } mixed;
-    struct {
-        double x[64], y[64], z[64], qr[64], qi[64];
-    } fp64;
-};
-
-// The FP32-phase mixed near field of a leaf whose coordinate differences and r^2 may be
-// FP32 (a.coord32): the same schedule as p2p_mixed_body, with the scaled coordinates
-// relative to the leaf centre rounded to FP32 once (targets in registers, sources staged
-// in LDS as (x, y, z) and the charge).
-template <int R>
-__device__ __forceinline__ void p2p_mixed_body_c32(const P2PArgs& a, const int leaf, P2PStage& st) {
-    float4* sxyz = (float4*)st.mixed.xy;
-    float2* sq = (float2*)st.mixed.zq;
-    const int b = a.leaf_box[leaf];
-    const int tstart = a.bx.pstart[b], tcnt = a.bx.count[b];
-    const double sc = a.scale;
-    const double cx = a.bx.centre[3 * b], cy = a.bx.centre[3 * b + 1], cz = a.bx.centre[3 * b + 2];
-    const int r0 = a.rng_ptr[leaf], r1 = a.rng_ptr[leaf + 1];
-    const int S = a.leaf_src_total[leaf];
-    // the floor in scaled coordinates, at least 2^-120 (an FP32 normal number)
-    const float fl2 = (float)fmax(a.floor2[leaf] * sc * sc, 0x1p-120);
-    const int lane = threadIdx.x;
-    for (int t0 = 0, tc = 0; t0 < tcnt; t0 += tc) {
-        tc = p2p_chunk<R>(tcnt - t0);
-        const int need = (tc + R - 1) / R;
-        int L = 1;
-        while (L < need) L <<= 1;
-        const int G = 64 / L;
-        const int li = lane & (L - 1), g = lane / L;
-        float xt[R], yt[R], zt[R];
-        double sr[R], si[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int it = tstart + t0 + min(li + r * L, tc - 1);
-            xt[r] = (float)((a.X[it] - cx) * sc);
-            yt[r] = (float)((a.Y[it] - cy) * sc);
-            zt[r] = (float)((a.Z[it] - cz) * sc);
-            sr[r] = 0.0;
-            si[r] = 0.0;
-        }
-        int ri = r0;
-        for (int base = 0; base < S; base += 64) {
-            const int v = base + lane;
-            if (v < S) {
-                const int idx = p2p_source_index(v, r1, a.rng_start, a.rng_pref, ri);
-                const double2 qq = a.q[idx];
-                sxyz[lane] = make_float4((float)((a.X[idx] - cx) * sc), (float)((a.Y[idx] - cy) * sc),
-                                         (float)((a.Z[idx] - cz) * sc), 0.0f);
-                sq[lane] = make_float2((float)qq.x, (float)qq.y);
-            }
-            __syncthreads();
-            const int nb = min(64, S - base);
-            float ar[R], ai[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r) ar[r] = ai[r] = 0.0f;
-            for (int j = g; j < nb; j += G) {
-                const float4 p = sxyz[j];
-                const float2 qj = sq[j];
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const float dx = xt[r] - p.x, dy = yt[r] - p.y, dz = zt[r] - p.z;
-                    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                    float c, s, rs;
-                    nearfield::halfturn_parts(fmaxf(r2, 0x1p-120f), c, s, rs);
-                    rs = r2 > fl2 ? rs : 0.0f;
-                    const float wr = c * rs, wi = s * rs;
-                    ar[r] = fmaf(wr, qj.x, ar[r]);
-                    ar[r] = fmaf(-wi, qj.y, ar[r]);
-                    ai[r] = fmaf(wr, qj.y, ai[r]);
-                    ai[r] = fmaf(wi, qj.x, ai[r]);
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                sr[r] += (double)ar[r];
-                si[r] += (double)ai[r];
-            }
-            __syncthreads();
-        }
-        for (int off = L; off < 64; off <<= 1)
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                sr[r] += __shfl_xor(sr[r], off);
-                si[r] += __shfl_xor(si[r], off);
-            }
-        if (g == 0) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int ti = li + r * L;
-                if (ti < tc) {
-                    const int it = tstart + t0 + ti;
-                    double2 f = a.far[it];
-                    f.x = fma(sr[r], a.wscale, f.x);
-                    f.y = fma(si[r], a.wscale, f.y);
-                    if (a.out_mode & 1) f.y = -f.y;   // k < 0: conjugate of the |k| result
-                    if (a.out_mode & 2) f.y = 0.0;    // k == 0 with real charges: the result is real
-                    a.out[a.perm[it]] = f;
-                }
-            }
-        }
-    }
-}
-
-template <bool PH, bool LOWK, int R>
-__device__ __forceinline__ void p2p_mixed_body(const P2PArgs& a, const int leaf, P2PStage& st) {
-    if constexpr (!PH && !LOWK) {
-        if (a.coord32 && a.coord32[leaf]) {   // uniform: one leaf per workgroup
-            p2p_mixed_body_c32<R>(a, leaf, st);
-            return;
-        }
-    }
-    double2* sxy = st.mixed.xy;
-    double2* szq = st.mixed.zq;
-    const int b = a.leaf_box[leaf];
-    const int tstart = a.bx.pstart[b], tcnt = a.bx.count[b];
-    const double sc = a.scale;
-    const double cx = a.bx.centre[3 * b], cy = a.bx.centre[3 * b + 1], cz = a.bx.centre[3 * b + 2];
-    const int r0 = a.rng_ptr[leaf], r1 = a.rng_ptr[leaf + 1];
-    const int S = a.leaf_src_total[leaf];
-    // the floor in scaled coordinates, and at least 2^-120 so that an FP32 r^2 above it is
-    // a normal number
-    const double fl2 = fmax(a.floor2[leaf] * sc * sc, 0x1p-120);
-    const float kf = (float)a.k;
-    const int lane = threadIdx.x;
-    for (int t0 = 0, tc = 0; t0 < tcnt; t0 += tc) {
-        tc = p2p_chunk<R>(tcnt - t0);
-        const int need = (tc + R - 1) / R;
-        int L = 1;
-        while (L < need) L <<= 1;
-        const int G = 64 / L;
-        const int li = lane & (L - 1), g = lane / L;
-        double xt[R], yt[R], zt[R], sr[R], si[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int it = tstart + t0 + min(li + r * L, tc - 1);
-            xt[r] = (a.X[it] - cx) * sc;
-            yt[r] = (a.Y[it] - cy) * sc;
-            zt[r] = (a.Z[it] - cz) * sc;
-            sr[r] = 0.0;
-            si[r] = 0.0;
-        }
-        int ri = r0;
-        for (int base = 0; base < S; base += 64) {
-            const int v = base + lane;
-            if (v < S) {
-                const int idx = p2p_source_index(v, r1, a.rng_start, a.rng_pref, ri);
-                const double2 qq = a.q[idx];
-                const float2 qf = make_float2((float)qq.x, (float)qq.y);
-                sxy[lane] = make_double2((a.X[idx] - cx) * sc, (a.Y[idx] - cy) * sc);
-                szq[lane] = make_double2((a.Z[idx] - cz) * sc, __builtin_bit_cast(double, qf));
-            }
-            __syncthreads();
-            const int nb = min(64, S - base);
-            float ar[R], ai[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r) ar[r] = ai[r] = 0.0f;
-            for (int j = g; j < nb; j += G) {
-                const double2 pxy = sxy[j], pzq = szq[j];
-                const float2 qj = __builtin_bit_cast(float2, pzq.y);
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const double dx = xt[r] - pxy.x, dy = yt[r] - pxy.y, dz = zt[r] - pzq.x;
-                    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-                    float wr, wi;
-                    if constexpr (LOWK) {
-                        const bool ok = r2 > fl2;
-                        const float rs = nearfield::rsq((float)r2);
-                        wr = ok ? rs : 0.0f;
-                        wi = ok ? kf : 0.0f;
-                    } else {
-                        nearfield::pair_weight<PH>(r2, fl2, wr, wi);
-                    }
-                    ar[r] = fmaf(wr, qj.x, ar[r]);
-                    ar[r] = fmaf(-wi, qj.y, ar[r]);
-                    ai[r] = fmaf(wr, qj.y, ai[r]);
-                    ai[r] = fmaf(wi, qj.x, ai[r]);
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                sr[r] += (double)ar[r];
-                si[r] += (double)ai[r];
-            }
-            __syncthreads();
-        }
-        for (int off = L; off < 64; off <<= 1)
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                sr[r] += __shfl_xor(sr[r], off);
-                si[r] += __shfl_xor(si[r], off);
-            }
-        if (g == 0) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int ti = li + r * L;
-                if (ti < tc) {
-                    const int it = tstart + t0 + ti;
-                    double2 f = a.far[it];
-                    f.x = fma(sr[r], a.wscale, f.x);
-                    f.y = fma(si[r], a.wscale, f.y);
-                    if (a.out_mode & 1) f.y = -f.y;   // k < 0: conjugate of the |k| result
-                    if (a.out_mode & 2) f.y = 0.0;    // k == 0 with real charges: the result is real
-                    a.out[a.perm[it]] = f;
-                }
-            }
-        }
-    }
-}
-
-// Leaf of workgroup i of a launch over n leaves: workgroup i runs on XCD i % 8, and XCD x
-// takes the contiguous range of n / 8 (+1 for x < n % 8) leaves starting at
-// x (n / 8) + min(x, n % 8), so that its L2 holds one region's points (leaves are in Morton
-// order, and a leaf's sources are its neighbours).  A bijection of [0, n).
-__device__ inline int xcd_leaf(int i, int n) {
-    const int q = n / kXcds, r = n % kXcds, x = i % kXcds;
-    return x * q + min(x, r) + i / kXcds;
-}
-
-template <bool PH, bool LOWK, int R>
-__global__ __launch_bounds__(64) void p2p_mixed_kernel(P2PArgs a) {
-    __shared__ P2PStage st;
-    p2p_mixed_body<PH, LOWK, R>(a, a.leaf0 + xcd_leaf(blockIdx.x, gridDim.x), st);
-}
-
-// FP64 near field (the plain form): one wave per target leaf on the schedule of the mixed form
-// (R targets per lane, G = 64 / L groups of lanes over the staged sources; coordinates relative
-// to the target leaf centre).  Pairs at or below the leaf's coincidence floor get the weight
-// zero.  Bound by the issue of its FP64 instructions, about 50 per pair with a v_rsq_f64: 350 G
-// pairs/s at N = 400k (9.3e8 pairs, leaves of about 98) against 172 with the device library's
-// sincos, square root and division (5.41 -> 2.65 ms).
-template <int R>
-__device__ __forceinline__ void p2p_fp64_body(const P2PArgs& a, const int leaf, P2PStage& st) {
-    double *sx = st.fp64.x, *sy = st.fp64.y, *sz = st.fp64.z, *sqr = st.fp64.qr, *sqi = st.fp64.qi;
-    const int b = a.leaf_box[leaf];
-    const int tstart = a.bx.pstart[b], tcnt = a.bx.count[b];
-    const double cx = a.bx.centre[3 * b], cy = a.bx.centre[3 * b + 1], cz = a.bx.centre[3 * b + 2];
-    const int r0 = a.rng_ptr[leaf], r1 = a.rng_ptr[leaf + 1];
-    const int S = a.leaf_src_total[leaf];
-    const double fl2 = a.floor2[leaf];
-    const HalfTurnK kp{a.kp_hi, a.kp_lo};
-    const nearfield::SinCosPi64 sp = nearfield::SinCosPi64::pinned();
-    const int lane = threadIdx.x;
-    for (int t0 = 0, tc = 0; t0 < tcnt; t0 += tc) {
-        tc = p2p_chunk<R>(tcnt - t0);
-        const int need = (tc + R - 1) / R;
-        int L = 1;
-        while (L < need) L <<= 1;
-        const int G = 64 / L;
-        const int li = lane & (L - 1), g = lane / L;
-        double xt[R], yt[R], zt[R], sr[R], si[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int it = tstart + t0 + min(li + r * L, tc - 1);
-            xt[r] = a.X[it] - cx;
-            yt[r] = a.Y[it] - cy;
-            zt[r] = a.Z[it] - cz;
-            sr[r] = 0.0;
-            si[r] = 0.0;
-        }
-        int ri = r0;
-        for (int base = 0; base < S; base += 64) {
-            const int v = base + lane;
-            if (v < S) {
-                const int idx = p2p_source_index(v, r1, a.rng_start, a.rng_pref, ri);
-                sx[lane] = a.X[idx] - cx;
-                sy[lane] = a.Y[idx] - cy;
-                sz[lane] = a.Z[idx] - cz;
-                const double2 qq = a.q[idx];
-                sqr[lane] = qq.x;
-                sqi[lane] = qq.y;
-            }
-            __syncthreads();
-            const int nb = min(64, S - base);
-            for (int j = g; j < nb; j += G) {
-                const double xs = sx[j], ys = sy[j], zs = sz[j], qr = sqr[j], qi = sqi[j];
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const double dx = xt[r] - xs, dy = yt[r] - ys, dz = zt[r] - zs;
-                    const double r2 = dx * dx + dy * dy + dz * dz;
-                    double wr, wi;
-                    nearfield::pair_weight64(r2, fl2, kp, sp, wr, wi);
-                    sr[r] = fma(wr, qr, fma(-wi, qi, sr[r]));
-                    si[r] = fma(wr, qi, fma(wi, qr, si[r]));
-                }
-            }
-            __syncthreads();
-        }
-        for (int off = L; off < 64; off <<= 1)
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                sr[r] += __shfl_xor(sr[r], off);
-                si[r] += __shfl_xor(si[r], off);
-            }
-        if (g == 0) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int ti = li + r * L;
-                if (ti < tc) {
-                    const int it = tstart + t0 + ti;
-                    double2 f = a.far[it];
-                    f.x += sr[r];
-                    f.y += si[r];
-                    if (a.out_mode & 1) f.y = -f.y;   // k < 0: conjugate of the |k| result
-                    if (a.out_mode & 2) f.y = 0.0;    // k == 0 with real charges: the result is real
-                    a.out[a.perm[it]] = f;
-                }
-            }
-        }
-    }
-}
-
-__global__ __launch_bounds__(64) void p2p_fp64_kernel(P2PArgs a) {
-    __shared__ P2PStage st;
-    p2p_fp64_body<kP2PFp64TargetsPerLane>(a, a.leaf0 + xcd_leaf(blockIdx.x, gridDim.x), st);
-}
-
-// Persistent near field over the leaves of many problems (batches), one launch per leaf
-// class CLS (kP2PClass*): one wave per workgroup takes (problem, leaf) work from the
-// queues q until all are empty; args[w.x] is the problem's near-field description.
-template <int CLS>
-__global__ __launch_bounds__(64) void p2p_persistent_kernel(const P2PBatchArgs* __restrict__ args, WorkQueues q) {
-    __shared__ P2PStage st;
-    const int home = blockIdx.x % kXcds;
-    for (;;) {
-        int w = 0;
-        if (threadIdx.x == 0) w = work_dequeue(q, home);
-        w = __builtin_amdgcn_readfirstlane(w);   // uniform: the descriptor is read with scalar loads
-        if (w < 0) break;
-        const int2 wk = q.work[w];
-        const int prob = __builtin_amdgcn_readfirstlane(wk.x), leaf = __builtin_amdgcn_readfirstlane(wk.y);
-        const P2PArgs a = args[prob].a;
-        if constexpr (CLS == kP2PClassFp64)
-            p2p_fp64_body<kP2PFp64TargetsPerLane>(a, leaf, st);
-        else if constexpr (CLS == kP2PClassLowK)
-            p2p_mixed_body<false, true, kP2PBatchTargetsPerLane>(a, leaf, st);
-        else if constexpr (CLS == kP2PClassPhase32)
-            p2p_mixed_body<false, false, kP2PBatchTargetsPerLane>(a, leaf, st);
-        else
-            p2p_mixed_body<true, false, kP2PBatchTargetsPerLane>(a, leaf, st);
-        __syncthreads();
-    }
-}
-
-// P2P with the field: the potential and E = -grad phi of the near field (same
-// decomposition and source ranges as p2p_kernel), added to the far-field values.
-// field[3 i + a] holds component a of point i (input order).
-template <typename T, bool PH>
-__global__ __launch_bounds__(64) void p2p_field_kernel(int leaf0, const int* leaf_box, DevBoxes bx,
-                                                       const int* rng_ptr, const int* rng_start, const int* rng_pref,
-                                                       const int* leaf_src_total, const double* floor2,
-                                                       const double* X, const double* Y, const double* Z,
-                                                       const double2* q, double k, HalfTurnK kp, const double2* far,
-                                                       const double2* far_e, const int* perm, int out_mode,
-                                                       double2* out, double2* field) {
-    // coordinates relative to the leaf centre and r^2 in FP64 at every precision: FP32
-    // coordinates would carry an absolute error of 2^-24 times the leaf size, a large
-    // relative error of r for close pairs (points on surfaces); FP64 adds and FMAs issue
-    // at the rate of the (unpacked) FP32 ones
-    using C = double;
-    __shared__ C sx[64], sy[64], sz[64];
-    __shared__ T sqr[64], sqi[64];
-    const int leaf = leaf0 + blockIdx.x;
-    const int b = leaf_box[leaf];
-    const int tstart = bx.pstart[b], tcnt = bx.count[b];
-    const double cx = bx.centre[3 * b], cy = bx.centre[3 * b + 1], cz = bx.centre[3 * b + 2];
-    const int r0 = rng_ptr[leaf], r1 = rng_ptr[leaf + 1];
-    const int S = leaf_src_total[leaf];
-    const double fl2 = floor2[leaf];
-    const int lane = threadIdx.x;
-    const T kk = (T)k;
-    const nearfield::SinCosPi64 sp = nearfield::SinCosPi64::pinned();
-    // target chunks of 64; a remainder of 33..63 targets goes as 32 + the rest, so that the
-    // lanes are not left idle with T' = 64 (each lane then scans half or less of the sources)
-    for (int t0 = 0, tc = 0; t0 < tcnt; t0 += tc) {
-        tc = tcnt - t0 >= 64 ? 64 : min(32, tcnt - t0);
-        int Tp = 1;
-        while (Tp < tc) Tp <<= 1;
-        const int G = 64 / Tp;
-        const int ti = lane & (Tp - 1), g = lane / Tp;
-        const bool has_t = ti < tc;
-        const int it = tstart + t0 + (has_t ? ti : 0);
-        const C xt = (C)(X[it] - cx), yt = (C)(Y[it] - cy), zt = (C)(Z[it] - cz);
-        double sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};   // phi, Ex, Ey, Ez (re, im); FP64 over batches
-        for (int base = 0; base < S; base += 64) {
-            T acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-            const int v = base + lane;
-            if (v < S) {
-                int lo = r0, hi = r1 - 1;
-                while (lo < hi) {
-                    const int mid = (lo + hi + 1) >> 1;
-                    if (rng_pref[mid] <= v)
-                        lo = mid;
-                    else
-                        hi = mid - 1;
-                }
-                const int idx = rng_start[lo] + (v - rng_pref[lo]);
-                sx[lane] = (C)(X[idx] - cx);
-                sy[lane] = (C)(Y[idx] - cy);
-                sz[lane] = (C)(Z[idx] - cz);
-                const double2 qq = q[idx];
-                sqr[lane] = (T)qq.x;
-                sqi[lane] = (T)qq.y;
-            }
-            __syncthreads();
-            const int nb = min(64, S - base);
-            for (int j = g; j < nb; j += G) {
-                const C dx = xt - sx[j], dy = yt - sy[j], dz = zt - sz[j];
-                const C r2 = dx * dx + dy * dy + dz * dz;
-                if (std::is_same<T, double>::value || r2 > fl2) {   // FP64: zero weights at the floor
-                    T wr, wi, fr, fi;
-                    if constexpr (std::is_same<T, double>::value) {
-                        field_weights64(r2, fl2, k, kp, sp, wr, wi, fr, fi);
-                    } else if constexpr (PH) {
-                        float rinv, kr;
-                        radian_weight_phase64(r2, k, wr, wi, rinv, kr);
-                        const float rinv2 = rinv * rinv;
-                        fr = (wr + kr * wi) * rinv2;
-                        fi = (wi - kr * wr) * rinv2;
-                    } else {
-                        field_weights((T)r2, kk, wr, wi, fr, fi);
-                    }
-                    const T qr = sqr[j], qi = sqi[j];
-                    acc[0] += wr * qr - wi * qi;
-                    acc[1] += wr * qi + wi * qr;
-                    const T gr = fr * qr - fi * qi, gi = fr * qi + fi * qr;
-                    acc[2] += (T)dx * gr;
-                    acc[3] += (T)dx * gi;
-                    acc[4] += (T)dy * gr;
-                    acc[5] += (T)dy * gi;
-                    acc[6] += (T)dz * gr;
-                    acc[7] += (T)dz * gi;
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < 8; ++c) sum[c] += (double)acc[c];
-            __syncthreads();
-        }
-        for (int off = Tp; off < 64; off <<= 1)
-#pragma unroll
-            for (int c = 0; c < 8; ++c) sum[c] += __shfl_xor(sum[c], off);
-        if (g == 0 && has_t) {
-            const int o = perm[it];
-            double2 f = far[it];
-            f.x += sum[0];
-            f.y += sum[1];
-            if (out_mode & 1) f.y = -f.y;   // k < 0: conjugate of the |k| result
-            if (out_mode & 2) f.y = 0.0;    // k == 0 with real charges: the result is real
-            out[o] = f;
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                double2 e = far_e[3 * (int64_t)it + a];
-                e.x += sum[2 + 2 * a];
-                e.y += sum[3 + 2 * a];
-                if (out_mode & 1) e.y = -e.y;
-                if (out_mode & 2) e.y = 0.0;
-                field[3 * (int64_t)o + a] = e;
-            }
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------------
 // FP64 direct sum at sampled targets: grid (target tiles of 256, source chunks);
 // partial sums combined with FP64 atomics into a zeroed output.  kp is |k| / pi; conj
 // (k < 0) takes the conjugate of the |k| sum of the conjugate charges.  Bound by FP64 issue:
@@ -1385,7 +855,7 @@ __global__ __launch_bounds__(64) void p2p_field_kernel(int leaf0, const int* lea
 // root and division (17.5 -> 8.2 ms).
 // ---------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void direct_kernel(const double* X, const double* Y, const double* Z,
-                                                     const double2* q, int64_t n, HalfTurnK kp, int conj,
+                                                     const double2* q, int64_t n, nearfield::HalfTurnK kp, int conj,
                                                      const double* tx, const double* ty, const double* tz,
                                                      int64_t nt, int64_t chunk, double2* out) {
     __shared__ double sx[256], sy[256], sz[256], sqr[256], sqi[256];
@@ -1550,30 +1020,6 @@ void launch_l2p_field(const int* leaves, int n_items, DevBoxes bx, DevLevels lv,
     check_launch("l2p_field");
 }
 
-void launch_p2p_field(int precision, int n_leaves, int n_fp32, const int* leaf_box, DevBoxes bx,
-                      const int* rng_ptr, const int* rng_start, const int* rng_pref, const int* leaf_src_total,
-                      const double* floor2, const double* X, const double* Y, const double* Z, const double2* q,
-                      double k, const double2* far, const double2* far_e, const int* perm, int out_mode,
-                      double2* out, double2* field, hipStream_t s) {
-    if (n_leaves <= 0) return;
-    const HalfTurnK kp = nearfield::halfturn_k(k);
-    if (precision == 0) {
-        hipLaunchKernelGGL((p2p_field_kernel<double, false>), dim3(n_leaves), dim3(64), 0, s, 0, leaf_box, bx,
-                           rng_ptr, rng_start, rng_pref, leaf_src_total, floor2, X, Y, Z, q, k, kp, far, far_e, perm,
-                           out_mode, out, field);
-    } else {
-        if (n_fp32 > 0)
-            hipLaunchKernelGGL((p2p_field_kernel<float, false>), dim3(n_fp32), dim3(64), 0, s, 0, leaf_box, bx,
-                               rng_ptr, rng_start, rng_pref, leaf_src_total, floor2, X, Y, Z, q, k, kp, far, far_e,
-                               perm, out_mode, out, field);
-        if (n_leaves > n_fp32)
-            hipLaunchKernelGGL((p2p_field_kernel<float, true>), dim3(n_leaves - n_fp32), dim3(64), 0, s, n_fp32,
-                               leaf_box, bx, rng_ptr, rng_start, rng_pref, leaf_src_total, floor2, X, Y, Z, q, k,
-                               kp, far, far_e, perm, out_mode, out, field);
-    }
-    check_launch("p2p_field");
-}
-
 void launch_xlate(const XlateArgs& a, int n_targets, hipStream_t s) {
     if (n_targets <= 0) return;
     if (a.split < 1 || (a.split > 1 && !a.accumulate)) fail(-9, "xlate: split needs accumulate");
@@ -1581,55 +1027,6 @@ void launch_xlate(const XlateArgs& a, int n_targets, hipStream_t s) {
     const size_t shm = 2 * (size_t)nmx * sizeof(double2) + (kMaxP + 1) * sizeof(int);
     hipLaunchKernelGGL(xlate_kernel, dim3((unsigned)n_targets * (unsigned)a.split), dim3(kXlateThreads), shm, s, a);
     check_launch("xlate");
-}
-
-P2PArgs p2p_scaled(P2PArgs a, int precision, bool lowk) {
-    if (precision != 0) {
-        // coordinates in units of pi / k: the weights are e^{i pi u}/u with u = k r / pi
-        a.scale = lowk ? 1.0 : a.k / M_PI;
-        a.wscale = lowk ? 1.0 : a.k / M_PI;
-    }
-    return a;
-}
-
-template <int CLS>
-static const void* p2p_persistent_fn() {
-    return (const void*)p2p_persistent_kernel<CLS>;
-}
-
-static const void* p2p_persistent_class_fn(int cls) {
-    switch (cls) {
-        case kP2PClassFp64: return p2p_persistent_fn<kP2PClassFp64>();
-        case kP2PClassLowK: return p2p_persistent_fn<kP2PClassLowK>();
-        case kP2PClassPhase32: return p2p_persistent_fn<kP2PClassPhase32>();
-        default: return p2p_persistent_fn<kP2PClassPhase64>();
-    }
-}
-
-int p2p_persistent_grid(int cls) {
-    int dev = 0, cus = 0, per_cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, p2p_persistent_class_fn(cls), 64, 0))
-        fail(-3, "occupancy query (p2p persistent) failed");
-    return std::max(kXcds, (std::max(1, per_cu) * cus) / kXcds * kXcds);
-}
-
-void launch_p2p_persistent(int cls, const P2PBatchArgs* d_args, const WorkQueues& q, int grid, hipStream_t s) {
-    if (grid <= 0) return;
-    switch (cls) {
-        case kP2PClassFp64:
-            hipLaunchKernelGGL(p2p_persistent_kernel<kP2PClassFp64>, dim3(grid), dim3(64), 0, s, d_args, q);
-            break;
-        case kP2PClassLowK:
-            hipLaunchKernelGGL(p2p_persistent_kernel<kP2PClassLowK>, dim3(grid), dim3(64), 0, s, d_args, q);
-            break;
-        case kP2PClassPhase32:
-            hipLaunchKernelGGL(p2p_persistent_kernel<kP2PClassPhase32>, dim3(grid), dim3(64), 0, s, d_args, q);
-            break;
-        default:
-            hipLaunchKernelGGL(p2p_persistent_kernel<kP2PClassPhase64>, dim3(grid), dim3(64), 0, s, d_args, q);
-    }
-    check_launch("p2p persistent");
 }
 
 __global__ void clear_ints_kernel(int* p, int n) {
@@ -1641,81 +1038,6 @@ void launch_clear_ints(int* p, int n, hipStream_t s) {
     if (n <= 0) return;
     hipLaunchKernelGGL(clear_ints_kernel, dim3((n + 255) / 256), dim3(256), 0, s, p, n);
     check_launch("clear");
-}
-
-template <int R>
-static void launch_p2p_mixed(P2PArgs a, int n_leaves, int n_fp32, bool lowk, hipStream_t s) {
-    a = p2p_scaled(a, 1, lowk);
-    if (lowk) {
-        hipLaunchKernelGGL((p2p_mixed_kernel<false, true, R>), dim3(n_leaves), dim3(64), 0, s, a);
-        return;
-    }
-    if (n_fp32 > 0) hipLaunchKernelGGL((p2p_mixed_kernel<false, false, R>), dim3(n_fp32), dim3(64), 0, s, a);
-    if (n_leaves > n_fp32) {
-        a.leaf0 = n_fp32;
-        hipLaunchKernelGGL((p2p_mixed_kernel<true, false, R>), dim3(n_leaves - n_fp32), dim3(64), 0, s, a);
-    }
-}
-
-void launch_p2p(const P2PArgs& a0, int precision, int n_leaves, int n_fp32, bool lowk, int tile, hipStream_t s) {
-    if (n_leaves <= 0) return;
-    P2PArgs a = a0;
-    a.leaf0 = 0;
-    if (precision == 0)
-        hipLaunchKernelGGL(p2p_fp64_kernel, dim3(n_leaves), dim3(64), 0, s, a);
-    else if (tile == 1)
-        launch_p2p_mixed<1>(a, n_leaves, n_fp32, lowk, s);
-    else if (tile == 4)
-        launch_p2p_mixed<4>(a, n_leaves, n_fp32, lowk, s);
-    else
-        launch_p2p_mixed<2>(a, n_leaves, n_fp32, lowk, s);
-    check_launch("p2p");
-}
-
-// One wave per leaf: lane t holds target t of a 64-target chunk; every source of the leaf is
-// read by all lanes (uniform loads), FP64 throughout.
-__global__ __launch_bounds__(64) void p2p_coord_check_kernel(P2PArgs a, double tol, unsigned char* flag) {
-    const int leaf = blockIdx.x;
-    const int b = a.leaf_box[leaf];
-    const int tstart = a.bx.pstart[b], tcnt = a.bx.count[b];
-    const double cx = a.bx.centre[3 * b], cy = a.bx.centre[3 * b + 1], cz = a.bx.centre[3 * b + 2];
-    const int r0 = a.rng_ptr[leaf], r1 = a.rng_ptr[leaf + 1];
-    const int S = a.leaf_src_total[leaf];
-    const double fl2 = a.floor2[leaf];
-    const int lane = threadIdx.x;
-    double cmax = 0.0, ratio = 0.0;
-    for (int t0 = 0; t0 < tcnt; t0 += 64) {
-        const bool has = t0 + lane < tcnt;
-        const int it = tstart + t0 + (has ? lane : 0);
-        const double xt = a.X[it] - cx, yt = a.Y[it] - cy, zt = a.Z[it] - cz;
-        if (has) cmax = fmax(cmax, fmax(fabs(xt), fmax(fabs(yt), fabs(zt))));
-        double s2 = 0.0, s4 = 0.0;
-        int ri = r0;
-        for (int v = 0; v < S; ++v) {
-            const int idx = p2p_source_index(v, r1, a.rng_start, a.rng_pref, ri);
-            const double xs = a.X[idx] - cx, ys = a.Y[idx] - cy, zs = a.Z[idx] - cz;
-            if (t0 == 0) cmax = fmax(cmax, fmax(fabs(xs), fmax(fabs(ys), fabs(zs))));
-            const double dx = xt - xs, dy = yt - ys, dz = zt - zs;
-            const double r2 = dx * dx + dy * dy + dz * dz;
-            if (r2 > fl2) {
-                const double w = 1.0 / r2;
-                s2 += w;
-                s4 += w * w;
-            }
-        }
-        if (has && s2 > 0.0) ratio = fmax(ratio, sqrt(s4 / s2));
-    }
-    for (int off = 1; off < 64; off <<= 1) {
-        cmax = fmax(cmax, __shfl_xor(cmax, off));
-        ratio = fmax(ratio, __shfl_xor(ratio, off));
-    }
-    if (lane == 0) flag[leaf] = 0x1p-21 * cmax * ratio <= tol ? 1 : 0;
-}
-
-void launch_p2p_coord_check(const P2PArgs& a, int n, double tol, unsigned char* flag, hipStream_t s) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(p2p_coord_check_kernel, dim3(n), dim3(64), 0, s, a, tol, flag);
-    check_launch("p2p coordinate check");
 }
 
 void launch_direct(const double* X, const double* Y, const double* Z, const double2* q, int64_t n, double k,

@@ -148,8 +148,11 @@ struct hfmm_plan {
     double* d_R = nullptr;
     int* d_far_leaves = nullptr;
     LeafDesc* d_leafdesc = nullptr;   // per far leaf (d_far_leaves order): P2M / L2P descriptors
-    int *d_leaf_box = nullptr, *d_rng_ptr = nullptr, *d_rng_start = nullptr, *d_rng_pref = nullptr,
-        *d_leaf_src_total = nullptr;
+    int *d_leaf_box = nullptr, *d_batch_ptr = nullptr, *d_rng_delta = nullptr, *d_leaf_src_total = nullptr;
+    NearBatch* d_batches = nullptr;
+    NearItems near_items[2], field_items[2];   // FP32-phase (or FP64) leaves, FP64-phase leaves
+    std::vector<int> leaf_box, leaf_total;     // plans of a batch: box and sources of each
+                                               // leaf, whose items the batch makes anew
     double* d_rot = nullptr;
     double2* d_phase = nullptr;
     DispInfo* d_dinfo = nullptr;
@@ -1086,6 +1089,70 @@ void build_tables(hfmm_plan& P) {
 
 P2PArgs p2p_args(const hfmm_plan& P, int out_mode, double2* out);
 
+// Near-field work items.  A leaf's targets go in chunks of up to 64 R (R per lane of a wave); a
+// remainder that is not a power of two (and above 4 R) goes as its largest power of two first, so
+// that few target slots of the R x L lanes are idle.  Chunks of more than `limit` pairs are halved,
+// down to 16 targets (each chunk stages the leaf's sources once more: about a tenth of the work of
+// 16 targets).
+struct NearWork {
+    std::vector<NearItem> items;
+    std::vector<int> prob;
+    std::vector<int64_t> cost;
+    void add(const Tree& t, const std::vector<int>& leaf_box, const std::vector<int>& total, int l0, int l1, int R,
+             int64_t limit, int problem) {
+        for (int l = l0; l < l1; ++l) {
+            const int b = leaf_box[l], n = t.count[b];
+            int cap = 16;
+            while (2 * cap <= 64 * R && (int64_t)2 * cap * total[l] <= limit) cap *= 2;
+            for (int t0 = 0, c = 0; t0 < n; t0 += c) {
+                c = std::min(n - t0, 64 * R);
+                if (c < 64 * R && c > 4 * R)
+                    while (c & (c - 1)) c &= c - 1;   // the largest power of two
+                c = std::min(c, cap);
+                items.push_back({l, b, t.pstart[b] + t0, c});
+                prob.push_back(problem);
+                cost.push_back((int64_t)(c + 8) * total[l] + 4096);
+            }
+        }
+    }
+    // Interleaved for the XCDs (workgroup i runs on XCD i % kXcds): XCD x takes a contiguous
+    // range of the (Morton ordered) items, so that its L2 holds one region's points, with 1 / 8 of
+    // the cost; within it the longest first, by powers of two.  Padded with empty items.
+    std::pair<std::vector<NearItem>, std::vector<int>> ordered() const {
+        int64_t sum = 0, acc = 0;
+        for (int64_t c : cost) sum += c;
+        std::vector<int> of[kXcds];
+        for (size_t i = 0; i < items.size(); ++i) {
+            of[std::min<int64_t>(kXcds - 1, (acc + cost[i] / 2) * kXcds / std::max<int64_t>(1, sum))].push_back((int)i);
+            acc += cost[i];
+        }
+        size_t most = 0;
+        for (auto& v : of) {
+            std::stable_sort(v.begin(), v.end(), [&](int x, int y) { return ilogb_cost(x) > ilogb_cost(y); });
+            most = std::max(most, v.size());
+        }
+        std::pair<std::vector<NearItem>, std::vector<int>> out;
+        out.first.assign(most * kXcds, NearItem{0, 0, 0, 0});
+        out.second.assign(most * kXcds, 0);
+        for (int x = 0; x < kXcds; ++x)
+            for (size_t i = 0; i < of[x].size(); ++i) {
+                out.first[i * kXcds + x] = items[of[x][i]];
+                out.second[i * kXcds + x] = prob[of[x][i]];
+            }
+        return out;
+    }
+    int ilogb_cost(int i) const { return 63 - __builtin_clzll((unsigned long long)cost[i]); }
+};
+
+// Pairs up to which a chunk stays whole: a thousandth of those of the launch, a quarter of a
+// SIMD's share on each of the kNearWaves that take it.
+int64_t near_pairs(const std::vector<int>& leaf_box, const std::vector<int>& total, const Tree& t, int l0, int l1) {
+    int64_t pairs = 0;
+    for (int l = l0; l < l1; ++l) pairs += (int64_t)total[l] * t.count[leaf_box[l]];
+    return pairs;
+}
+int64_t near_limit(int64_t pairs) { return pairs / 1024; }
+
 void build_p2p(hfmm_plan& P) {
     const Tree& t = P.tree;
     const Lists& ls = P.lists;
@@ -1137,7 +1204,8 @@ void build_p2p(hfmm_plan& P) {
     }
     P.n_p2p_fp32 = (int)leaves[0].size();
     P.p2p_lowk = P.precision == HFMM_PREC_MIXED && kr_max <= kP2PLowKr;
-    std::vector<int> leaf_box, rng_ptr{0}, rng_start, rng_pref, total;
+    std::vector<int> leaf_box, batch_ptr{0}, rng_delta, total;
+    std::vector<NearBatch> batches;
     std::vector<double> floor2;
     std::vector<int> far_leaves;
     int64_t pairs = 0;
@@ -1148,18 +1216,24 @@ void build_p2p(hfmm_plan& P) {
             leaf_box.push_back(b);
             int acc = 0;
             double src_maxabs = 0.0;
+            const size_t batch0 = batches.size();
+            // a range of the leaf's sources: its start in the batch it begins in, and the batches
+            // that begin within it
             auto add = [&](int box) {
-                rng_start.push_back(t.pstart[box]);
-                rng_pref.push_back(acc);
-                acc += t.count[box];
                 src_maxabs = std::max(src_maxabs, P.box_maxabs[box]);
+                if (t.count[box] == 0) return;
+                const int range = (int)rng_delta.size();
+                rng_delta.push_back(t.pstart[box] - acc);
+                if (acc % 64) batches[batch0 + acc / 64].mask |= 1ull << (acc % 64);
+                acc += t.count[box];
+                while ((int)(batches.size() - batch0) * 64 < acc) batches.push_back({0, range, 0});
             };
             add(b);
             for (int e = up[b]; e < up[b + 1]; ++e) add(us[e]);
             for (int e = wp[b]; e < wp[b + 1]; ++e) add(ws[e]);
             for (int a = b; a >= 0; a = t.parent[a])
                 for (int e = xp[a]; e < xp[a + 1]; ++e) add(xs[e]);
-            rng_ptr.push_back((int)rng_start.size());
+            batch_ptr.push_back((int)batches.size());
             total.push_back(acc);
             // the reference's coincidence floor (jaxfmm/near.py:252-261, "pair" form in FP64):
             // pairs with r <= 16 eps (max |x_t| + max |x_s|) contribute nothing
@@ -1172,12 +1246,28 @@ void build_p2p(hfmm_plan& P) {
     P.n_p2p_pairs = pairs;
     P.d_leaf_box = P.upload(leaf_box);
     P.d_far_leaves = P.upload(far_leaves);
-    P.d_rng_ptr = P.upload(rng_ptr);
-    P.d_rng_start = P.upload(rng_start);
-    P.d_rng_pref = P.upload(rng_pref);
+    P.d_batch_ptr = P.upload(batch_ptr);
+    P.d_batches = P.upload(batches);
+    P.d_rng_delta = P.upload(rng_delta);
     P.d_leaf_src_total = P.upload(total);
     P.d_floor2 = P.upload(floor2);
     P.box_maxabs = std::vector<double>();
+    for (int cls = 0; cls < 2; ++cls) {
+        const int l0 = cls ? P.n_p2p_fp32 : 0, l1 = cls ? P.n_leaves : P.n_p2p_fp32;
+        const int R = P.precision == HFMM_PREC_FP64 ? kP2PFp64TargetsPerLane : P.p2p_tile;
+        for (auto& [dst, r] : {std::make_pair(&P.near_items[cls], R),
+                               std::make_pair(&P.field_items[cls], kP2PFieldTargetsPerLane)}) {
+            NearWork w;
+            w.add(t, leaf_box, total, l0, l1, r, near_limit(near_pairs(leaf_box, total, t, l0, l1)), 0);
+            const std::vector<NearItem> items = w.ordered().first;
+            dst->n = (int)items.size();
+            dst->items = P.upload(items);
+        }
+    }
+    if (P.in_batch) {
+        P.leaf_box = std::move(leaf_box);
+        P.leaf_total = std::move(total);
+    }
     // FP32-phase leaves whose estimated error from FP32 coordinate differences is within
     // p2p_coord32_tol take them (the check runs once, on the GPU, in FP64)
     if (P.precision == HFMM_PREC_MIXED && !P.p2p_lowk && P.p2p_coord32_tol > 0.0 && P.n_p2p_fp32 > 0) {
@@ -1497,9 +1587,9 @@ P2PArgs p2p_args(const hfmm_plan& P, int out_mode, double2* out) {
     P2PArgs pa{};
     pa.leaf_box = P.d_leaf_box;
     pa.bx = P.boxes();
-    pa.rng_ptr = P.d_rng_ptr;
-    pa.rng_start = P.d_rng_start;
-    pa.rng_pref = P.d_rng_pref;
+    pa.batch_ptr = P.d_batch_ptr;
+    pa.batches = P.d_batches;
+    pa.rng_delta = P.d_rng_delta;
     pa.leaf_src_total = P.d_leaf_src_total;
     pa.floor2 = P.d_floor2;
     pa.X = P.dX;
@@ -1636,12 +1726,13 @@ void run_sequence(hfmm_plan& P, const void* q, int q_type, double2* out, hipStre
         mark(6);
     }
     if (parts & kSeqP2P) {
+        P2PArgs pa = p2p_args(P, out_mode, out);
+        pa.far_e = P.d_far_e;
+        pa.field = field;
         if (field)
-            launch_p2p_field(P.precision, P.n_leaves, P.n_p2p_fp32, P.d_leaf_box, bx, P.d_rng_ptr, P.d_rng_start,
-                             P.d_rng_pref, P.d_leaf_src_total, P.d_floor2, P.dX, P.dY, P.dZ, P.d_q, P.k, P.d_far,
-                             P.d_far_e, P.d_perm, out_mode, out, field, s);
+            launch_p2p_field(pa, P.field_items, P.precision, s);
         else
-            launch_p2p(p2p_args(P, out_mode, out), P.precision, P.n_leaves, P.n_p2p_fp32, P.p2p_lowk, P.p2p_tile, s);
+            launch_p2p(pa, P.near_items, P.precision, P.p2p_lowk, P.p2p_tile, s);
         mark(7);
     }
 }
@@ -2152,9 +2243,10 @@ struct hfmm_batch {
     };
     std::vector<M2LInstance> m2l_inst;
     std::vector<const M2LBlockArgs*> m2l_args;   // device descriptors per instance
-    const P2PBatchArgs* d_p2p_args = nullptr;
-    WorkQueues p2p_q[4]{};                 // per near-field leaf class (kP2PClass*)
-    int p2p_grid[4] = {0, 0, 0, 0};
+    const P2PArgs* d_p2p_args = nullptr;
+    const NearItem* p2p_items[4] = {};     // per near-field leaf class (kP2PClass*)
+    const int* p2p_prob[4] = {};
+    int p2p_n[4] = {};
     int* d_counters = nullptr;
     int n_counters = 0;
     std::vector<void*> pallocs;             // device buffers of the persistent launches
@@ -2245,7 +2337,7 @@ void build_persistent(hfmm_batch& B, void* const* out, int q_type) {
             waves[pk].push_back({P, &c});
             wave_groups[pk] += c.n_groups;
         }
-    B.n_counters = 16 * kXcds * ((int)groups.size() + 4);
+    B.n_counters = 16 * kXcds * (int)groups.size();
     std::vector<int> zeros(B.n_counters, 0);
     B.d_counters = B.upload(zeros);
     int qi = 0;
@@ -2294,23 +2386,41 @@ void build_persistent(hfmm_batch& B, void* const* out, int q_type) {
         in.args = B.upload(args);
         B.wave_inst.push_back(in);
     }
-    std::vector<P2PBatchArgs> pa(np);
-    std::vector<int2> work[4];
-    for (int i = 0; i < np; ++i) {
-        hfmm_plan& P = *B.plans[i];
-        pa[i].a = p2p_scaled(p2p_args(P, out_mode_of(P, q_type), (double2*)out[i]), P.precision, P.p2p_lowk);
-        for (int l = 0; l < P.n_leaves; ++l) {
-            const int cls = P.precision == HFMM_PREC_FP64 ? kP2PClassFp64
-                            : P.p2p_lowk                  ? kP2PClassLowK
-                            : l < P.n_p2p_fp32            ? kP2PClassPhase32
-                                                          : kP2PClassPhase64;
-            work[cls].push_back(make_int2(i, l));
-        }
-    }
+    std::vector<P2PArgs> pa(np);
+    // leaves [l0, l1) of a problem in near-field class cls
+    auto leaves = [](const hfmm_plan& P, int cls) {
+        const bool fp64 = P.precision == HFMM_PREC_FP64;
+        if (fp64 ? cls != kP2PClassFp64 : P.p2p_lowk ? cls != kP2PClassLowK : cls < kP2PClassPhase32)
+            return std::make_pair(0, 0);
+        if (fp64 || P.p2p_lowk) return std::make_pair(0, P.n_leaves);
+        return cls == kP2PClassPhase32 ? std::make_pair(0, P.n_p2p_fp32) : std::make_pair(P.n_p2p_fp32, P.n_leaves);
+    };
+    for (int i = 0; i < np; ++i)
+        pa[i] = p2p_scaled(p2p_args(*B.plans[i], out_mode_of(*B.plans[i], q_type), (double2*)out[i]),
+                           B.plans[i]->precision, B.plans[i]->p2p_lowk);
     B.d_p2p_args = B.upload(pa);
     for (int c = 0; c < 4; ++c) {
-        B.p2p_q[c] = make_queues(B, work[c], B.d_counters + 16 * kXcds * (qi + c));
-        B.p2p_grid[c] = work[c].empty() ? 0 : p2p_persistent_grid(c);
+        int64_t pairs = 0;
+        for (const hfmm_plan* P : B.plans) {
+            const auto [l0, l1] = leaves(*P, c);
+            pairs += near_pairs(P->leaf_box, P->leaf_total, P->tree, l0, l1);
+        }
+        NearWork w;
+        for (int i = 0; i < np; ++i) {
+            const hfmm_plan& P = *B.plans[i];
+            const auto [l0, l1] = leaves(P, c);
+            // the chunks of a mixed problem are those of its plan alone: they decide which sources
+            // are summed in FP32, and a batch gives each problem's own result
+            if (c == kP2PClassFp64)
+                w.add(P.tree, P.leaf_box, P.leaf_total, l0, l1, kP2PFp64TargetsPerLane, near_limit(pairs), i);
+            else
+                w.add(P.tree, P.leaf_box, P.leaf_total, l0, l1, kP2PBatchTargetsPerLane,
+                      near_limit(near_pairs(P.leaf_box, P.leaf_total, P.tree, l0, l1)), i);
+        }
+        const auto [items, prob] = w.ordered();
+        B.p2p_n[c] = (int)items.size();
+        B.p2p_items[c] = B.upload(items);
+        B.p2p_prob[c] = B.upload(prob);
     }
 }
 
@@ -2354,7 +2464,7 @@ void batch_sequence(hfmm_batch& B, const void* const* q, int q_type, void* const
     }
     mark(3);
     // the near field of every problem: one persistent launch per leaf class
-    for (int c = 0; c < 4; ++c) launch_p2p_persistent(c, B.d_p2p_args, B.p2p_q[c], B.p2p_grid[c], s);
+    for (int c = 0; c < 4; ++c) launch_p2p_batch(c, B.d_p2p_args, B.p2p_items[c], B.p2p_prob[c], B.p2p_n[c], s);
     mark(4);
 }
 
