@@ -5,7 +5,6 @@
 #include <algorithm>
 #include <array>
 #include <chrono>
-#include <climits>
 #include <cmath>
 #include <cstring>
 #include <functional>
@@ -673,7 +672,8 @@ void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt
                    const std::vector<double>& coax, int n_dist, const std::vector<DispInfo>& dinfo) {
     const int ps = P.p_level[src_level], pt = P.p_level[tgt_level], pm = std::max(ps, pt);
     if (P.m2l_kernel != 0 || pm > kWave64MaxP || !P.d_cr1) return;
-    if (P.n_sd > INT_MAX) return;   // 32-bit source offsets
+    // the kernel addresses the sources with 32-bit byte offsets
+    if ((P.n_sd + wave_sd_pad(P.pmax)) * (int64_t)sizeof(double4) > (int64_t)UINT32_MAX) return;
     const Tree& t = P.tree;
     const int nt = (int)targets.size();
     constexpr int pairs = kWave64Pairs;
