@@ -305,8 +305,9 @@ struct M2LWaveArgs {
     const int4* items;               // (block, first group, end group, part): part 0 is the whole
                                      // block, s > 0 leaves its sums in slot s - 1 of `part`
     int n_blocks;
-    double4* part;                   // partial sums of split blocks (null: none), per slot and
-                                     // accumulator register 4 tb values
+    void* part;                      // partial sums of split blocks (null: none); FP64: per slot
+                                     // and accumulator register 4 tb double4, FP32: per slot the
+                                     // U, then the V entries, 2 tb floats each
     const int* part_ptr;             // n_blocks + 1: the slots of each block
     int tb;                          // targets per block, a power of two up to the pairs per group
     const int* blk_targets;          // blocks x tb target boxes (-1: empty slot)
@@ -314,12 +315,12 @@ struct M2LWaveArgs {
     const int* grp_src;              // per pair of a group: source offset in (S, D) entries (no
                                      // pair: 0, a block of zeros)
     const unsigned short* grp_dir;   // per pair: direction
-    const double* rot1;              // fragments of E_n^T per theta (forward)
-    const double* rot3;              // fragments of E_n per theta (back)
+    const void* rot1;                // fragments of E_n^T per theta (forward)
+    const void* rot3;                // fragments of E_n per theta (back)
     int rot_stride;
-    const double2* phase;            // e^{i m phi} per direction
+    const void* phase;               // e^{i m phi} per direction
     int phase_stride;
-    const double* coax;
+    const void* coax;
     int coax_stride;
     const void* M;                   // (S, D) entries
     double2* L;                      // expansions added to (x basis)
@@ -334,6 +335,42 @@ void launch_m2l_wave64_batch(const M2LWaveArgs* d_args, const int2* work, int n,
                              hipStream_t s);
 // the expansions of n_boxes consecutive boxes of degree p as (S_re, S_im, D_re, D_im) entries
 void launch_to_sd64(const double2* x, double4* sd, int64_t n_boxes, int p, hipStream_t s);
+
+// FP32 M2L with one wave per work item (m2l_wave32.hip), the lists as for FP64 with 32 pairs per
+// group and source offsets in pairs of (S, D) entries.  The operators are sequences of columns of four
+// rows (64 of them per 1 KiB block: wave32_pos).  Rotations, degrees from 1 ascending: split, for the u
+// half and from block kWave32VBlock for the v half, per input the output rows; joint, per input k the
+// u rows, then (k > 0) the v rows.  Coaxial operators, orders ascending: per input degree the real,
+// then the imaginary parts.
+constexpr int kWave32MaxP = 15;
+constexpr int kWave32Pairs = 32;
+// waves per SIMD: two (split layout) while the accumulators leave room in 256 registers, one (joint) above
+__host__ __device__ constexpr int wave32_wpe(int p) { return p <= 11 ? 2 : 1; }
+__host__ __device__ constexpr int wave32_rot_vecs(int h, int n) {   // columns of degrees below n of half h
+    int v = 0;
+    for (int j = 1; j < n; ++j) v += (j + 4 - h) / 4 * (j + 1 - h);
+    return v;
+}
+__host__ __device__ constexpr int wave32_joint_vecs(int n) { return wave32_rot_vecs(0, n) + wave32_rot_vecs(1, n); }
+__host__ __device__ constexpr int wave32_blocks(int vecs) { return (vecs + 63) / 64; }
+constexpr int kWave32VBlock = wave32_blocks(wave32_rot_vecs(0, kWave32MaxP + 1));   // first block of the v rotations
+// a theta's rotations: the split layout, then the joint one
+constexpr int kWave32SplitFloats = 256 * (kWave32VBlock + wave32_blocks(wave32_rot_vecs(1, kWave32MaxP + 1)));
+constexpr int kWave32RotFloats = kWave32SplitFloats + 256 * wave32_blocks(wave32_joint_vecs(kWave32MaxP + 1));
+__host__ __device__ constexpr int wave32_coax_vecs(int p, int m) {   // columns of orders below m
+    int v = 0;
+    for (int j = 0; j < m; ++j) v += 2 * ((p + 1 - j + 3) / 4) * (p + 1 - j);
+    return v;
+}
+constexpr int wave32_pos(int v, int i) { return ((v / 64) * 64 + 4 * (v % 16) + i) * 4 + v % 64 / 16; }   // row i of column v
+// pairs of the block of zeros at the front, which degrees above a source's read
+constexpr int wave32_sd_pad(int pmax) { return (pmax + 1) * (pmax + 2) / 4 + 8; }
+void launch_m2l_wave32(const M2LWaveArgs& a, int p, hipStream_t s);
+int wave32_sum_chunks(int p, int tb);
+void launch_m2l_wave32_batch(const M2LWaveArgs* d_args, const int2* work, int n, const int4* sums, int n_sums, int p,
+                             hipStream_t s);
+// the expansions of n_boxes consecutive boxes of degree p as FP32 pairs of entries
+void launch_to_sd32(const double2* x, float4* sd, int64_t n_boxes, int p, hipStream_t s);
 
 // near field of the problems of a batch: one launch per leaf class (FP64 plans; mixed plans with
 // k r <= kP2PLowKr; mixed, FP32 phase; mixed, FP64 phase) over items of all problems,

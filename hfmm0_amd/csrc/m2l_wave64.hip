@@ -125,15 +125,15 @@ __device__ __forceinline__ void wave64_body(const M2LWaveArgs& a, const int4 ite
 #pragma unroll 1
     for (int e = item.y; e < item.z; ++e) {
         const int cls = ((ScalarInts)a.grp_class)[e];   // theta | dist << 16
-        const double2* R1 = (const double2*)(a.rot1 + (size_t)(cls & 0xFFFF) * a.rot_stride);
-        const double2* R3 = (const double2*)(a.rot3 + (size_t)(cls & 0xFFFF) * a.rot_stride);
-        const double2* T = (const double2*)(a.coax + (size_t)(cls >> 16) * a.coax_stride);
+        const double2* R1 = (const double2*)((const double*)a.rot1 + (size_t)(cls & 0xFFFF) * a.rot_stride);
+        const double2* R3 = (const double2*)((const double*)a.rot3 + (size_t)(cls & 0xFFFF) * a.rot_stride);
+        const double2* T = (const double2*)((const double*)a.coax + (size_t)(cls >> 16) * a.coax_stride);
         const uint32_t lane16 = 16 * (uint32_t)lane;
         // (S, D) entries of the source; degrees above the source's read the block of zeros
         const uint32_t so = 32 * (uint32_t)(src + lk), sz = 32 * (uint32_t)lk;
         double2 ph[KP];   // (cos, sin) of order 4 r + lk
 #pragma unroll
-        for (int r = 0; r < KP; ++r) ph[r] = a.phase[(size_t)dir * a.phase_stride + min(4 * r + lk, a.phase_stride - 1)];
+        for (int r = 0; r < KP; ++r) ph[r] = ((const double2*)a.phase)[(size_t)dir * a.phase_stride + min(4 * r + lk, a.phase_stride - 1)];
         // the next group's sources and directions are on their way while this one is processed
         const int en = e + 1 < item.z ? e + 1 : e;
         src = a.grp_src[(size_t)en * 16 + li];
@@ -288,7 +288,7 @@ __device__ __forceinline__ void wave64_body(const M2LWaveArgs& a, const int4 ite
             v.w += __shfl_xor(v.w, off);
         }
         if (item.w > 0) {   // one of several parts of the block: summed by wave64_sum_kernel
-            if (li < tb) a.part[((size_t)(item.w - 1) * NR + k) * (4 * tb) + tb * lk + li] = v;
+            if (li < tb) ((double4*)a.part)[((size_t)(item.w - 1) * NR + k) * (4 * tb) + tb * lk + li] = v;
         } else if (tbox >= 0 && li < tb) {
             store_expansion(a.L + a.exp_off[tbox], n, 4 * r + lk, pt, a.overwrite, v);
         }
@@ -309,7 +309,7 @@ __device__ __forceinline__ void wave64_sum(const M2LWaveArgs& a, int P, int b, i
     const int tb = a.tb, NR = regs_before(P + 1), total = NR * 4 * tb;
     const int e = threadIdx.x % kSumValues, j = threadIdx.x / kSumValues;
     const int t = min(chunk * kSumValues + e, total - 1), q = t % (4 * tb);
-    const double4* p = a.part + (size_t)s0 * total + t;
+    const double4* p = (const double4*)a.part + (size_t)s0 * total + t;
     double4 v = make_double4(0.0, 0.0, 0.0, 0.0);
     const int n_parts = s1 - s0;
     for (int s = j; s < n_parts; s += 4 * kSumSlices) {   // four loads in flight

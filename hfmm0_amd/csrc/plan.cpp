@@ -71,12 +71,13 @@ struct M2LBlockLevel {
     int* zero = nullptr;
 };
 
-// items an M2L launch of the wave kernel is split into (m2l_wave64.hip)
+// items an M2L launch of the FP64 wave kernel is split into (m2l_wave64.hip)
 constexpr int kWaveItems = 3072;
 
-// FP64 translation of one level with one wave per work item (m2l_wave64.hip)
+// Translation of one level with one wave per work item (m2l_wave64.hip, m2l_wave32.hip)
 struct M2LWaveLevel {
     bool use = false;
+    bool fp32 = false;
     int tb = 0;                    // targets per block
     int ps = 0, pt = 0;            // table degrees
     int src_level = 0, tgt_level = 0;
@@ -88,12 +89,13 @@ struct M2LWaveLevel {
     unsigned short* dir = nullptr;
     std::vector<double> tab;       // packed coaxial tables (host): fragments are made per degree
     int n_dist = 0;
-    double* coax = nullptr;        // fragments for the effective degrees
+    void* coax = nullptr;          // fragments for the effective degrees
     int coax_stride = 0;
     int n_blocks = 0, n_slots = 0;
     int* part_ptr = nullptr;
-    double4* part = nullptr;       // partial sums of blocks split over items, shared by the levels
+    void* part = nullptr;          // partial sums of blocks split over items, shared by the levels
     int n_groups = 0;
+    std::vector<int> host_part_ptr;            // ... FP32: the slots of the plan's own split
     std::vector<int> host_targets, host_ptr;   // plans of a batch: blocks and their groups,
                                    // which the batch splits anew
 };
@@ -159,12 +161,17 @@ struct hfmm_plan {
     M2LBlockLevel m2lb[kMaxLevels];
     bool m2l_fp32[kMaxLevels] = {};  // M2L of the level in FP32 (mixed precision)
     M2LBlockLevel m2mb[kMaxLevels], l2lb[kMaxLevels];   // M2M / L2L on matrix cores
-    M2LWaveLevel m2lc[kMaxLevels], m2mc[kMaxLevels], l2lc[kMaxLevels];   // FP64, one wave per item
+    M2LWaveLevel m2lc[kMaxLevels], m2mc[kMaxLevels], l2lc[kMaxLevels];   // one wave per item
     bool in_batch = false;           // one of a batch (also evaluated alone)
     std::vector<int64_t> sd_off;     // offset of each box's (S, D) entries
     int64_t n_sd = 0;
     double *d_cr1 = nullptr, *d_cr3 = nullptr;   // rotation fragments of the wave kernel
     int cr_stride = 0;
+    float *d_wr1 = nullptr, *d_wr3 = nullptr;    // ... and of its FP32 form
+    int wr_stride = 0;
+    std::vector<int64_t> sd32_off;   // offset of each box's FP32 (S, D) entries, in pairs
+    int64_t n_sd32 = 0;
+    float4* dMs32 = nullptr;         // multipoles as FP32 (S, D) entries, two float4 per pair
     double4 *dMs = nullptr, *dLs = nullptr;      // multipoles / parents' locals in (S, D) form
     int m2l_kernel = 0;
     int p2p_tile = 2;               // targets per lane of the mixed near field
@@ -641,9 +648,31 @@ void build_tree_blocks(hfmm_plan& P, int L, int kind, const std::vector<double>&
     prepare_m2l_block(pm, tb, grp, fp32);
 }
 
-// Coaxial fragments of a level for its effective degrees (m2l_wave64.hip), into B.coax
+// Coaxial fragments of a level for its effective degrees, into B.coax
 void pack_wave_coax(const hfmm_plan& P, M2LWaveLevel& B) {
     const int ps = P.p_eff[B.src_level], pt = P.p_eff[B.tgt_level], pm = std::max(ps, pt);
+    if (B.fp32) {
+        const int csz = coax_size(B.pt, B.ps);
+        B.coax_stride = 256 * wave32_blocks(wave32_coax_vecs(pm, pm + 1));
+        std::vector<float> cf((size_t)B.n_dist * B.coax_stride, 0.0f);
+        for (int d = 0; d < B.n_dist; ++d) {
+            size_t off = (size_t)d * csz;
+            float* f = &cf[(size_t)d * B.coax_stride];
+            for (int m = 0; m <= std::min(B.ps, B.pt); ++m) {
+                const int lens = B.ps + 1 - m, q = (pm + 1 - m + 3) / 4;
+                for (int n2 = m; n2 <= pt; ++n2)
+                    for (int n = m; n <= ps; ++n) {
+                        const size_t t = off + (size_t)(n2 - m) * lens + n - m;
+                        const int v = wave32_coax_vecs(pm, m) + 2 * q * (n - m) + (n2 - m) / 4;
+                        f[wave32_pos(v, (n2 - m) % 4)] = (float)B.tab[2 * t];
+                        f[wave32_pos(v + q, (n2 - m) % 4)] = (float)B.tab[2 * t + 1];
+                    }
+                off += (size_t)(B.pt + 1 - m) * lens;
+            }
+        }
+        HIPCHK(hipMemcpy(B.coax, cf.data(), cf.size() * sizeof(float), hipMemcpyHostToDevice));
+        return;
+    }
     const int regs = wave64_coax_regs(pm, pm + 1), csz = coax_size(B.pt, B.ps);
     B.coax_stride = regs * 128;
     std::vector<double> cf((size_t)B.n_dist * B.coax_stride, 0.0);
@@ -669,14 +698,16 @@ void pack_wave_coax(const hfmm_plan& P, M2LWaveLevel& B) {
 // kind 0: M2L, 1: M2M, 2: L2L; coax: packed tables as X.coax (interleaved complex).
 void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt_level, const std::vector<int>& targets,
                    const std::vector<int>& ptr, const std::vector<int>& src, const std::vector<unsigned short>& dir,
-                   const std::vector<double>& coax, int n_dist, const std::vector<DispInfo>& dinfo) {
+                   const std::vector<double>& coax, int n_dist, const std::vector<DispInfo>& dinfo, bool fp32 = false) {
     const int ps = P.p_level[src_level], pt = P.p_level[tgt_level], pm = std::max(ps, pt);
-    if (P.m2l_kernel != 0 || pm > kWave64MaxP || !P.d_cr1) return;
-    // the kernel addresses the sources with 32-bit byte offsets
-    if ((P.n_sd + wave_sd_pad(P.pmax)) * (int64_t)sizeof(double4) > (int64_t)UINT32_MAX) return;
+    if (P.m2l_kernel != 0 || pm > (fp32 ? kWave32MaxP : kWave64MaxP) || !P.d_cr1) return;
+    // the kernels address the sources with 32-bit byte offsets
+    const int64_t bytes = fp32 ? (P.n_sd32 + wave32_sd_pad(P.pmax)) * 2 * (int64_t)sizeof(float4)
+                               : (P.n_sd + wave_sd_pad(P.pmax)) * (int64_t)sizeof(double4);
+    if (bytes > (int64_t)UINT32_MAX) return;
     const Tree& t = P.tree;
     const int nt = (int)targets.size();
-    constexpr int pairs = kWave64Pairs;
+    const int pairs = fp32 ? kWave32Pairs : kWave64Pairs;
     // classes (theta, dist) present, and the targets ordered by the octant's z bit, then in
     // space: V displacements of one z bit have the same classes
     std::vector<int> cls_of(kNumDirs, -1), cls_key;
@@ -702,11 +733,11 @@ void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt
     std::vector<unsigned short> cnt((size_t)nt * nc, 0);
     for (int i = 0; i < nt; ++i)
         for (int e = ptr[i]; e < ptr[i + 1]; ++e) ++cnt[(size_t)i * nc + cls_of[dir[e]]];
-    // targets per block: the one with the fewest groups (each is 16 pairs of work); on a tie the
+    // targets per block: the one with the fewest groups (each is 16 or 32 pairs of work); on a tie the
     // smaller, whose blocks are more and end in fewer stores
     int tb = 0;
-    int64_t best = 0;
-    for (int c : {2, 4, 8, 16}) {
+    int64_t best = 0, best_cost = 0;
+    for (int c = 2; c <= pairs; c *= 2) {
         const int slots = pairs / c;
         int64_t g = 0;
         for (int b0 = 0; b0 < nt; b0 += c)
@@ -715,7 +746,10 @@ void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt
                 for (int j = b0; j < std::min(nt, b0 + c); ++j) mx = std::max<int>(mx, cnt[(size_t)order[j] * nc + k]);
                 g += (mx + slots - 1) / slots;
             }
-        if (!tb || g < best) tb = c, best = g;
+        // FP32: an item leaves c targets' sums in memory, about c / 64 of a group's time.  On 5.4M pairs
+        // c = 16 and 32 both need 193.6k groups; the sums of 32 took 157 us against 65.
+        const int64_t cost = g + (fp32 ? (int64_t)kWaveItems * c / 64 : 0);
+        if (!tb || cost < best_cost) tb = c, best = g, best_cost = cost;
     }
     // The kernel's code for one group is straight-line, 15 to 40 KB, and every compute unit
     // fetches it once: a launch of a group or two per wave spends most of its time on that (M2M
@@ -747,13 +781,14 @@ void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt
             for (int e = ptr[i]; e < ptr[i + 1]; ++e) {
                 const int k = cls_of[dir[e]], f = fill[k]++;
                 const size_t o = (size_t)(first[k] + f / slots) * pairs + (f % slots) * tb + (j - j0);
-                gsrc[o] = (int)P.sd_off[src[e]];
+                gsrc[o] = (int)(fp32 ? P.sd32_off : P.sd_off)[src[e]];
                 gdir[o] = dir[e];
             }
         }
         blk_ptr.push_back((int)gcls.size());
     }
     B.use = true;
+    B.fp32 = fp32;
     B.tb = tb;
     B.ps = ps;
     B.pt = pt;
@@ -765,20 +800,39 @@ void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt
     B.dir = P.upload(gdir);
     B.tab = coax;
     B.n_dist = n_dist;
-    B.coax = P.alloc<double>((size_t)n_dist * wave64_coax_regs(pm, pm + 1) * 128);
+    B.coax = P.alloc<char>((size_t)n_dist * (fp32 ? 256 * wave32_blocks(wave32_coax_vecs(pm, pm + 1)) * sizeof(float)
+                                                  : wave64_coax_regs(pm, pm + 1) * 128 * sizeof(double)));
     pack_wave_coax(P, B);
     B.n_blocks = nblk;
     B.n_groups = blk_ptr[nblk];
-    // M2L blocks are split into items whose sums meet in a second kernel: three items for each
-    // wave that runs at a time (1024 SIMDs)
+    // M2L blocks are split into items whose sums meet in a second kernel
     std::vector<int> part_ptr;
-    const std::vector<int4> items = wave_items(
-        t, blk_targets, blk_ptr, tb, kind == 0 ? std::max(1, (B.n_groups + kWaveItems - 1) / kWaveItems) : B.n_groups, part_ptr);
+    int per_item = B.n_groups;
+    if (kind == 0 && fp32) {
+        // An item's start and end cost about half a group, and a wave too many a whole round: one
+        // item for each wave that runs at a time, up to three where they keep 16 groups.  The 2900
+        // items of a group or two that a fixed 3072 gave 512 targets at p = 11 took 82 us, 1024 43;
+        // 4096 targets at p = 12 in 3040 items 0.32 + 0.03 ms (sums), in 960 0.315 + 0.009.
+        const int slots = 1024 * wave32_wpe(pm);
+        const int64_t max_items = (int64_t)slots * std::max(1, std::min(3, B.n_groups / slots / 16));
+        int most = 1;
+        for (int b = 0; b < nblk; ++b) most = std::max(most, blk_ptr[b + 1] - blk_ptr[b]);
+        for (per_item = std::max<int>(1, B.n_groups / max_items); per_item < most; per_item += 1 + per_item / 32) {
+            int64_t n = 0;
+            for (int b = 0; b < nblk; ++b) n += std::max(1, (blk_ptr[b + 1] - blk_ptr[b] + per_item - 1) / per_item);
+            if (n <= max_items) break;
+        }
+    } else if (kind == 0) {
+        // three items for each wave that runs at a time (1024 SIMDs)
+        per_item = std::max(1, (B.n_groups + kWaveItems - 1) / kWaveItems);
+    }
+    const std::vector<int4> items = wave_items(t, blk_targets, blk_ptr, tb, per_item, part_ptr);
     B.n_items = (int)items.size();
     B.items = P.upload(items);
     B.n_slots = part_ptr[nblk];
     B.part_ptr = P.upload(part_ptr);
-    if (P.in_batch && kind == 0) {
+    if (P.in_batch && kind == 0 && fp32) B.host_part_ptr = part_ptr;
+    if (P.in_batch && kind == 0 && !fp32) {
         B.host_targets = std::move(blk_targets);
         B.host_ptr = std::move(blk_ptr);
     }
@@ -972,6 +1026,36 @@ void build_tables(hfmm_plan& P) {
                     }
             P.d_cr1 = P.upload(c1);
             P.d_cr3 = P.upload(c3);
+            if (P.precision == HFMM_PREC_MIXED) {
+                const int pw = std::min(pmax, kWave32MaxP);
+                P.wr_stride = kWave32RotFloats;
+                std::vector<float> w1((size_t)thetas.size() * P.wr_stride, 0.0f), w3(w1.size(), 0.0f);
+                for (size_t th = 0; th < thetas.size(); ++th)
+                    for (int n = 1; n <= pw; ++n)
+                        for (int st = 0; st < 2; ++st) {
+                            rotation_uv_blocks(&rot[th * rsz + rot_offset(n)], n, st == 0, Wu, Wv);
+                            float* f = &(st == 0 ? w1 : w3)[th * P.wr_stride];
+                            const int qu = n / 4 + 1, qv = (n + 3) / 4;
+                            const int u0 = wave32_rot_vecs(0, n), v0 = 64 * kWave32VBlock + wave32_rot_vecs(1, n);
+                            for (int k = 0; k <= n; ++k)
+                                for (int i = 0; i <= n; ++i)
+                                    f[wave32_pos(u0 + qu * k + i / 4, i % 4)] = (float)Wu[(size_t)i * (n + 1) + k];
+                            for (int k = 0; k < n; ++k)
+                                for (int i = 0; i < n; ++i)
+                                    f[wave32_pos(v0 + qv * k + i / 4, i % 4)] = (float)Wv[(size_t)i * n + k];
+                            f += kWave32SplitFloats;
+                            int v = wave32_joint_vecs(n);
+                            for (int k = 0; k <= n; ++k) {
+                                for (int i = 0; i <= n; ++i) f[wave32_pos(v + i / 4, i % 4)] = (float)Wu[(size_t)i * (n + 1) + k];
+                                v += qu;
+                                if (k == 0) continue;
+                                for (int i = 0; i < n; ++i) f[wave32_pos(v + i / 4, i % 4)] = (float)Wv[(size_t)i * n + k - 1];
+                                v += qv;
+                            }
+                        }
+                P.d_wr1 = P.upload(w1);
+                P.d_wr3 = P.upload(w3);
+            }
         }
     }
     std::vector<double2> phase((size_t)kNumDirs * (pmax + 1));
@@ -1026,8 +1110,7 @@ void build_tables(hfmm_plan& P) {
                 coax_table(0, G, P.k, 2.0 * P.h[L] * std::sqrt((double)dist_d2[i]), P.R[L], P.R[L], X.ps, X.pt,
                            &cx[i * X.coax_stride * 2]);
             X.coax = (double2*)P.upload(cx);
-            if (!P.m2l_fp32[L])
-                build_waves(P, P.m2lc[L], 0, L, L, targets, ptr, src, dir, cx, (int)dist_d2.size(), dinfo);
+            build_waves(P, P.m2lc[L], 0, L, L, targets, ptr, src, dir, cx, (int)dist_d2.size(), dinfo, P.m2l_fp32[L]);
             if (!P.m2lc[L].use) build_m2l_blocks(P, L, targets, ptr, src, dir, cx, (int)dist_d2.size(), dinfo);
         }
     }
@@ -1281,17 +1364,19 @@ void build_p2p(hfmm_plan& P) {
     }
 }
 
-size_t wave_part_size(const M2LWaveLevel& B, int n_slots) {
-    return (size_t)n_slots * wave64_regs(std::max(B.ps, B.pt)) * 4 * B.tb;
+size_t wave_part_bytes(const M2LWaveLevel& B, int n_slots) {
+    const int p = std::max(B.ps, B.pt);
+    return (size_t)n_slots * B.tb *
+           (B.fp32 ? 2 * (p + 1) * (p + 1) * sizeof(float) : 4 * wave64_regs(p) * sizeof(double4));
 }
 
 // The partial sums of the wave kernel's split blocks: one buffer for all levels, which run one
 // after another
 void alloc_wave_parts(hfmm_plan& P) {
     size_t most = 0;
-    for (const M2LWaveLevel& B : P.m2lc) most = std::max(most, wave_part_size(B, B.n_slots));
+    for (const M2LWaveLevel& B : P.m2lc) most = std::max(most, wave_part_bytes(B, B.n_slots));
     if (!most) return;
-    double4* all = P.alloc<double4>(most);
+    void* all = P.alloc<char>(most);
     for (M2LWaveLevel& B : P.m2lc)
         if (B.n_slots) B.part = all;
 }
@@ -1377,6 +1462,7 @@ void build_plan(hfmm_plan& P, const double* xyz, int64_t n, double k, const hfmm
     std::vector<double> centre(3 * (size_t)nb);
     P.exp_off.assign(nb, 0);
     P.sd_off.assign(nb, 0);
+    P.sd32_off.assign(nb, 0);
     int64_t off = 0;
     for (int b = 0; b < nb; ++b) {
         int gx, gy, gz;
@@ -1390,7 +1476,11 @@ void build_plan(hfmm_plan& P, const double* xyz, int64_t n, double k, const hfmm
         off += ncoef(P.p_level[t.level[b]]);
         if (b == 0) P.n_sd = wave_sd_pad(P.pmax);
         P.sd_off[b] = P.n_sd;
-        P.n_sd += (P.p_level[t.level[b]] + 1) * (P.p_level[t.level[b]] + 2) / 2;
+        const int entries = (P.p_level[t.level[b]] + 1) * (P.p_level[t.level[b]] + 2) / 2;
+        P.n_sd += entries;
+        if (b == 0) P.n_sd32 = wave32_sd_pad(P.pmax);
+        P.sd32_off[b] = P.n_sd32;
+        P.n_sd32 += (entries + 1) / 2;
     }
     P.n_coef = off;
     P.d_centre = P.upload(centre);
@@ -1437,9 +1527,10 @@ void build_plan(hfmm_plan& P, const double* xyz, int64_t n, double k, const hfmm
     if (any_fp32) P.dM32 = P.alloc<float2>(P.n_coef);
     P.dL = P.alloc<double2>(P.n_coef);
     if (any_l2l32) P.dL32 = P.alloc<float2>(P.n_coef);
-    bool any_col = false, any_l2l_col = false;
+    bool any_col = false, any_l2l_col = false, any_wave32 = false;
     for (int L = 0; L < kMaxLevels; ++L) {
-        any_col = any_col || P.m2lc[L].use || P.m2mc[L].use;
+        any_col = any_col || (P.m2lc[L].use && !P.m2lc[L].fp32) || P.m2mc[L].use;
+        any_wave32 = any_wave32 || (P.m2lc[L].use && P.m2lc[L].fp32);
         any_l2l_col = any_l2l_col || P.l2lc[L].use;
     }
     alloc_wave_parts(P);
@@ -1449,6 +1540,11 @@ void build_plan(hfmm_plan& P, const double* xyz, int64_t n, double k, const hfmm
             *buf = P.alloc<double4>(n_sd);
             HIPCHK(hipMemset(*buf, 0, n_sd * sizeof(double4)));
         }
+    if (any_wave32) {
+        const size_t n32 = 2 * (P.n_sd32 + wave32_sd_pad(P.pmax));
+        P.dMs32 = P.alloc<float4>(n32);
+        HIPCHK(hipMemset(P.dMs32, 0, n32 * sizeof(float4)));
+    }
     P.d_q = P.alloc<double2>(n);
     P.d_far = P.alloc<double2>(n);
     P.d_qin = P.alloc<double2>(n);
@@ -1520,7 +1616,7 @@ M2LBlockArgs block_args(const hfmm_plan& P, const M2LBlockLevel& B, bool fp32, c
     return a;
 }
 
-M2LWaveArgs wave_args(const hfmm_plan& P, const M2LWaveLevel& B, const double4* src, double2* dst, int overwrite) {
+M2LWaveArgs wave_args(const hfmm_plan& P, const M2LWaveLevel& B, const void* src, double2* dst, int overwrite) {
     M2LWaveArgs a;
     a.ps = P.p_eff[B.src_level];
     a.pt = P.p_eff[B.tgt_level];
@@ -1535,10 +1631,11 @@ M2LWaveArgs wave_args(const hfmm_plan& P, const M2LWaveLevel& B, const double4* 
     a.grp_class = B.cls;
     a.grp_src = B.src;
     a.grp_dir = B.dir;
-    a.rot1 = P.d_cr1;
-    a.rot3 = P.d_cr3;
-    a.rot_stride = P.cr_stride;
-    a.phase = P.d_phase;
+    const int layout = wave32_wpe(std::max(a.ps, a.pt)) == 1 ? kWave32SplitFloats : 0;
+    a.rot1 = B.fp32 ? (const void*)(P.d_wr1 + layout) : P.d_cr1;
+    a.rot3 = B.fp32 ? (const void*)(P.d_wr3 + layout) : P.d_cr3;
+    a.rot_stride = B.fp32 ? P.wr_stride : P.cr_stride;
+    a.phase = B.fp32 ? (const void*)P.d_phase32 : P.d_phase;
     a.phase_stride = P.pmax + 1;
     a.coax = B.coax;
     a.coax_stride = B.coax_stride;
@@ -1548,10 +1645,14 @@ M2LWaveArgs wave_args(const hfmm_plan& P, const M2LWaveLevel& B, const double4* 
     return a;
 }
 
-void launch_wave(const hfmm_plan& P, const M2LWaveLevel& B, const double4* src, double2* dst, int overwrite,
+const void* wave_source(const hfmm_plan& P, const M2LWaveLevel& B) {
+    return B.fp32 ? (const void*)P.dMs32 : P.dMs;
+}
+
+void launch_wave(const hfmm_plan& P, const M2LWaveLevel& B, const void* src, double2* dst, int overwrite,
                  hipStream_t s) {
     const M2LWaveArgs a = wave_args(P, B, src, dst, overwrite);
-    launch_m2l_wave64(a, std::max(a.ps, a.pt), s);
+    (B.fp32 ? launch_m2l_wave32 : launch_m2l_wave64)(a, std::max(a.ps, a.pt), s);
 }
 
 // parts of one evaluate's device sequence (a batch runs them for all problems, with the
@@ -1653,7 +1754,13 @@ void run_sequence(hfmm_plan& P, const void* q, int q_type, double2* out, hipStre
         // multipoles in FP32 for the FP32 block levels: every level not converted for an FP32
         // M2M (the converted ones need not be contiguous), one launch per run of levels
         for (int L = 2; L <= P.depth; ++L)
-            if (P.m2lc[L].use && !conv_sd[L]) level_to_sd(P, L, P.dM, P.dMs, s);
+            if (P.m2lc[L].use && P.m2lc[L].fp32) {
+                const Tree& t = P.tree;
+                const int b0 = t.level_start[L], b1 = t.level_start[L + 1];
+                launch_to_sd32(P.dM + P.exp_off[b0], P.dMs32 + 2 * P.sd32_off[b0], b1 - b0, P.p_level[L], s);
+            } else if (P.m2lc[L].use && !conv_sd[L]) {
+                level_to_sd(P, L, P.dM, P.dMs, s);
+            }
         bool any_fp32 = false;
         for (int L = 2; L <= P.depth; ++L) any_fp32 |= P.m2l[L].n_targets && P.m2lb[L].use && P.m2lb[L].fp32;
         if (any_fp32)
@@ -1675,7 +1782,7 @@ void run_sequence(hfmm_plan& P, const void* q, int q_type, double2* out, hipStre
         if (P.m2lc[L].use) {
             if (!(parts & kSeqM2LBlock)) continue;
             if (lev) HIPCHK(hipEventRecord(lev[2 * L], s));
-            launch_wave(P, P.m2lc[L], P.dMs, P.dL, 0, s);
+            launch_wave(P, P.m2lc[L], wave_source(P, P.m2lc[L]), P.dL, 0, s);
             if (lev) HIPCHK(hipEventRecord(lev[2 * L + 1], s));
             continue;
         }
@@ -1859,7 +1966,8 @@ int hfmm_plan_info_get(const hfmm_plan* P, hfmm_plan_info* info) {
         for (int L = 0; L < HFMM_MAX_LEVELS; ++L) {
             info->p_level[L] = (L >= 1 && L <= P->depth) ? P->p_eff[L] : 0;
             info->p_table[L] = (L >= 1 && L <= P->depth) ? P->p_level[L] : 0;
-            if (P->m2lb[L].use && P->m2lb[L].fp32) info->m2l_fp32_levels |= 1 << L;
+            if ((P->m2lb[L].use && P->m2lb[L].fp32) || (P->m2lc[L].use && P->m2lc[L].fp32))
+                info->m2l_fp32_levels |= 1 << L;
             if (P->m2mb[L].use && P->m2mb[L].fp32) info->m2m_fp32_levels |= 1 << L;
             if (P->l2lb[L].use && P->l2lb[L].fp32) info->l2l_fp32_levels |= 1 << L;
         }
@@ -2229,7 +2337,8 @@ struct hfmm_batch {
     int g_qtype = -1;
     // persistent launches over all problems (rebuilt with the graph): the block M2L, one
     // launch per kernel instance, and the near field
-    struct WaveInstance {                   // the FP64 wave kernel, one launch per degree
+    struct WaveInstance {                   // the wave kernels, one launch per degree
+        bool fp32 = false;
         int p = 0, n = 0, n_sums = 0;
         const int2* work = nullptr;
         const int4* sums = nullptr;
@@ -2328,14 +2437,17 @@ void build_persistent(hfmm_batch& B, void* const* out, int q_type) {
     // of a single level.  Split by level as for a plan alone, 16 problems of 2k to 20k points at
     // p = 10 made 36128 items, of a group or two each: 2.67 ms, and 0.29 for the sums, against
     // 1.37 and 0.05 for the 6016 items of this rule.
-    std::map<int, std::vector<std::pair<hfmm_plan*, const M2LWaveLevel*>>> waves;   // by degree
-    std::map<int, int64_t> wave_groups;
+    // FP32 levels keep their items: they decide what is summed in FP32, and a batch gives each
+    // problem's own result.
+    using WaveKey = std::pair<bool, int>;   // FP32, degree
+    std::map<WaveKey, std::vector<std::pair<hfmm_plan*, const M2LWaveLevel*>>> waves;
+    std::map<WaveKey, int64_t> wave_groups;
     for (hfmm_plan* P : B.plans)
         for (const M2LWaveLevel& c : P->m2lc) {
             if (!c.use || !c.n_groups) continue;
             const int pk = std::max(P->p_eff[c.src_level], P->p_eff[c.tgt_level]);
-            waves[pk].push_back({P, &c});
-            wave_groups[pk] += c.n_groups;
+            waves[{c.fp32, pk}].push_back({P, &c});
+            wave_groups[{c.fp32, pk}] += c.n_groups;
         }
     B.n_counters = 16 * kXcds * (int)groups.size();
     std::vector<int> zeros(B.n_counters, 0);
@@ -2359,24 +2471,30 @@ void build_persistent(hfmm_batch& B, void* const* out, int q_type) {
     }
     for (auto& kv : waves) {   // every translation's items are a multiple of kXcds
         hfmm_batch::WaveInstance in;
-        in.p = kv.first;
-        const int per_item = (int)std::max<int64_t>(1, (wave_groups[in.p] + 2 * kWaveItems - 1) / (2 * kWaveItems));
+        in.fp32 = kv.first.first;
+        in.p = kv.first.second;
+        const int per_item = (int)std::max<int64_t>(1, (wave_groups[kv.first] + 2 * kWaveItems - 1) / (2 * kWaveItems));
         std::vector<M2LWaveArgs> args;
         std::vector<int2> work;
         std::vector<int4> sums;
         for (auto& [P, c] : kv.second) {
-            std::vector<int> part_ptr;
-            const std::vector<int4> items = wave_items(P->tree, c->host_targets, c->host_ptr, c->tb, per_item, part_ptr);
-            const int n_slots = part_ptr[c->n_blocks], j = (int)args.size();
-            M2LWaveArgs w = wave_args(*P, *c, P->dMs, P->dL, 0);
-            w.n_items = (int)items.size();
-            w.items = B.upload(items);
-            w.part_ptr = B.upload(part_ptr);
-            w.part = n_slots ? B.alloc<double4>(wave_part_size(*c, n_slots)) : nullptr;
+            std::vector<int> part_ptr = c->host_part_ptr;
+            const int j = (int)args.size();
+            M2LWaveArgs w = wave_args(*P, *c, wave_source(*P, *c), P->dL, 0);
+            if (!in.fp32) {
+                const std::vector<int4> items =
+                    wave_items(P->tree, c->host_targets, c->host_ptr, c->tb, per_item, part_ptr);
+                w.n_items = (int)items.size();
+                w.items = B.upload(items);
+                w.part_ptr = B.upload(part_ptr);
+            }
+            const int n_slots = part_ptr[c->n_blocks];
+            w.part = n_slots ? B.alloc<char>(wave_part_bytes(*c, n_slots)) : nullptr;
             for (int t = 0; t < w.n_items; ++t) work.push_back(make_int2(j, t));
+            const int chunks = in.fp32 ? wave32_sum_chunks(in.p, c->tb) : wave64_sum_chunks(in.p, c->tb);
             for (int b = 0; b < c->n_blocks; ++b)
                 if (part_ptr[b + 1] > part_ptr[b])
-                    for (int i = 0; i < wave64_sum_chunks(in.p, c->tb); ++i) sums.push_back(make_int4(j, b, i, 0));
+                    for (int i = 0; i < chunks; ++i) sums.push_back(make_int4(j, b, i, 0));
             args.push_back(w);
         }
         in.n = (int)work.size();
@@ -2450,7 +2568,7 @@ void batch_sequence(hfmm_batch& B, const void* const* q, int q_type, void* const
         launch_m2l_block_persistent(B.m2l_args[j], in.q, in.grid, in.p, in.tb, in.g, in.fp32, in.shm, s);
     }
     for (const auto& in : B.wave_inst) {
-        launch_m2l_wave64_batch(in.args, in.work, in.n, in.sums, in.n_sums, in.p, s);
+        (in.fp32 ? launch_m2l_wave32_batch : launch_m2l_wave64_batch)(in.args, in.work, in.n, in.sums, in.n_sums, in.p, s);
     }
     mark(2);
     // downward passes
