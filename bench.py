@@ -72,11 +72,11 @@ def run_form(hf, x, q_dev, out_dev, k, leaf, p, p_level, precision, steps, warmu
 
 
 def kernel_source_sha256():
-    """SHA-256 of the sources the matrix-core M2L kernel is compiled from (kernel file,
+    """SHA-256 of the sources the matrix-core M2L kernels are compiled from (kernel files,
     shared headers, build flags): a traffic figure measured on other sources is stale."""
     import hashlib
     h = hashlib.sha256()
-    for name in ("m2l_mfma.hip", "kernels.h", "common.h", "Makefile"):
+    for name in ("m2l_wave32.hip", "m2l_wave64.hip", "m2l_mfma.hip", "kernels.h", "common.h", "Makefile"):
         with open(os.path.join(ROOT, "hfmm0_amd", "csrc", name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()
@@ -109,13 +109,15 @@ def m2l_roofline(form, precision):
             else:
                 traffic_note = "profiles/m2l_traffic.json was measured on other kernel sources: not used"
     total = form["m2l_flops"] / (sum(lv_ms.values()) * 1e-3)
+    # the wave kernels take levels up to degree 15 (FP32) and 14 (FP64)
+    wave = p <= (15 if precision == "mixed" else 14)
+    kernel = ("m2l_wave32" if precision == "mixed" else "m2l_wave64") if wave else "m2l_block_kernel"
     return {"bound": "mfma",
-            "kernel": f"m2l_block_kernel, level {lvl} (p={p}, {form['v_per_level'][lvl]} V pairs), "
+            "kernel": f"{kernel}, level {lvl} (p={p}, {form['v_per_level'][lvl]} V pairs), "
                       f"{'FP32' if precision == 'mixed' else 'FP64'} MFMA",
             "achieved": achieved / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
             "frac": achieved / peak, "traffic": traffic, "traffic_source": traffic_note,
-            # compulsory bytes of the launch (multipoles read once, locals read and written);
-            # the measured traffic above them is mostly register spill (profiles/m2l_traffic.json)
+            # compulsory bytes of the launch (multipoles read once, locals read and written)
             "traffic_algorithmic": traffic_alg,
             "launch_ms": lv_ms[lvl], "flops_per_launch": flops,
             "all_levels_tflops": total / 1e12, "m2l_level_ms": {str(k): v for k, v in lv_ms.items()}}

@@ -2,8 +2,8 @@
 
 One plan per problem.  An evaluate is one captured hipGraph: the upward and downward
 passes of the problems forked over a few streams, and the matrix-core M2L and the near
-field of all problems as persistent launches whose resident workgroups take (problem,
-item) work from device queues, so that many small problems fill the GPU together.  The reference has no batch API:
+field of all problems as launches over the (problem, item) work of all of them, so that
+many small problems fill the GPU together.  The reference has no batch API:
 its tuner driver (``jaxfmm/tune.py:32-172``) loops over problems.
 """
 import ctypes
@@ -101,7 +101,7 @@ class Batch:
 
     def benchmark_phases(self, q_devs, out_devs, reps=5):
         """Mean milliseconds of the parts of one batch evaluate run eagerly: upward passes,
-        persistent M2L, downward passes, persistent near field."""
+        M2L, downward passes, near field."""
         qp, op, qt = self._dev_ptrs(q_devs, out_devs)
         ph = (ctypes.c_double * 4)()
         L.check(L.lib().hfmm_batch_benchmark_phases(self.handle, qp, qt, op, int(reps), ph))

@@ -1656,7 +1656,7 @@ void launch_wave(const hfmm_plan& P, const M2LWaveLevel& B, const void* src, dou
 }
 
 // parts of one evaluate's device sequence (a batch runs them for all problems, with the
-// block M2L and the near field as persistent launches over every problem)
+// matrix-core M2L and the near field as launches over the work of every problem)
 constexpr int kSeqUp = 1;          // charges, clears, P2M, M2M
 constexpr int kSeqM2LGeneric = 2;  // M2L levels on the generic kernel
 constexpr int kSeqM2LBlock = 4;    // M2L levels on the matrix-core block kernel
@@ -2335,8 +2335,8 @@ struct hfmm_batch {
     std::vector<void*> g_out;
     std::vector<unsigned> g_ver;            // degree versions of the plans at capture
     int g_qtype = -1;
-    // persistent launches over all problems (rebuilt with the graph): the block M2L, one
-    // launch per kernel instance, and the near field
+    // launches over all problems (rebuilt with the graph): the wave and block M2L, one per
+    // kernel instance (the block kernel's are persistent), and the near field
     struct WaveInstance {                   // the wave kernels, one launch per degree
         bool fp32 = false;
         int p = 0, n = 0, n_sums = 0;
@@ -2414,9 +2414,9 @@ WorkQueues make_queues(hfmm_batch& B, const std::vector<int2>& work, int* counte
     return q;
 }
 
-// Device descriptors and work lists of the persistent launches for the current degrees
-// and pointers: the block M2L levels of every problem grouped by kernel instance, and the
-// leaves of every problem for the near field.
+// Device descriptors and work lists of the launches over all problems for the current
+// degrees and pointers: the M2L levels of every problem grouped by kernel instance, and the
+// near-field items of every problem.
 void build_persistent(hfmm_batch& B, void* const* out, int q_type) {
     B.free_persistent();
     const int np = (int)B.plans.size();
@@ -2542,8 +2542,8 @@ void build_persistent(hfmm_batch& B, void* const* out, int q_type) {
     }
 }
 
-// ev (optional, 5 events): brackets of the upward part, the persistent M2L, the downward
-// part and the persistent near field
+// ev (optional, 5 events): brackets of the upward part, the M2L, the downward part and the
+// near field
 void batch_sequence(hfmm_batch& B, const void* const* q, int q_type, void* const* out, hipStream_t s,
                     hipEvent_t* ev = nullptr) {
     auto mark = [&](int i) {
@@ -2562,7 +2562,8 @@ void batch_sequence(hfmm_batch& B, const void* const* q, int q_type, void* const
         HIPCHK(hipStreamWaitEvent(s, B.join[b], 0));
     }
     mark(1);
-    // the block M2L of every problem and level: persistent launches
+    // the matrix-core M2L of every problem and level: persistent launches of the block
+    // kernel, the wave kernels' items
     for (size_t j = 0; j < B.m2l_inst.size(); ++j) {
         const auto& in = B.m2l_inst[j];
         launch_m2l_block_persistent(B.m2l_args[j], in.q, in.grid, in.p, in.tb, in.g, in.fp32, in.shm, s);
@@ -2581,7 +2582,7 @@ void batch_sequence(hfmm_batch& B, const void* const* q, int q_type, void* const
         HIPCHK(hipStreamWaitEvent(s, B.join2[b], 0));
     }
     mark(3);
-    // the near field of every problem: one persistent launch per leaf class
+    // the near field of every problem: one launch per leaf class
     for (int c = 0; c < 4; ++c) launch_p2p_batch(c, B.d_p2p_args, B.p2p_items[c], B.p2p_prob[c], B.p2p_n[c], s);
     mark(4);
 }

@@ -60,7 +60,7 @@ typedef struct hfmm_opts {
     int max_depth;                  /* <= 0: automatic depth (reference rule) */
     int precision;                  /* HFMM_PREC_* */
     int use_graph;                  /* 1: replay evaluate as a captured hipGraph */
-    int m2l_kernel;                 /* 0: matrix-core block kernel where it fits, chosen shape;
+    int m2l_kernel;                 /* 0: matrix-core kernels where they fit, chosen shape;
                                        1: generic kernel; 8, 16, 32, 64: block kernel with that
                                        many pairs per operator application (target boxes x
                                        directions of equal theta and |d|) where it fits */
@@ -243,8 +243,8 @@ int hfmm_mlp_destroy(hfmm_mlp* mlp);
  * One plan per problem (opts[i], k[i]).  hfmm_batch_evaluate runs all problems as one
  * hipGraph (captured once per set of pointers and replayed): the upward and downward
  * passes forked over a few streams balanced by point count, the matrix-core M2L of every
- * problem and level and the near field of every problem as persistent launches whose
- * resident workgroups take (problem, item) work from device queues, one per XCD.
+ * problem and level and the near field of every problem as launches over the (problem, item)
+ * work of all problems.
  * q[i] / out[i] as in hfmm_evaluate.
  * --------------------------------------------------------------------------------- */
 typedef struct hfmm_batch hfmm_batch;
@@ -259,7 +259,7 @@ int hfmm_batch_benchmark(hfmm_batch* batch, const void* const* q_dev, int q_type
                          int warmup, int reps, double* median_ms);
 /* mean milliseconds of the four parts of a device-resident batch evaluate, run eagerly
  * with hipEvents between them: phase_ms[0] upward passes (and generic-kernel M2L levels),
- * [1] the persistent matrix-core M2L, [2] downward passes, [3] the persistent near field */
+ * [1] the matrix-core M2L, [2] downward passes, [3] the near field */
 int hfmm_batch_benchmark_phases(hfmm_batch* batch, const void* const* q_dev, int q_type, void* const* out_dev,
                                 int reps, double* phase_ms);
 int hfmm_batch_destroy(hfmm_batch* batch);
