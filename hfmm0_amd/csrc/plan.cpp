@@ -71,6 +71,12 @@ struct M2LBlockLevel {
     int* zero = nullptr;
 };
 
+// L2P takes leaves of levels of different degrees in launches of their own, each with the LDS (and so
+// the resident workgroups) of its degree, where every launch has this many: about the workgroups that
+// fit the chip at once.  200k clustered points, degrees 13, 12 and 11 on the levels with leaves: L2P
+// 0.204 ms in one launch sized for degree 13, 0.162 in three (evaluate 3.045 -> 2.995 ms).
+constexpr int kL2PRunLeaves = 3072;
+
 // items an M2L launch of the FP64 wave kernel is split into (m2l_wave64.hip)
 constexpr int kWaveItems = 3072;
 
@@ -149,6 +155,8 @@ struct hfmm_plan {
     double* d_R = nullptr;
     int* d_far_leaves = nullptr;
     LeafDesc* d_leafdesc = nullptr;   // per far leaf (d_far_leaves order): P2M / L2P descriptors
+    struct LeafRun { int first, n, p; };
+    std::vector<LeafRun> l2p_runs;    // far leaves of consecutive levels and their largest table degree
     int *d_leaf_box = nullptr, *d_batch_ptr = nullptr, *d_rng_delta = nullptr, *d_leaf_src_total = nullptr;
     NearBatch* d_batches = nullptr;
     NearItems near_items[2], field_items[2];   // FP32-phase (or FP64) leaves, FP64-phase leaves
@@ -1518,6 +1526,19 @@ void build_plan(hfmm_plan& P, const double* xyz, int64_t n, double k, const hfmm
     for (int b = 0; b < t.n_boxes(); ++b)
         if (t.is_leaf[b]) P.p_leafmax = std::max(P.p_leafmax, P.p_level[t.level[b]]);
     P.p2m_chunk = p2m_chunk(P.p_leafmax);
+    for (int l = 2, first = 0; l <= P.depth; ++l) {   // the far leaves are ordered by level
+        int n = 0;
+        for (int b = t.level_start[l]; b < t.level_start[l + 1]; ++b) n += t.is_leaf[b] ? 1 : 0;
+        if (!n) continue;
+        if (!P.l2p_runs.empty() && (P.l2p_runs.back().p == P.p_level[l] || P.l2p_runs.back().n < kL2PRunLeaves ||
+                                    P.n_far_leaves - first < kL2PRunLeaves)) {
+            P.l2p_runs.back().n += n;
+            P.l2p_runs.back().p = std::max(P.l2p_runs.back().p, P.p_level[l]);
+        } else {
+            P.l2p_runs.push_back({first, n, P.p_level[l]});
+        }
+        first += n;
+    }
     P.dM = P.alloc<double2>(P.n_coef);
     bool any_fp32 = false, any_l2l32 = false;
     for (int L = 0; L < kMaxLevels; ++L) {
@@ -1828,7 +1849,8 @@ void run_sequence(hfmm_plan& P, const void* q, int q_type, double2* out, hipStre
             launch_l2p_field(P.d_far_leaves, P.n_far_leaves, bx, lv, P.dX, P.dY, P.dZ, P.dL, P.k, P.p_leafmax,
                              P.d_far, P.d_far_e, s);
         } else {
-            launch_l2p(P.d_leafdesc, P.n_far_leaves, lv, P.dX, P.dY, P.dZ, P.dL, P.k, P.p_leafmax, P.d_far, s);
+            for (const auto& r : P.l2p_runs)
+                launch_l2p(P.d_leafdesc + r.first, r.n, lv, P.dX, P.dY, P.dZ, P.dL, P.k, r.p, P.d_far, s);
         }
         mark(6);
     }
