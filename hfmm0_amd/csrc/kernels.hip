@@ -545,10 +545,15 @@ __global__ __launch_bounds__(64) void l2p_kernel(const LeafDesc* __restrict__ le
             const double2 u = make_double2(dx * invR, dy * invR);
             double2 phi = make_double2(0.0, 0.0);
             double2 um = make_double2(1.0, 0.0);   // ((x + i y)/R)^m
-            for (int m = 0; m <= p; ++m) {
-                if (m > 0) um = cmul(um, u);
-                const int mr = m % S;
-                if (((m / S) & 1 ? S - 1 - mr : mr) != part) continue;
+            int mu = 0;
+            // Every lane takes its own order in every step: a loop over all m in which a lane skips the
+            // other parts' orders takes a wave through every order with 1 / S of its lanes.  200k
+            // clustered points in leaves of up to 32: 0.109 -> 0.079 ms at p = 11, 0.184 -> 0.121 at
+            // p = 12, 0.206 -> 0.141 at p = 13; 1M points (24 to 40 a leaf) 0.162 -> 0.156.
+            for (int j = 0; j * S <= p; ++j) {
+                const int m = j * S + (j & 1 ? S - 1 - part : part);
+                if (m > p) continue;
+                for (; mu < m; ++mu) um = cmul(um, u);
                 const double2* abm = lg.ab + leg_col(PM1, m) - m;     // (a_nm, b_nm) at abm[n]
                 const double2* ABm = s_AB + 2 * (leg_col(P1, m) - m);  // (A_nm, B_nm) at ABm[2n], ABm[2n + 1]
                 double h = rad[64 * m];
