@@ -72,6 +72,15 @@ constexpr int reg_degree(int i) {
     return n;
 }
 
+// Rows of the LDS columns pass between the lane groups (the v half is read one row up from where it
+// was gathered, the coaxial operators read along the degrees): LDS accesses before stay before those
+// after.  A wave's LDS instructions are executed in order, so this holds the compiler only; without it
+// addresses a constant apart look independent, being those of one lane.
+__device__ __forceinline__ void lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // U and V (v: U_re, U_im, V_re, V_im) of degree n and order m, back in the x basis: x_0 = U_0,
 // x_m = (U + V) / 2, x_{-m} = (-1)^m (U - V) / 2
 __device__ __forceinline__ void store_expansion(double2* dst, int n, int m, int pt, int overwrite, double4 v) {
@@ -112,6 +121,7 @@ __device__ __forceinline__ void wave64_body(const M2LWaveArgs& a, const int4 ite
     unrolled<0, NR>([&](auto ic) { U[IDX(ic)][0] = U[IDX(ic)][1] = V[IDX(ic)][0] = V[IDX(ic)][1] = 0.0; });
     double2* dump = X + 16 * (tri(P + 1) + 3) + lane;   // results of rows outside a block
     for (int i = lane; i < 16 * (tri(P + 1) + 3); i += 64) X[i] = make_double2(0.0, 0.0);
+    lds_order();
     // LDS addresses: rows of one degree are consecutive (lane group lk: row 4 j + lk); rows of one
     // order m lie at tri(n) + m, n = 4 j + lk (degrees above P: the row of degree P, whose
     // products meet zeros of the operator)
@@ -145,6 +155,7 @@ __device__ __forceinline__ void wave64_body(const M2LWaveArgs& a, const int4 ite
             // what a degree's last register writes past its rows the next degree overwrites.
             // kAhead registers' entries are in flight
             constexpr int kAhead = NR < kGatherAhead ? NR : kGatherAhead;
+            lds_order();
             double4 g[kAhead];
             auto gather_load = [&](auto ic) {
                 constexpr int i = IDX(ic), n = reg_degree(i), r = i - regs_before(n);
@@ -162,6 +173,7 @@ __device__ __forceinline__ void wave64_body(const M2LWaveArgs& a, const int4 ite
                 const double2 q = h ? make_double2(s.x, s.y) : make_double2(s.z, s.w);
                 xr[16 * (tri(n) + 4 * r)] = make_double2(fma(ph[r].x, o.x, -ph[r].y * q.y),
                                                          fma(ph[r].x, o.y, ph[r].y * q.x));
+                if constexpr (r == n / 4 && (n % 4 != 3 || n == P)) lds_order();   // past its rows; all rows done
                 __builtin_amdgcn_sched_barrier(0);
             });
             // The stages' blocks are one sequence q: forward rotations (degree h + q), coaxial
@@ -267,7 +279,10 @@ __device__ __forceinline__ void wave64_body(const M2LWaveArgs& a, const int4 ite
                 __builtin_amdgcn_sched_barrier(0);
                 // the previous block's results are taken while this one's products run
                 if constexpr (q % NB > 0) finish(std::integral_constant<int, q - 1>{});
-                if constexpr (q % NB == NB - 1) finish(qc);
+                if constexpr (q % NB == NB - 1) {
+                    finish(qc);
+                    lds_order();
+                }
                 // the loads stay the stated number of blocks ahead: moved further up they would
                 // not fit the registers
                 __builtin_amdgcn_sched_barrier(0);
