@@ -160,7 +160,10 @@ __device__ __forceinline__ void wave64_body(const M2LWaveArgs& a, const int4 ite
             auto gather_load = [&](auto ic) {
                 constexpr int i = IDX(ic), n = reg_degree(i), r = i - regs_before(n);
                 const double2* m0 = (const double2*)a.M + 2 * (tri(n) + 4 * r);
-                const uint32_t o = n <= ps ? so : sz;
+                // lanes past degree P's last order read zeros too: the MFMAs of degree P read the rows
+                // that they write, and 0 x NaN of an entry that this call has not written is NaN
+                uint32_t o = n <= ps ? so : sz;
+                if constexpr (n == P && 4 * r + 3 > P) o = 4 * r + lk <= P ? o : sz;
                 const double2 s0 = load16(m0, o), d0 = load16(m0 + 1, o);
                 g[i % kAhead] = make_double4(s0.x, s0.y, d0.x, d0.y);
             };
