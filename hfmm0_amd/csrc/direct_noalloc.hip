@@ -64,6 +64,7 @@ __global__ __launch_bounds__(256) void direct_aos_kernel(const double* xyz, cons
     const nearfield::SinCosPi64 sp = nearfield::SinCosPi64::pinned();
     for (int64_t base = s0; base < s1; base += 256) {
         const int64_t v = base + threadIdx.x;
+        bool bad = false;   // a charge that is not finite: pairs at r = 0 are left out
         if (v < s1) {
             sx[threadIdx.x] = xyz[3 * v];
             sy[threadIdx.x] = xyz[3 * v + 1];
@@ -71,16 +72,28 @@ __global__ __launch_bounds__(256) void direct_aos_kernel(const double* xyz, cons
             const double2 qq = q[v];
             sqr[threadIdx.x] = qq.x;
             sqi[threadIdx.x] = conj ? -qq.y : qq.y;
+            bad = !nearfield::finite_charge(qq.x, qq.y);
         }
-        __syncthreads();
+        const bool odd = __syncthreads_or(bad);
         const int nb = (int)min((int64_t)256, s1 - base);
-#pragma unroll 2
-        for (int j = 0; j < nb; ++j) {
-            const double dx = x - sx[j], dy = y - sy[j], dz = z - sz[j];
+        auto pair = [&](int j, double r2) {
             double wr, wi;
-            nearfield::pair_weight64(dx * dx + dy * dy + dz * dz, 0.0, kp, sp, wr, wi);
+            nearfield::pair_weight64(r2, 0.0, kp, sp, wr, wi);
             ar = fma(wr, sqr[j], fma(-wi, sqi[j], ar));
             ai = fma(wr, sqi[j], fma(wi, sqr[j], ai));
+        };
+        auto dist2 = [&](int j) {
+            const double dx = x - sx[j], dy = y - sy[j], dz = z - sz[j];
+            return dx * dx + dy * dy + dz * dz;
+        };
+        if (odd) {
+            for (int j = 0; j < nb; ++j) {
+                const double r2 = dist2(j);
+                if (r2 > 0.0) pair(j, r2);
+            }
+        } else {
+#pragma unroll 2
+            for (int j = 0; j < nb; ++j) pair(j, dist2(j));
         }
         __syncthreads();
     }

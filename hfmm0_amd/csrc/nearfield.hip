@@ -67,13 +67,22 @@ __device__ inline void field_weights64(double r2, double fl2, double k, HalfTurn
 //   pos(x, y, z)             of a point relative to the leaf centre,
 //   stage(st, lane, ...)     a source (relative position, charge) into the stage,
 //   load(st, j)              a staged source (Src),
-//   pair(t, src, acc)        one pair into the sums.
+//   pair(t, src, acc)        one pair into the sums,
+//   apart(t, src)            (kSkips) r^2 above the floor: pairs at it enter with the weight zero, which
+//                            is nothing where the charge is finite; else they are left out.
+
+template <typename Pos, typename Src>
+__device__ __forceinline__ bool apart_at(const Pos& t, const Src& s, double fl2) {
+    const double dx = t.x - s.x, dy = t.y - s.y, dz = t.z - s.z;
+    return dx * dx + dy * dy + dz * dz > fl2;
+}
 
 // FP64 throughout.  Pairs at or below the leaf's coincidence floor get the weight zero.  About 50
 // FP64 instructions a pair with a v_rsq_f64: 2.65 ms for 9.3e8 pairs, against 5.41 with the device
 // library's sincos, square root and division.
 struct FormFp64 {
     static constexpr int kStage = 5 * 64, kSums = 2;
+    static constexpr bool kSkips = true;
     using Acc = double;
     struct Pos { double x, y, z; };
     struct Src { double x, y, z, qr, qi; };
@@ -91,6 +100,7 @@ struct FormFp64 {
         st[256 + lane] = q.y;
     }
     __device__ Src load(const double* st, int j) const { return {st[j], st[64 + j], st[128 + j], st[192 + j], st[256 + j]}; }
+    __device__ bool apart(const Pos& t, const Src& s) const { return apart_at(t, s, fl2); }
     __device__ void pair(const Pos& t, const Src& s, double* acc) const {
         const double dx = t.x - s.x, dy = t.y - s.y, dz = t.z - s.z;
         const double r2 = dx * dx + dy * dy + dz * dz;
@@ -117,6 +127,7 @@ __device__ __forceinline__ void add_pair32(float wr, float wi, float2 q, float* 
 template <bool PH, bool LOWK>
 struct FormMixed {
     static constexpr int kStage = 4 * 64, kSums = 2;
+    static constexpr bool kSkips = false;
     using Acc = float;
     struct Pos { double x, y, z; };
     struct Src { double x, y, z; float2 q; };
@@ -154,6 +165,7 @@ struct FormMixed {
 // in FP32: the FP32-phase leaves flagged in a.coord32
 struct FormMixed32 {
     static constexpr int kStage = 4 * 64, kSums = 2;
+    static constexpr bool kSkips = false;
     using Acc = float;
     struct Pos { float x, y, z; };
     struct Src { float4 p; float2 q; };
@@ -184,6 +196,7 @@ struct FormMixed32 {
 template <typename T, bool PH>
 struct FormField {
     static constexpr int kStage = 5 * 64, kSums = 8;   // phi, Ex, Ey, Ez (re, im)
+    static constexpr bool kSkips = std::is_same<T, double>::value;
     using Acc = T;
     struct Pos { double x, y, z; };
     struct Src { double x, y, z; T qr, qi; };
@@ -204,6 +217,7 @@ struct FormField {
     __device__ Src load(const double* st, int j) const {
         return {st[j], st[64 + j], st[128 + j], ((const T*)(st + 192))[j], ((const T*)(st + 256))[j]};
     }
+    __device__ bool apart(const Pos& t, const Src& s) const { return apart_at(t, s, fl2); }
     __device__ void pair(const Pos& t, const Src& s, T* acc) const {
         const double dx = t.x - s.x, dy = t.y - s.y, dz = t.z - s.z;
         const double r2 = dx * dx + dy * dy + dz * dz;
@@ -286,6 +300,7 @@ __device__ __forceinline__ void near_body(const P2PArgs& a, const NearItem item,
     sh = shift(b0 + kNearWaves, rec);
     rec = record(b0 + 2 * kNearWaves);
     for (int b = b0; b < n_batches; b += kNearWaves) {
+        const bool odd = F::kSkips && __ballot(!nearfield::finite_charge(q.x, q.y)) != 0;
         f.stage(st, lane, x - cx, y - cy, z - cz, q);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -302,10 +317,20 @@ __device__ __forceinline__ void near_body(const P2PArgs& a, const NearItem item,
 #pragma unroll
             for (int c = 0; c < NS; ++c) acc[r][c] = 0;
         const int n = min(64, S - 64 * b);
-        for (int j = g; j < n; j += G) {
-            const typename F::Src s = f.load(st, j);
+        if (odd) {
+            if constexpr (F::kSkips)
+                for (int j = g; j < n; j += G) {
+                    const typename F::Src s = f.load(st, j);
 #pragma unroll
-            for (int r = 0; r < R; ++r) f.pair(t[r], s, acc[r]);
+                    for (int r = 0; r < R; ++r)
+                        if (f.apart(t[r], s)) f.pair(t[r], s, acc[r]);
+                }
+        } else {
+            for (int j = g; j < n; j += G) {
+                const typename F::Src s = f.load(st, j);
+#pragma unroll
+                for (int r = 0; r < R; ++r) f.pair(t[r], s, acc[r]);
+            }
         }
 #pragma unroll
         for (int r = 0; r < R; ++r)

@@ -203,7 +203,9 @@ HFMM_HD inline void halfturn64(double r2, HalfTurnK k, const SinCosPi64& sp, dou
     rs = __builtin_bit_cast(double, dbits(rinv) | (dbits(m) << 63));
 }
 
-// Weight of one pair in FP64, e^{ikr}/r, exactly zero at or below the floor fl2.
+// Weight of one pair in FP64, e^{ikr}/r, exactly zero at or below the floor fl2.  A pair at the
+// floor contributes nothing whatever its charge: with a charge that is not finite the caller leaves
+// the pair out, 0 x NaN being NaN.
 HFMM_HD inline void pair_weight64(double r2, double fl2, HalfTurnK k, const SinCosPi64& sp, double& wr,
                                   double& wi) {
     double c, s, rs, rinv, r;
@@ -212,6 +214,9 @@ HFMM_HD inline void pair_weight64(double r2, double fl2, HalfTurnK k, const SinC
     wr = c * rs;
     wi = s * rs;
 }
+
+// false for every charge that is not finite (and for finite ones whose parts' sum overflows)
+HFMM_HD inline bool finite_charge(double re, double im) { return fabs(re) + fabs(im) < __builtin_inf(); }
 
 // ---------------------------------------------------------------------------------
 // Radian form (the field kernel): y = k r reduced by pi to [-pi/2, pi/2].
