@@ -56,7 +56,7 @@ __device__ inline void field_weights64(double r2, double fl2, double k, HalfTurn
     rs = r2 > fl2 ? rs : 0.0;
     wr = c * rs;
     wi = s * rs;
-    const double kr = k * r, rinv2 = rinv * rinv;
+    const double kr = k * r, rinv2 = rs * rs;
     fr = fma(kr, wi, wr) * rinv2;
     fi = fma(-kr, wr, wi) * rinv2;
 }

@@ -138,9 +138,10 @@ HFMM_HD inline double rsq64_estimate(double x) {
 #endif
 }
 
-// 1/r and r from r2 = r^2 (a normal number).  With y the estimate and e = 1 - r2 y^2,
+// 1/r and r from r2 = r^2 > 0.  With y the estimate and e = 1 - r2 y^2,
 // r^-1 = y (1 - e)^-1/2 = y (1 + e/2 + 3 e^2/8) up to 5 e^3 / 16 (e <= 2e-6: below 1e-17); r is
-// r2 / r with one correction from its residual.
+// r2 / r with one correction from its residual.  A subnormal r2 holds fewer bits, which the residual
+// of r then rounds to as well; 1/r is that of the r2 given.
 HFMM_HD inline void rsqrt64(double r2, double& rinv, double& r) {
     const double y = rsq64_estimate(r2);
     const double e = fma(-(r2 * y), y, 1.0);
@@ -190,11 +191,11 @@ HFMM_HD inline void sincospi_half64(double y, const SinCosPi64& p, double& s, do
 // e^{ikr} = (-1)^n (c + i s) from r2 = r^2 > 0 in FP64: c = cos(pi y), s = sin(pi y), and rs
 // the signed 1/r, so that e^{ikr}/r is (c rs, s rs); also 1/r and r.  The reduction
 // y = r k/pi - n takes k/pi in two terms, so only its own rounding (2^-53 of n) and r's enter
-// the phase.  r^2 below the smallest normal number counts as that number.  Beyond
+// the phase.  r^2 = 0 counts as the smallest subnormal number (1/r^2 overflows there).  Beyond
 // k r / pi = 2^50, where an FP64 k r carries an error of a radian, the phase stays that of
 // 2^50 (the parity trick needs integers below 2^51).
 HFMM_HD inline void halfturn64(double r2, HalfTurnK k, const SinCosPi64& sp, double& c, double& s, double& rs, double& rinv, double& r) {
-    rsqrt64(fmax(r2, 0x1p-1022), rinv, r);
+    rsqrt64(fmax(r2, 0x1p-1074), rinv, r);
     const double p = fmin(r * k.hi, 0x1p50);
     const double m = p + 6755399441055744.0;  // 1.5 * 2^52
     const double n = m - 6755399441055744.0;
