@@ -1378,11 +1378,14 @@ size_t wave_part_bytes(const M2LWaveLevel& B, int n_slots) {
            (B.fp32 ? 2 * (p + 1) * (p + 1) * sizeof(float) : 4 * wave64_regs(p) * sizeof(double4));
 }
 
-// The partial sums of the wave kernel's split blocks: one buffer for all levels, which run one
-// after another
+// The partial sums of the wave kernels' split blocks: one buffer for all levels, which run one after
+// another (FP64, 16 targets a block: up to 132 MB at p = 10, 226 MB at p = 14).  Allocated with the plan;
+// a plan of a batch, which has a buffer for all its problems, gets its own when it is first evaluated
+// alone (64 problems of 2k to 200k points in FP64: 9.3 GB with a buffer each, 2.7 GB without).
 void alloc_wave_parts(hfmm_plan& P) {
     size_t most = 0;
-    for (const M2LWaveLevel& B : P.m2lc) most = std::max(most, wave_part_bytes(B, B.n_slots));
+    for (const M2LWaveLevel& B : P.m2lc)
+        if (!B.part) most = std::max(most, wave_part_bytes(B, B.n_slots));
     if (!most) return;
     void* all = P.alloc<char>(most);
     for (M2LWaveLevel& B : P.m2lc)
@@ -1554,7 +1557,7 @@ void build_plan(hfmm_plan& P, const double* xyz, int64_t n, double k, const hfmm
         any_wave32 = any_wave32 || (P.m2lc[L].use && P.m2lc[L].fp32);
         any_l2l_col = any_l2l_col || P.l2lc[L].use;
     }
-    alloc_wave_parts(P);
+    if (!P.in_batch) alloc_wave_parts(P);
     const size_t n_sd = P.n_sd + wave_sd_pad(P.pmax);
     for (double4** buf : {any_col ? &P.dMs : nullptr, any_l2l_col ? &P.dLs : nullptr})
         if (buf) {
@@ -1878,6 +1881,7 @@ void sequence_typed(hfmm_plan& P, const void* q, int q_type, void* out, int out_
 }
 
 void evaluate_device(hfmm_plan& P, const void* q, int q_type, void* out, hipStream_t s, int out_type = HFMM_C128) {
+    alloc_wave_parts(P);
     if (!P.use_graph) {
         sequence_typed(P, q, q_type, out, out_type, s);
         return;
@@ -2078,6 +2082,7 @@ int hfmm_evaluate_field(hfmm_plan* P, const void* q, int q_type, void* phi, void
         if (P->p_leafmax + 1 > kMaxP) fail(HFMM_ERR_ARG, "the field needs leaf degrees of at most 39");
         hipStream_t s = stream ? (hipStream_t)stream : P->stream;
         if (!P->d_far_e) P->d_far_e = P->alloc<double2>(3 * P->n);
+        alloc_wave_parts(*P);
         if (ptr_kind == HFMM_HOST) {
             if (!P->d_field_out) P->d_field_out = P->alloc<double2>(3 * P->n);
             HIPCHK(hipMemcpyAsync(P->d_qin, q, (size_t)P->n * charge_bytes(q_type), hipMemcpyHostToDevice, s));
@@ -2144,6 +2149,7 @@ int hfmm_benchmark_m2l_levels(hfmm_plan* P, const void* q_dev, int q_type, void*
     return guarded([&] {
         if (!P || !q_dev || !out_dev || !level_ms || reps < 1) fail(HFMM_ERR_ARG, "bad argument");
         hipStream_t s = P->stream;
+        alloc_wave_parts(*P);
         std::vector<hipEvent_t> ev(2 * kMaxLevels);
         for (auto& e : ev) HIPCHK(hipEventCreate(&e));
         for (int L = 0; L < HFMM_MAX_LEVELS; ++L) level_ms[L] = 0.0;
@@ -2422,6 +2428,12 @@ namespace {
 
 constexpr int kBatchStreams = 4;
 
+// Partial sums that a batch holds: a launch leaves up to 0.2 GB of a level (FP32, p = 14, 32 targets a
+// block), so 256 mixed problems of 2k to 200k points left 4.8 GB and thousands would not fit.  Every
+// further launch ends with a tail of its own: at 1 GiB, 64 such problems (1.2 GB) took two launches and
+// 18.5 ms instead of 18.0.
+constexpr size_t kBatchPartBytes = (size_t)4 << 30;
+
 // kernel instance of the block M2L (the table-degree range selects KT and MAXU)
 int m2l_degree_range(int p) { return p <= 7 ? 0 : p <= 11 ? 1 : p <= 15 ? 2 : p <= 17 ? 3 : p <= 19 ? 4 : 5; }
 
@@ -2455,7 +2467,7 @@ void build_persistent(hfmm_batch& B, void* const* out, int q_type) {
             pmax[key] = std::max(pmax[key], pk);
         }
     }
-    // wave kernel: one launch per degree over every problem and level, split to twice the items
+    // wave kernel: one launch per degree over problems and levels, split to twice the items
     // of a single level.  Split by level as for a plan alone, 16 problems of 2k to 20k points at
     // p = 10 made 36128 items, of a group or two each: 2.67 ms, and 0.29 for the sums, against
     // 1.37 and 0.05 for the 6016 items of this rule.
@@ -2491,40 +2503,64 @@ void build_persistent(hfmm_batch& B, void* const* out, int q_type) {
         B.m2l_inst.push_back(in);
         B.m2l_args.push_back(d_args);
     }
-    for (auto& kv : waves) {   // every translation's items are a multiple of kXcds
+    // The launches run one after another and share one buffer of partial sums; a launch takes levels
+    // up to kBatchPartBytes of them (or one level that needs more).
+    struct Pending {
         hfmm_batch::WaveInstance in;
-        in.fp32 = kv.first.first;
-        in.p = kv.first.second;
-        const int per_item = (int)std::max<int64_t>(1, (wave_groups[kv.first] + 2 * kWaveItems - 1) / (2 * kWaveItems));
         std::vector<M2LWaveArgs> args;
+        std::vector<size_t> part;               // offset of each descriptor's partial sums
         std::vector<int2> work;
         std::vector<int4> sums;
+        size_t bytes = 0;
+    };
+    std::vector<Pending> launches;
+    for (auto& kv : waves) {   // every translation's items are a multiple of kXcds
+        const bool fp32 = kv.first.first;
+        const int p = kv.first.second;
+        const int per_item = (int)std::max<int64_t>(1, (wave_groups[kv.first] + 2 * kWaveItems - 1) / (2 * kWaveItems));
+        bool first = true;
         for (auto& [P, c] : kv.second) {
             std::vector<int> part_ptr = c->host_part_ptr;
-            const int j = (int)args.size();
             M2LWaveArgs w = wave_args(*P, *c, wave_source(*P, *c), P->dL, 0);
-            if (!in.fp32) {
+            if (!fp32) {
                 const std::vector<int4> items =
                     wave_items(P->tree, c->host_targets, c->host_ptr, c->tb, per_item, part_ptr);
                 w.n_items = (int)items.size();
                 w.items = B.upload(items);
                 w.part_ptr = B.upload(part_ptr);
             }
-            const int n_slots = part_ptr[c->n_blocks];
-            w.part = n_slots ? B.alloc<char>(wave_part_bytes(*c, n_slots)) : nullptr;
-            for (int t = 0; t < w.n_items; ++t) work.push_back(make_int2(j, t));
-            const int chunks = in.fp32 ? wave32_sum_chunks(in.p, c->tb) : wave64_sum_chunks(in.p, c->tb);
+            const size_t bytes = wave_part_bytes(*c, part_ptr[c->n_blocks]);
+            if (first || launches.back().bytes + bytes > kBatchPartBytes) {
+                launches.emplace_back();
+                launches.back().in.fp32 = fp32;
+                launches.back().in.p = p;
+                first = false;
+            }
+            Pending& l = launches.back();
+            const int j = (int)l.args.size();
+            l.part.push_back(l.bytes);
+            l.bytes += bytes;
+            w.part = nullptr;
+            for (int t = 0; t < w.n_items; ++t) l.work.push_back(make_int2(j, t));
+            const int chunks = fp32 ? wave32_sum_chunks(p, c->tb) : wave64_sum_chunks(p, c->tb);
             for (int b = 0; b < c->n_blocks; ++b)
                 if (part_ptr[b + 1] > part_ptr[b])
-                    for (int i = 0; i < chunks; ++i) sums.push_back(make_int4(j, b, i, 0));
-            args.push_back(w);
+                    for (int i = 0; i < chunks; ++i) l.sums.push_back(make_int4(j, b, i, 0));
+            l.args.push_back(w);
         }
-        in.n = (int)work.size();
-        in.work = B.upload(work);
-        in.n_sums = (int)sums.size();
-        in.sums = B.upload(sums);
-        in.args = B.upload(args);
-        B.wave_inst.push_back(in);
+    }
+    size_t most = 0;
+    for (const Pending& l : launches) most = std::max(most, l.bytes);
+    char* parts = most ? B.alloc<char>(most) : nullptr;
+    for (Pending& l : launches) {
+        for (size_t j = 0; j < l.args.size(); ++j)
+            if ((j + 1 < l.part.size() ? l.part[j + 1] : l.bytes) > l.part[j]) l.args[j].part = parts + l.part[j];
+        l.in.n = (int)l.work.size();
+        l.in.work = B.upload(l.work);
+        l.in.n_sums = (int)l.sums.size();
+        l.in.sums = B.upload(l.sums);
+        l.in.args = B.upload(l.args);
+        B.wave_inst.push_back(l.in);
     }
     std::vector<P2PArgs> pa(np);
     // leaves [l0, l1) of a problem in near-field class cls
