@@ -537,30 +537,42 @@ void build_m2l_blocks(hfmm_plan& P, int L, const std::vector<int>& targets, cons
     prepare_m2l_block(p, tb, grp, fp32);
 }
 
+// targets of a block of the tree translations, each of one direction per group
+constexpr int kTreeBlock = 8;
+
+// an M2M level with fewer blocks is split: their groups go over items that add atomically
+bool tree_split(int kind, size_t n_parents) { return kind == 1 && (n_parents + kTreeBlock - 1) / kTreeBlock < 512; }
+
+// FP32 arithmetic (FP64 results) of the M2M into level L (kind 1) or the L2L out of it (kind 2): where
+// the M2L of every level from 2 to L+1 runs in FP32, since the translated expansions then only
+// feed FP32 translations, whose own rounding is of the same size; a chain through an FP64 M2L
+// level keeps FP64.  Split M2M levels keep FP64 as well: there the FP32 form was slower (N=1M,
+// k=40: 55.7 against 40.4 us for level 4 -> 3, where the level 5 -> 4 M2M took 81.9 against 113.5 us).
+bool tree_fp32(const hfmm_plan& P, int L, int kind, size_t n_parents) {
+    if (P.m2l_kernel == 1 || !P.d_rf1_32 || tree_split(kind, n_parents)) return false;
+    for (int l = 2; l <= L + 1; ++l)
+        if (!P.m2l_fp32[l] || P.p_level[l] > kM2LBlockMaxP) return false;
+    return m2l_block_lds_bytes(std::max(P.p_level[L], P.p_level[L + 1]), kTreeBlock, 1, 8) <= P.max_lds;
+}
+
 // M2M (kind 1: the parents of level L from their children) and L2L (kind 2: the children
-// at level L+1 from their parents) on the matrix-core block kernel, in FP32 or FP64 (see
-// below; the results are FP64 either way).  Blocks of 8 targets,
+// at level L+1 from their parents) on the matrix-core block kernel, in FP32 (tree_fp32) or FP64:
+// the levels that the wave kernel does not take.  Blocks of 8 targets,
 // one direction per group: an M2M block runs one group per child octant present among
 // its parents, every target receiving all of its children within the one work item, so
 // the result is stored (no clear of the parent multipoles is needed); an L2L block holds
 // 8 children of one octant and a single group (their parents' locals), added to what
 // M2L left there.  tab: the coaxial table (pt+1-m) x (ps+1-m) per m of this level pair.
-void build_tree_blocks(hfmm_plan& P, int L, int kind, const std::vector<double>& tab) {
+void build_tree_blocks(hfmm_plan& P, int L, int kind, const std::vector<double>& tab, bool fp32) {
     if (P.m2l_kernel == 1 || !P.d_rf1) return;
     const Tree& t = P.tree;
     const int ps = kind == 1 ? P.p_level[L + 1] : P.p_level[L];
     const int pt = kind == 1 ? P.p_level[L] : P.p_level[L + 1];
     const int pm = std::max(ps, pt);
     if (pm > kM2LBlockMaxP) return;
-    // FP32 arithmetic (FP64 results) where the M2L of every level from 2 to L+1 runs in FP32:
-    // the translated expansions then only feed FP32 translations, whose own rounding is of
-    // the same size; a chain through an FP64 M2L level keeps FP64.  Split M2M levels (below)
-    // keep FP64 as well: there the FP32 form was slower (N=1M, k=40: 55.7 against 40.4 us
-    // for level 4 -> 3, where the level 5 -> 4 M2M took 81.9 against 113.5 us).
-    bool fp32 = P.d_rf1_32 != nullptr;
-    for (int l = 2; l <= L + 1; ++l) fp32 = fp32 && P.m2l_fp32[l] && P.p_level[l] <= kM2LBlockMaxP;
-    const int tb = 8, grp = 1;
+    const int tb = kTreeBlock, grp = 1;
     if (m2l_block_lds_bytes(pm, tb, grp, 8) > P.max_lds) return;
+    size_t n_parents = 0;
     std::vector<int> blk_targets, blk_ptr{0}, grp_off;
     std::vector<unsigned short> grp_dir;
     if (kind == 1) {
@@ -575,6 +587,7 @@ void build_tree_blocks(hfmm_plan& P, int L, int kind, const std::vector<double>&
             }
             child.back()[octant(t.code[c])] = c;
         }
+        n_parents = parents.size();
         for (size_t b0 = 0; b0 < parents.size(); b0 += tb) {
             for (int j = 0; j < tb; ++j) blk_targets.push_back(b0 + j < parents.size() ? parents[b0 + j] : -1);
             for (int o = 0; o < 8; ++o) {
@@ -608,9 +621,7 @@ void build_tree_blocks(hfmm_plan& P, int L, int kind, const std::vector<double>&
     if (blk_ptr.size() < 2) return;
     // coarse M2M levels have few blocks: their groups (child octants) are split over items
     // that add atomically, after the parents are cleared; L2L blocks hold one group
-    const int nblk = (int)blk_ptr.size() - 1;
-    const bool split = kind == 1 && nblk < 512;
-    if (split) fp32 = false;
+    const bool split = tree_split(kind, n_parents);
     const std::vector<int4> items = make_items(t, blk_targets, blk_ptr, tb, split);
     std::vector<int> units1, units2, units3;
     make_units(ps, pt, units1, units2, units3, fp32 && m2l_tiles(pm + 1) == 1);
@@ -1157,8 +1168,9 @@ void build_tables(hfmm_plan& P) {
         std::vector<double> cx((size_t)A.coax_stride * 2);
         coax_table(1, G, P.k, P.R[L + 1], P.R[L + 1], P.R[L], A.ps, A.pt, cx.data());
         A.coax = (double2*)P.upload(cx);
-        build_tree_blocks(P, L, 1, cx);
-        if (!P.m2mb[L].fp32) build_waves(P, P.m2mc[L], 1, L + 1, L, targets, ptr, src, dir, cx, 1, dinfo);
+        const bool up32 = tree_fp32(P, L, 1, targets.size()), down32 = tree_fp32(P, L, 2, targets.size());
+        if (!up32) build_waves(P, P.m2mc[L], 1, L + 1, L, targets, ptr, src, dir, cx, 1, dinfo);
+        if (!P.m2mc[L].use) build_tree_blocks(P, L, 1, cx, up32);
         XlateLaunch& B = P.l2l[L];
         B.n_targets = (int)ctargets.size();
         B.targets = P.upload(ctargets);
@@ -1173,8 +1185,8 @@ void build_tables(hfmm_plan& P) {
         std::vector<double> cy((size_t)B.coax_stride * 2);
         coax_table(2, G, P.k, P.R[L + 1], P.R[L], P.R[L + 1], B.ps, B.pt, cy.data());
         B.coax = (double2*)P.upload(cy);
-        build_tree_blocks(P, L, 2, cy);
-        if (!P.l2lb[L].fp32) build_waves(P, P.l2lc[L], 2, L, L + 1, ctargets, cptr, csrc, cdir, cy, 1, dinfo);
+        if (!down32) build_waves(P, P.l2lc[L], 2, L, L + 1, ctargets, cptr, csrc, cdir, cy, 1, dinfo);
+        if (!P.l2lc[L].use) build_tree_blocks(P, L, 2, cy, down32);
     }
 }
 
