@@ -300,7 +300,7 @@ __host__ __device__ constexpr int wave64_coax_regs(int P, int m) {   // register
 __host__ __device__ constexpr int wave_sd_pad(int pmax) { return (pmax + 1) * (pmax + 2) / 2 + 8; }
 struct M2LWaveArgs {
     int ps, pt;                      // effective source and target degrees
-    int overwrite;                   // store instead of add (every block in one item)
+    int overwrite;                   // store instead of add: targets that this launch alone writes
     int n_items;
     const int4* items;               // (block, first group, end group, part): part 0 is the whole
                                      // block, s > 0 leaves its sums in slot s - 1 of `part`
@@ -323,7 +323,7 @@ struct M2LWaveArgs {
     const void* coax;
     int coax_stride;
     const void* M;                   // (S, D) entries
-    double2* L;                      // expansions added to (x basis)
+    double2* L;                      // target expansions (x basis)
     const int64_t* exp_off;
 };
 void launch_m2l_wave64(const M2LWaveArgs& a, int p, hipStream_t s);
@@ -337,7 +337,8 @@ void launch_m2l_wave64_batch(const M2LWaveArgs* d_args, const int2* work, int n,
 void launch_to_sd64(const double2* x, double4* sd, int64_t n_boxes, int p, hipStream_t s);
 
 // FP32 M2L with one wave per work item (m2l_wave32.hip), the lists as for FP64 with 32 pairs per
-// group and source offsets in pairs of (S, D) entries.  The operators are sequences of columns of four
+// group and source offsets in pairs of (S, D) entries.  M2L alone: source and target degree are the
+// same, and the sums are stored (overwrite = 1), the first that a level's locals receive.  The operators are sequences of columns of four
 // rows (64 of them per 1 KiB block: wave32_pos).  Rotations, degrees from 1 ascending: split, for the u
 // half and from block kWave32VBlock for the v half, per input the output rows; joint, per input k the
 // u rows, then (k > 0) the v rows.  Coaxial operators, orders ascending: per input degree the real,
@@ -363,7 +364,7 @@ __host__ __device__ constexpr int wave32_coax_vecs(int p, int m) {   // columns 
     return v;
 }
 constexpr int wave32_pos(int v, int i) { return ((v / 64) * 64 + 4 * (v % 16) + i) * 4 + v % 64 / 16; }   // row i of column v
-// pairs of the block of zeros at the front, which degrees above a source's read
+// pairs of the block of zeros at the front, the source of absent pairs
 constexpr int wave32_sd_pad(int pmax) { return (pmax + 1) * (pmax + 2) / 4 + 8; }
 void launch_m2l_wave32(const M2LWaveArgs& a, int p, hipStream_t s);
 int wave32_sum_chunks(int p, int tb);

@@ -67,17 +67,9 @@ __device__ __forceinline__ void unrolled(F&& f) {
 
 // row of (degree n, order m) of half h in the lane's column: u_0..u_n or v_1..v_n, degrees in order
 constexpr int row(int h, int n, int m) { return h ? tri(n - 1) + m - 1 : tri(n) + m; }
-// degree of pair i of entries (its first entry)
-constexpr int pair_degree(int i) {
-    int n = 0;
-    while (tri(n + 1) <= 2 * i) ++n;
-    return n;
-}
-
 // U and V parts (real for even lanes) of degree n and order m stored in the x basis: x_0 = U_0,
 // x_m = (U + V) / 2, x_{-m} = (-1)^m (U - V) / 2
-__device__ __forceinline__ void store_expansion(double* dst, int n, int m, int pt, double u, double v) {
-    if (n > pt || m > n) return;
+__device__ __forceinline__ void store_expansion(double* dst, int n, int m, double u, double v) {
     const double sg = (m & 1) ? -0.5 : 0.5;
     dst[2 * (n * n + n + m)] = m == 0 ? u : 0.5 * (u + v);
     if (m > 0) dst[2 * (n * n + n - m)] = sg * (u - v);
@@ -95,7 +87,7 @@ __host__ __device__ constexpr int joint_lds_bytes(int P) { return 256 * ((P + 1)
 template <int P>
 __device__ __forceinline__ void store_item(const M2LWaveArgs& a, const int4 item, float* U, float* V) {
     constexpr int NU = tri(P + 1), NV = tri(P);
-    const int lane = threadIdx.x, c = lane >> 1, pt = a.pt;
+    const int lane = threadIdx.x, c = lane >> 1;
     const int tb = a.tb;
     unrolled<0, NV>([&](auto ic) { V[IDX(ic)] = other(V[IDX(ic)]); });
     for (int off = 2 * tb; off < 64; off <<= 1) {
@@ -117,7 +109,7 @@ __device__ __forceinline__ void store_item(const M2LWaveArgs& a, const int4 item
     unrolled<0, P + 1>([&](auto nc) {
         unrolled<0, IDX(nc) + 1>([&](auto mc) {
             constexpr int n = IDX(nc), m = IDX(mc), iv = m ? tri(n - 1) + m - 1 : 0;
-            store_expansion(dst, n, m, pt, U[tri(n) + m], m ? V[iv] : 0.0f);
+            store_expansion(dst, n, m, U[tri(n) + m], m ? V[iv] : 0.0f);
         });
     });
 }
@@ -132,7 +124,6 @@ __device__ __forceinline__ void wave32_joint_body(const M2LWaveArgs& a, const in
     constexpr int NB = 2 * BR + BC, RING = kFragAhead + 1, GA = kGatherAhead < NP ? kGatherAhead : NP;
     if (item.y >= item.z) return;   // padding item
     const int lane = threadIdx.x, c = lane >> 1;
-    const int ps = a.ps, pt = a.pt;
     const float sgn = (lane & 1) ? 1.0f : -1.0f;
     float* const X = lds32 + lane;
     float xr[RK > 0 ? RK : 1];
@@ -180,11 +171,10 @@ __device__ __forceinline__ void wave32_joint_body(const M2LWaveArgs& a, const in
     // pair i of the source's entries: S, D, S, D (D the other part of the pair's than S)
     f4 g[GA];
     uint32_t so;
-    const uint32_t sz = 16 * (uint32_t)(lane & 1);   // the block of zeros
+    const uint32_t ri = 16 * (uint32_t)(lane & 1);   // the lane's parts of a pair
     auto gather_load = [&](auto ic) {
         constexpr int i = IDX(ic);
-        const uint32_t o = pair_degree(i) <= ps ? so : sz;
-        g[i % GA] = *(const f4*)((const char*)a.M + 32 * i + o);
+        g[i % GA] = *(const f4*)((const char*)a.M + 32 * i + so);
     };
     float cp[P + 1], tp[P + 1];   // cos m phi; -sin m phi (even lanes), sin m phi (odd)
     float2 phn[P + 1];
@@ -196,7 +186,7 @@ __device__ __forceinline__ void wave32_joint_body(const M2LWaveArgs& a, const in
     };
     int src = a.grp_src[(size_t)item.y * 32 + c], dir = a.grp_dir[(size_t)item.y * 32 + c];
     operators(((ScalarInts)a.grp_class)[item.y]);
-    so = 32 * (uint32_t)src + sz;
+    so = 32 * (uint32_t)src + ri;
     unrolled<0, GA>(gather_load);
     phase_load(dir);
     unrolled<0, kFragAhead>([&](auto bc) {
@@ -255,9 +245,8 @@ __device__ __forceinline__ void wave32_joint_body(const M2LWaveArgs& a, const in
             unrolled<0, n + 1>([&](auto mc) {
                 constexpr int m = IDX(mc), i = tri(n) + m;
                 const f4 w = g[(i / 2) % GA];
-                float S = (i & 1) ? w.z : w.x, D = (i & 1) ? w.w : w.y;
+                const float S = (i & 1) ? w.z : w.x, D = (i & 1) ? w.w : w.y;
                 if constexpr (m == 0) {
-                    if constexpr (i & 1) S = n <= ps ? S : 0.0f;   // beside an entry of degree n - 1
                     u[0] = S;
                 } else {
                     u[m] = fmaf(tp[m], D, cp[m] * S);
@@ -277,7 +266,7 @@ __device__ __forceinline__ void wave32_joint_body(const M2LWaveArgs& a, const in
         finish1(std::integral_constant<int, P>{});
 
         // 2. coaxial operators; the rows of the next order are read before this one's products
-        so = 32 * (uint32_t)src + sz;
+        so = 32 * (uint32_t)src + ri;
         float xu[2][P + 1], xv[2][P + 1];
         auto rows2 = [&](auto mc) {
             constexpr int m = IDX(mc);
@@ -383,7 +372,6 @@ __device__ __forceinline__ void wave32_split_body(const M2LWaveArgs& a, const in
     constexpr int RING = kFragAhead + 1, GA = kGatherAhead < NP ? kGatherAhead : NP;
     if (item.y >= item.z) return;   // padding item
     const int lane = threadIdx.x, c = lane >> 1;
-    const int ps = a.ps, pt = a.pt;
     const float sgn = (lane & 1) ? 1.0f : -1.0f;
     float* const X = lds32 + lane;
     float U[NU], V[NV];   // [tri(n) + m], [tri(n - 1) + m - 1]
@@ -400,11 +388,10 @@ __device__ __forceinline__ void wave32_split_body(const M2LWaveArgs& a, const in
     f4 fr[RING], g[GA];
     // pair i of the source's entries: S, D, S, D (D the other part of the pair's than S)
     uint32_t so;
-    const uint32_t sz = 16 * (uint32_t)(lane & 1);   // the block of zeros
+    const uint32_t ri = 16 * (uint32_t)(lane & 1);   // the lane's parts of a pair
     auto gather_load = [&](auto ic) {
         constexpr int i = IDX(ic);
-        const uint32_t o = pair_degree(i) <= ps ? so : sz;
-        g[i % GA] = *(const f4*)((const char*)a.M + 32 * i + o);
+        g[i % GA] = *(const f4*)((const char*)a.M + 32 * i + so);
     };
     // block b of 64 operator columns of half h: forward rotations, coaxial operators, back rotations
     auto frag_load = [&](auto hc, auto bc) {
@@ -424,7 +411,7 @@ __device__ __forceinline__ void wave32_split_body(const M2LWaveArgs& a, const in
     };
     int src = a.grp_src[(size_t)item.y * 32 + c], dir = a.grp_dir[(size_t)item.y * 32 + c];
     operators(((ScalarInts)a.grp_class)[item.y]);
-    so = 32 * (uint32_t)src + sz;
+    so = 32 * (uint32_t)src + ri;
     unrolled<0, GA>(gather_load);
     unrolled<0, kFragAhead>([&](auto bc) { frag_load(std::integral_constant<int, 0>{}, bc); });
 #pragma unroll 1
@@ -491,12 +478,11 @@ __device__ __forceinline__ void wave32_split_body(const M2LWaveArgs& a, const in
                 unrolled<0, n + 1>([&](auto mc) {
                     constexpr int m = IDX(mc), i = tri(n) + m;
                     const f4 w = g[(i / 2) % GA];
-                    float S = (i & 1) ? w.z : w.x;
+                    const float S = (i & 1) ? w.z : w.x;
                     const float D = (i & 1) ? w.w : w.y;
                     if constexpr (m > 0) {
                         in[m - h] = h ? fmaf(-tp[m], S, cp[m] * D) : fmaf(tp[m], D, cp[m] * S);
                     } else if constexpr (h == 0) {
-                        if constexpr (i & 1) S = n <= ps ? S : 0.0f;   // beside an entry of degree n - 1
                         in[0] = S;
                     }
                     if constexpr (((i & 1) || i == NU - 1) && i / 2 + GA < NP) gather_load(std::integral_constant<int, i / 2 + GA>{});
@@ -551,7 +537,7 @@ __device__ __forceinline__ void wave32_split_body(const M2LWaveArgs& a, const in
             };
             if constexpr (h == 0) U[0] += X[0];
             get_rows(std::integral_constant<int, 1>{});
-            if constexpr (h == 1) so = 32 * (uint32_t)src + sz;
+            if constexpr (h == 1) so = 32 * (uint32_t)src + ri;
             unrolled<0, GA>(gather_load);
             __builtin_amdgcn_sched_barrier(0);
             unrolled<1, P + 1>([&](auto nc) {
@@ -624,7 +610,7 @@ __device__ __forceinline__ void wave32_sum(const M2LWaveArgs& a, int P, int b, i
     if (chunk * kValues + e >= total) return;
     const int tbox = a.blk_targets[(size_t)b * a.tb + l / 2];
     if (tbox < 0) return;
-    store_expansion((double*)(a.L + a.exp_off[tbox]) + (l & 1), n, m, a.pt, u, v);
+    store_expansion((double*)(a.L + a.exp_off[tbox]) + (l & 1), n, m, u, v);
 }
 
 template <int J>
@@ -640,7 +626,7 @@ __global__ __launch_bounds__(kSumThreads) void wave32_sum_batch_kernel(const M2L
 
 // blocks of operator columns and pairs of entries that loads run ahead of their use
 constexpr int kFragsAhead = 2;
-constexpr int pairs_ahead(int p) { return p == 11 ? 3 : 8; }   // p = 11: what 256 registers leave
+constexpr int pairs_ahead(int p) { return p == 11 ? 3 : p == 15 ? 5 : 8; }   // 11, 15: what 256 or 512 registers leave
 
 template <int P>
 __device__ __forceinline__ void wave32_item(const M2LWaveArgs& a, const int4 item) {
@@ -727,6 +713,7 @@ __global__ __launch_bounds__(256) void to_sd32_kernel(const double2* x, float4* 
 
 void launch_m2l_wave32(const M2LWaveArgs& a, int p, hipStream_t s) {
     if (a.n_items <= 0) return;
+    if (!a.overwrite || a.ps != p || a.pt != p) fail(-9, "internal: the FP32 wave kernel stores M2L sums of one degree");
     with_degree(p, [&](auto* k, auto*) { hipLaunchKernelGGL(k, dim3(a.n_items), dim3(64), lds_bytes(p), s, a); });
     check_launch("m2l wave32");
     if (!a.part) return;

@@ -1818,7 +1818,7 @@ void run_sequence(hfmm_plan& P, const void* q, int q_type, double2* out, hipStre
         if (P.m2lc[L].use) {
             if (!(parts & kSeqM2LBlock)) continue;
             if (lev) HIPCHK(hipEventRecord(lev[2 * L], s));
-            launch_wave(P, P.m2lc[L], wave_source(P, P.m2lc[L]), P.dL, 0, s);
+            launch_wave(P, P.m2lc[L], wave_source(P, P.m2lc[L]), P.dL, P.m2lc[L].fp32, s);
             if (lev) HIPCHK(hipEventRecord(lev[2 * L + 1], s));
             continue;
         }
@@ -2533,7 +2533,7 @@ void build_persistent(hfmm_batch& B, void* const* out, int q_type) {
         bool first = true;
         for (auto& [P, c] : kv.second) {
             std::vector<int> part_ptr = c->host_part_ptr;
-            M2LWaveArgs w = wave_args(*P, *c, wave_source(*P, *c), P->dL, 0);
+            M2LWaveArgs w = wave_args(*P, *c, wave_source(*P, *c), P->dL, fp32);
             if (!fp32) {
                 const std::vector<int4> items =
                     wave_items(P->tree, c->host_targets, c->host_ptr, c->tb, per_item, part_ptr);
