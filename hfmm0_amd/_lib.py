@@ -59,6 +59,7 @@ def _declare(lib):
         "hfmm_opts_default": (None, [ctypes.POINTER(Opts)]),
         "hfmm_plan_create": (I, [vp, L, D, ctypes.POINTER(Opts), ctypes.POINTER(vp)]),
         "hfmm_plan_info_get": (I, [vp, ctypes.POINTER(PlanInfo)]),
+        "hfmm_plan_wave_levels": (I, [vp, vp, vp, vp]),
         "hfmm_plan_export_tree": (I, [vp, vp, vp, vp, vp, vp, vp, vp]),
         "hfmm_plan_export_list": (I, [vp, ctypes.c_char, vp]),
         "hfmm_evaluate": (I, [vp, vp, I, vp, I, vp]),
@@ -102,7 +103,7 @@ def _declare(lib):
 
 
 EXPORTED = [
-    "hfmm_opts_default", "hfmm_plan_create", "hfmm_plan_info_get", "hfmm_plan_export_tree", "hfmm_plan_set_degrees",
+    "hfmm_opts_default", "hfmm_plan_create", "hfmm_plan_info_get", "hfmm_plan_wave_levels", "hfmm_plan_export_tree", "hfmm_plan_set_degrees",
     "hfmm_plan_export_list", "hfmm_evaluate", "hfmm_evaluate_typed", "hfmm_evaluate_field", "hfmm_benchmark", "hfmm_benchmark_m2l_levels",
     "hfmm_plan_destroy", "hfmm_direct", "hfmm_direct_noalloc",
     "hfmm_tree_create", "hfmm_tree_create_device", "hfmm_tree_info_get", "hfmm_tree_export", "hfmm_tree_export_list",

@@ -73,6 +73,14 @@ class HFMMState:
         m = self.info.l2l_fp32_levels
         return [i for i in range(1, self.info.depth + 1) if (m >> i) & 1]
 
+    def wave_levels(self):
+        """Levels on the one-wave-per-item matrix-core kernels: {"m2l": [...], "m2m": levels into
+        which, "l2l": levels out of which}."""
+        masks = [ctypes.c_int() for _ in range(3)]
+        L.check(L.lib().hfmm_plan_wave_levels(self.handle, *(ctypes.addressof(m) for m in masks)))
+        return {name: [i for i in range(1, self.info.depth + 1) if (m.value >> i) & 1]
+                for name, m in zip(("m2l", "m2m", "l2l"), masks)}
+
     @property
     def p_table(self):
         """Degree the tables of levels 1..depth were built for."""

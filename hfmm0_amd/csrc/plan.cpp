@@ -2015,6 +2015,21 @@ int hfmm_plan_info_get(const hfmm_plan* P, hfmm_plan_info* info) {
     });
 }
 
+int hfmm_plan_wave_levels(const hfmm_plan* P, int* m2l, int* m2m, int* l2l) {
+    return guarded([&] {
+        if (!P) fail(HFMM_ERR_ARG, "null plan");
+        auto mask = [](const M2LWaveLevel* levels, int* out) {
+            if (!out) return;
+            *out = 0;
+            for (int L = 0; L < kMaxLevels; ++L)
+                if (levels[L].use) *out |= 1 << L;
+        };
+        mask(P->m2lc, m2l);
+        mask(P->m2mc, m2m);
+        mask(P->l2lc, l2l);
+    });
+}
+
 int hfmm_plan_export_tree(const hfmm_plan* P, int* level, uint64_t* code, int* count, int* pstart, int* parent,
                           uint8_t* is_leaf, int64_t* perm) {
     return guarded([&] {

@@ -124,6 +124,11 @@ int hfmm_plan_create(const double* xyz /* N x 3, host */, int64_t n, double k, c
                      hfmm_plan** out);
 int hfmm_plan_info_get(const hfmm_plan* plan, hfmm_plan_info* info);
 
+/* Levels on the matrix-core kernels with one wave per work item (the others run on the block or the
+ * generic kernel): bit l of *m2l is the M2L of level l, of *m2m the M2M into level l, of *l2l the
+ * L2L out of level l.  Each pointer may be NULL. */
+int hfmm_plan_wave_levels(const hfmm_plan* plan, int* m2l, int* m2m, int* l2l);
+
 /* Tree export (canonical order: level ascending, Morton code ascending).  Each array
  * pointer may be NULL; sizes are n_boxes (per-box arrays) or n_points (perm). */
 int hfmm_plan_export_tree(const hfmm_plan* plan, int* level, uint64_t* code, int* count, int* pstart,

@@ -62,6 +62,8 @@ def test_call_after_bad_charges(hf, p):
     q = rng.normal(size=len(x))
     st = hf.setup(x, 3.0, p=p, N_max=1, max_depth=6, tree_device=True)
     assert st.depth == 6
+    w = st.wave_levels()
+    assert w["m2m"] == [4, 5] and w["l2l"] == [4, 5], w
     first = hf.evaluate(st, q)
     q2 = q.copy()
     q2[::7] = np.nan
