@@ -1716,6 +1716,30 @@ void level_to_sd(const hfmm_plan& P, int l, const double2* e, double4* sd, hipSt
     if (b1 > b0) launch_to_sd64(e + P.exp_off[b0], sd + P.sd_off[b0], b1 - b0, P.p_level[l], s);
 }
 
+// The multipoles of the levels whose M2L the wave kernels take, in (S, D) form (FP64 levels but those
+// of `done`): one launch per run of levels of one precision and table degree.  A launch per level made
+// the upward passes of 64 problems of 30 points, which are launches alone, 10% longer.
+void levels_to_sd(const hfmm_plan& P, const bool* done, hipStream_t s) {
+    const Tree& t = P.tree;
+    auto needed = [&](int l, bool fp32) {
+        return l <= P.depth && P.m2lc[l].use && P.m2lc[l].fp32 == fp32 && (fp32 || !done[l]);
+    };
+    for (int l = 2; l <= P.depth;) {
+        const bool fp32 = P.m2lc[l].fp32;
+        if (!needed(l, fp32)) {
+            ++l;
+            continue;
+        }
+        const int b0 = t.level_start[l], p = P.p_level[l];
+        while (needed(l, fp32) && P.p_level[l] == p) ++l;
+        const int n = t.level_start[l] - b0;
+        if (fp32)
+            launch_to_sd32(P.dM + P.exp_off[b0], P.dMs32 + 2 * P.sd32_off[b0], n, p, s);
+        else
+            launch_to_sd64(P.dM + P.exp_off[b0], P.dMs + P.sd_off[b0], n, p, s);
+    }
+}
+
 int out_mode_of(const hfmm_plan& P, int q_type) {
     return (P.conj ? 1 : 0) | ((P.k == 0.0 && real_charges(q_type)) ? 2 : 0);
 }
@@ -1787,16 +1811,9 @@ void run_sequence(hfmm_plan& P, const void* q, int q_type, double2* out, hipStre
                 launch_xlate(xargs(P, P.m2m[L], P.dM, P.dM, 0), P.m2m[L].n_targets, s);
         }
         mark(3);
+        levels_to_sd(P, conv_sd, s);
         // multipoles in FP32 for the FP32 block levels: every level not converted for an FP32
         // M2M (the converted ones need not be contiguous), one launch per run of levels
-        for (int L = 2; L <= P.depth; ++L)
-            if (P.m2lc[L].use && P.m2lc[L].fp32) {
-                const Tree& t = P.tree;
-                const int b0 = t.level_start[L], b1 = t.level_start[L + 1];
-                launch_to_sd32(P.dM + P.exp_off[b0], P.dMs32 + 2 * P.sd32_off[b0], b1 - b0, P.p_level[L], s);
-            } else if (P.m2lc[L].use && !conv_sd[L]) {
-                level_to_sd(P, L, P.dM, P.dMs, s);
-            }
         bool any_fp32 = false;
         for (int L = 2; L <= P.depth; ++L) any_fp32 |= P.m2l[L].n_targets && P.m2lb[L].use && P.m2lb[L].fp32;
         if (any_fp32)
