@@ -713,6 +713,21 @@ void pack_wave_coax(const hfmm_plan& P, M2LWaveLevel& B) {
     HIPCHK(hipMemcpy(B.coax, cf.data(), cf.size() * sizeof(double), hipMemcpyHostToDevice));
 }
 
+// Pairs from which the M2L of a level runs on the wave kernels.  Below, the level is over in one wave per
+// group whatever their number: the time is that of fetching the straight-line code, and of the launches
+// for the sums and the (S, D) form, while the block kernel's is a few sources per target.  Whole
+// evaluates with one M2L level, wave against block kernel, FP64: 190 pairs 44.3 / 41.6 us at p = 2, 59.9 / 50.9
+// at p = 8, 87.5 / 63.2 at p = 14; 514 pairs 44.7 / 45.8, 61.6 / 62.3, 91.3 / 86.2; 986 pairs 44.2 / 49.0, 61.2 /
+// 73.2, 99.3 / 104.9 (but a level of 956 at p = 14 10 us longer).  FP32, whose sums are shorter: 34 pairs
+// 40.8 / 43.3 at p = 2, 56.2 / 56.2 at p = 10; 190 pairs 64.1 / 69.4 at p = 11, 78.1 / 69.5 at p = 14; 388
+// pairs 78.1 / 84.0 at p = 14, 106 / 83.5 at p = 15.  A batch's FP64 levels share their launches and take
+// the wave kernel at any size (64 problems of 30 points at p = 9: M2L 0.25 ms, 1.38 on the block kernel);
+// its FP32 levels follow the plan's own rule, so that a problem's result is the one it has alone.
+int wave_min_pairs(int p, bool fp32) {
+    if (fp32) return p <= 10 ? 0 : p == 11 ? 128 : p <= 14 ? 288 : 960;
+    return p <= 13 ? 128 + 48 * p : 1024;
+}
+
 // Translation of one level on the wave kernel: targets with their (source, direction) lists.
 // kind 0: M2L, 1: M2M, 2: L2L; coax: packed tables as X.coax (interleaved complex).
 void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt_level, const std::vector<int>& targets,
@@ -720,6 +735,7 @@ void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt
                    const std::vector<double>& coax, int n_dist, const std::vector<DispInfo>& dinfo, bool fp32 = false) {
     const int ps = P.p_level[src_level], pt = P.p_level[tgt_level], pm = std::max(ps, pt);
     if (P.m2l_kernel != 0 || pm > (fp32 ? kWave32MaxP : kWave64MaxP) || !P.d_cr1) return;
+    if (kind == 0 && (fp32 || !P.in_batch) && (int)src.size() < wave_min_pairs(pm, fp32)) return;
     // the kernels address the sources with 32-bit byte offsets
     const int64_t bytes = fp32 ? (P.n_sd32 + wave32_sd_pad(P.pmax)) * 2 * (int64_t)sizeof(float4)
                                : (P.n_sd + wave_sd_pad(P.pmax)) * (int64_t)sizeof(double4);

@@ -83,3 +83,35 @@ def test_cluster_alone(hf):
     q = rng.normal(size=len(x)) + 1j * rng.normal(size=len(x))
     st = hf.setup(x, 3.0, p=4, N_max=2600, max_depth=1)
     assert D.relative_error(hf.evaluate(st, q), D.direct_c(x, q, 3.0)) < 1e-13
+
+
+@pytest.mark.parametrize("n,p,precision,wave", [(26, 2, "fp64", False), (26, 9, "fp64", False), (100, 9, "fp64", True),
+                                                (52, 13, "fp64", True), (52, 14, "fp64", False), (100, 14, "fp64", True),
+                                                (8, 2, "mixed", True), (8, 10, "mixed", True), (8, 11, "mixed", False),
+                                                (26, 14, "mixed", False), (52, 14, "mixed", True), (52, 15, "mixed", True),
+                                                (40, 15, "mixed", False)])
+def test_small_levels(hf, n, p, precision, wave):
+    """One M2L level of 34 pairs (8 points) to 1886 (100 points): few pairs stay on the block kernel,
+    whose time they are (a whole evaluate of 26 points at p = 9 took 62 us on the wave kernel, 53 on the
+    block kernel).  In a batch the FP64 level takes the wave kernel at any size."""
+    from hfmm0_amd.batch import Batch
+    print(f"case: one small M2L level, {n} points, p={p}, {precision}", flush=True)
+    rng = np.random.default_rng(n)
+    x = rng.uniform(size=(n, 3))
+    x[0], x[1] = 0.001, 0.999
+    q = rng.normal(size=n) + 1j * rng.normal(size=n)
+    kw = dict(p=p, N_max=1, max_depth=2, precision=precision)
+    st = hf.setup(x, 6.0, **kw)
+    assert st.depth == 2 and st.wave_levels()["m2l"] == ([2] if wave else [])
+    kw["precision"] = "fp64"
+    ref = hf.evaluate(hf.setup(x, 6.0, m2l_kernel="generic", **kw), q)
+    tol = 1e-13 if precision == "fp64" else 2e-6
+    phi = hf.evaluate(st, q)
+    assert D.relative_error(phi, ref) < tol
+    kw["precision"] = precision
+    kw.pop("max_depth")
+    B = Batch([x, x], [6.0, 6.0], max_depth=2, **kw)
+    assert B.plan(0).wave_levels()["m2l"] == ([2] if wave or precision == "fp64" else [])
+    for v in B.evaluate([q, q]):
+        assert D.relative_error(v, ref) < tol
+    B.close()
