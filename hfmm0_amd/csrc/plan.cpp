@@ -728,6 +728,12 @@ int wave_min_pairs(int p, bool fp32) {
     return p <= 13 ? 128 + 48 * p : 1024;
 }
 
+// Largest degrees whose M2M and L2L run on the wave kernel: their few directions suit the block kernel,
+// and above p = 7 the wave kernel has one wave per SIMD.  Levels 4 and 5 of 600k points, wave against block
+// kernel, M2M: 0.39 / 0.57 ms at p = 7, 0.75 / 0.81 at 10, 0.86 / 0.85 at 11, 1.06 / 0.97 at 12, 1.53 / 1.09 at
+// 14; L2L: 0.35 / 0.67 at p = 7, 0.82 / 1.05 at 10, 1.13 / 1.30 at 12, 1.29 / 1.40 at 13, 1.68 / 1.58 at 14.
+constexpr int kWaveM2MMaxP = 10, kWaveL2LMaxP = 13;
+
 // Translation of one level on the wave kernel: targets with their (source, direction) lists.
 // kind 0: M2L, 1: M2M, 2: L2L; coax: packed tables as X.coax (interleaved complex).
 void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt_level, const std::vector<int>& targets,
@@ -736,6 +742,7 @@ void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt
     const int ps = P.p_level[src_level], pt = P.p_level[tgt_level], pm = std::max(ps, pt);
     if (P.m2l_kernel != 0 || pm > (fp32 ? kWave32MaxP : kWave64MaxP) || !P.d_cr1) return;
     if (kind == 0 && (fp32 || !P.in_batch) && (int)src.size() < wave_min_pairs(pm, fp32)) return;
+    if ((kind == 1 && pm > kWaveM2MMaxP) || (kind == 2 && pm > kWaveL2LMaxP)) return;
     // the kernels address the sources with 32-bit byte offsets
     const int64_t bytes = fp32 ? (P.n_sd32 + wave32_sd_pad(P.pmax)) * 2 * (int64_t)sizeof(float4)
                                : (P.n_sd + wave_sd_pad(P.pmax)) * (int64_t)sizeof(double4);
@@ -786,10 +793,8 @@ void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt
         const int64_t cost = g + (fp32 ? (int64_t)kWaveItems * c / 64 : 0);
         if (!tb || cost < best_cost) tb = c, best = g, best_cost = cost;
     }
-    // The kernel's code for one group is straight-line, 15 to 40 KB, and every compute unit
-    // fetches it once: a launch of a group or two per wave spends most of its time on that (M2M
-    // of 512 children at p = 10: 42 us, against 20 for the block kernel; M2L of 3096 pairs: 28
-    // against 53).  M2M and L2L take it from 2 groups per SIMD on.
+    // M2M and L2L take the kernel from 2 groups per SIMD on: a launch of a group or two per wave spends
+    // most of its time on fetching the code (M2M of 512 children at p = 10: 42 us, 20 on the block kernel).
     if (kind != 0 && best < 2048) return;
     const int slots = pairs / tb, nblk = (nt + tb - 1) / tb;
     std::vector<int> blk_targets((size_t)nblk * tb, -1), blk_ptr{0}, gcls, gsrc;

@@ -115,3 +115,18 @@ def test_small_levels(hf, n, p, precision, wave):
     for v in B.evaluate([q, q]):
         assert D.relative_error(v, ref) < tol
     B.close()
+
+
+@pytest.mark.parametrize("p,m2m,l2l", [(10, True, True), (11, False, True), (13, False, True), (14, False, False)])
+def test_tree_levels_by_degree(hf, p, m2m, l2l):
+    """M2M runs on the wave kernel up to p = 10 and L2L up to 13, where the block kernel is slower; a
+    level at a higher degree on either side counts as that degree.  Results against the generic kernel."""
+    print(f"case: tree levels at p={p}", flush=True)
+    x, q = _cube(250000, p)
+    levels = [4, 4, 4, p, 4, 4]            # levels 3 -> 4 and 4 -> 5 with degree p on one side
+    kw = dict(p=p, N_max=1, max_depth=6, tree_device=True, p_level=levels)
+    s = hf.setup(x, 5.0, **kw)
+    w = s.wave_levels()
+    assert (4 in w["m2m"]) == m2m and (4 in w["l2l"]) == l2l, w
+    assert 5 in w["m2m"] and 5 in w["l2l"], w
+    assert D.relative_error(hf.evaluate(s, q), hf.evaluate(hf.setup(x, 5.0, m2l_kernel="generic", **kw), q)) < 1e-13
