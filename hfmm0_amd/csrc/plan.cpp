@@ -755,7 +755,10 @@ void build_waves(hfmm_plan& P, M2LWaveLevel& B, int kind, int src_level, int tgt
     std::vector<int> cls_of(kNumDirs, -1), cls_key;
     {
         std::map<std::pair<int, int>, int> ids;
-        for (unsigned short d : dir) ids.emplace(std::make_pair(dinfo[d].theta, dinfo[d].dist), 0);
+        std::vector<char> present(kNumDirs, 0);
+        for (unsigned short d : dir) present[d] = 1;
+        for (int d = 0; d < kNumDirs; ++d)
+            if (present[d]) ids.emplace(std::make_pair(dinfo[d].theta, dinfo[d].dist), 0);
         for (auto& kv : ids) {
             kv.second = (int)cls_key.size();
             cls_key.push_back(kv.first.first | kv.first.second << 16);
