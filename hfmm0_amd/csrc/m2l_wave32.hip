@@ -22,9 +22,9 @@
 // SIMD; above, one wave per SIMD takes both at once (wave32_joint_body), each with its layout of the
 // operators (p = 11: split 1.81 ms, joint 1.97 on 5.4M pairs; p = 12: split 0.366, joint 0.329 on 584136).
 // Bound by the issue of MFMA and VALU instructions, which do not overlap on this chip (1358 MFMAs of 8
-// cycles and 870 VALU instructions per group at p = 11, three quarters of its time), and by what the
-// latencies leave exposed.  Against the block kernel (16 x 16 x 4 tiles, 16 targets x 2 directions per
-// workgroup): 5.4M pairs at p = 11 3.96 -> 1.84 + 0.04 ms (sums), 584136 at p = 12 0.84 -> 0.325, 53352 at
+// cycles and 744 VALU instructions per group at p = 11: 50% and 14% of the time on 5.4M pairs, 43% and
+// 13% at p = 12, one wave per SIMD), and by what the latencies leave exposed.  Against the block kernel (16 x 16 x 4 tiles, 16 targets x 2 directions per
+// workgroup): 5.4M pairs at p = 11 3.96 -> 1.65 ms with the sums, 584136 at p = 12 0.84 -> 0.325, 53352 at
 // p = 14 0.19 -> 0.077; the five levels of 100k points (p = 11) 1.39 -> 0.33 ms, of 300k on surfaces (p = 10)
 // 2.3 -> 0.52, of 150k at k = 0 (p = 7) 0.52 -> 0.136.  Errors against FP64 are those of the block kernel
 // (1.1e-7 to 1.6e-7 of the potential).

@@ -17,13 +17,14 @@
 // and once for the imaginary parts, so that an operator fragment feeds two MFMAs and the complex
 // products need no exchange between lanes.  No other wave touches the wave's columns: there are no
 // barriers, and the whole group is straight-line code for a degree P known at compile time, whose
-// operator loads run ahead of their use.  Bound by the issue of FP64 MFMA and FP64 VALU
-// instructions, which do not overlap on this chip, and by what the latencies of a single wave per
-// SIMD leave exposed (degrees above 7 take more than 256 registers).
+// operator loads run ahead of their use.  Degrees above 7 take more than 256 registers, so that one
+// wave per SIMD is left, and its latencies are exposed: of 584136 pairs at p = 14 (1.9 ms) the matrix
+// pipe is busy 34% of the time (two thirds of that on entries of the operators, the rest on tile
+// padding), other VALU instructions take 7%, and the wave waits on dependencies for a third.
 // Against the block kernel's 8 targets x 1 direction per workgroup: 584136 pairs at p = 14 1.95 ms
 // against 2.41, 53352 pairs at p = 10 0.13 + 0.01 ms against 0.29, the levels of 60k points on
 // surfaces (p = 12) 0.99 ms against 2.00, a batch of 16 problems of 2k to 20k points (p = 10) 1.4 ms
-// against 9.7.  Where levels are irregular the gain is in the packing: pairs of a target
+// against 9.7.  (plan.cpp has the sizes and degrees at which a level takes this kernel.)  Where levels are irregular the gain is in the packing: pairs of a target
 // fill the columns whatever their azimuth, where the block kernel leaves a column empty for every
 // target without a source in the block's direction.
 //
@@ -98,14 +99,14 @@ __device__ __forceinline__ void store_expansion(double2* dst, int n, int m, int 
     if (m > 0) *ym = xm;
 }
 
-// One work item (block, first group, end group, part) at degree P: part 0 stores its sums, part
-// s > 0 leaves them in slot s - 1 of the partial sums.
 // 16 bytes at a uniform base plus a 32-bit lane offset: a scalar base register pair and one
 // vector register (64-bit lane addresses of the many fragments would take the registers)
 __device__ __forceinline__ double2 load16(const void* base, uint32_t off) {
     return *(const double2*)((const char*)base + off);
 }
 
+// One work item (block, first group, end group, part) at degree P: part 0 stores its sums, part
+// s > 0 leaves them in slot s - 1 of the partial sums.
 template <int P, int kFragAhead, int kGatherAhead>
 __device__ __forceinline__ void wave64_body(const M2LWaveArgs& a, const int4 item) {
     // row tri(n) + m: 16 pairs of (re, im); the last rows pad the reads of the last block

@@ -2653,8 +2653,9 @@ void build_persistent(hfmm_batch& B, void* const* out, int q_type) {
         for (int i = 0; i < np; ++i) {
             const hfmm_plan& P = *B.plans[i];
             const auto [l0, l1] = leaves(P, c);
-            // the chunks of a mixed problem are those of its plan alone: they decide which sources
-            // are summed in FP32, and a batch gives each problem's own result
+            // the chunks of a mixed problem are those of its plan alone at the default tile of two
+            // targets per lane (other tiles split the sources over the lanes otherwise): they decide
+            // which sources are summed in FP32, and a batch gives each problem's own result
             if (c == kP2PClassFp64)
                 w.add(P.tree, P.leaf_box, P.leaf_total, l0, l1, kP2PFp64TargetsPerLane, near_limit(pairs), i);
             else
