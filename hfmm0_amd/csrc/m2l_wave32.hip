@@ -1,17 +1,15 @@
 // M2L in FP32 on matrix cores, one wave per work item and one matrix column per lane.
 //
-// Basis, groups and work items are those of the FP64 kernel (m2l_wave64.hip): S and D halves, pairs
-// (target box, source box) of equal polar angle and length, partial sums for split blocks.  Here a
-// group is 32 pairs, and lane 2 c + j holds the real (j = 0) or imaginary (j = 1) part of every
-// S or u entry of pair c, and the other part of every D or v entry: u = c S + i s D and
-// v = c D + i s S then need no exchange between lanes.  Every product is a chain of 4 x 4 x 1 MFMAs of 16 blocks: their 64 columns are
-// the lanes, a B operand is one entry of the lane's column in one register, and the A operand, a
-// column of four operator entries, is the same for all blocks (cbsz = 4 broadcasts the block `abid`
-// of a register, so that one register holds 16 such columns and a 16-byte load 64 of them).
-// Compared with 16 x 16 x 4 tiles the inner dimension needs no padding and the rows are padded to
-// four, and no data moves between lanes but the exchange of real and imaginary parts for the complex
-// coaxial products (DPP).  Per group and
-// half, u, then v:
+// Basis, groups and work items are those of the FP64 kernel (m2l_wave64.hip): S and D halves, pairs (target
+// box, source box) of equal polar angle and length, partial sums for split blocks.  Here a group is 32 pairs,
+// and lane 2 c + j holds the real (j = 0) or imaginary (j = 1) part of every S or u entry of pair c, and the
+// other part of every D or v entry: u = c S + i s D and v = c D + i s S then need no exchange between lanes.
+// Every product is a chain of 4 x 4 x 1 MFMAs of 16 blocks: their 64 columns are the lanes, a B operand is one
+// entry of the lane's column in one register, and the A operand, a column of four operator entries, is the
+// same for all blocks (cbsz = 4 broadcasts the block `abid` of a register, so that one register holds 16 such
+// columns and a 16-byte load 64 of them). Compared with 16 x 16 x 4 tiles the inner dimension needs no padding
+// and the rows are padded to four, and no data moves between lanes but the exchange of real and imaginary
+// parts for the complex coaxial products (DPP).  Per group and half, u, then v:
 //   1. per degree n: the source's S and D entries (loaded straight into registers) times e^{i m phi}
 //      are the inputs of the forward rotation; its results go to LDS, which serves as a register
 //      extension: a lane reads its own column only;
@@ -21,13 +19,13 @@
 // Up to degree 11 the two halves go one after the other (wave32_split_body), which lets two waves fit a
 // SIMD; above, one wave per SIMD takes both at once (wave32_joint_body), each with its layout of the
 // operators (p = 11: split 1.81 ms, joint 1.97 on 5.4M pairs; p = 12: split 0.366, joint 0.329 on 584136).
-// Bound by the issue of MFMA and VALU instructions, which do not overlap on this chip (1358 MFMAs of 8
-// cycles and 744 VALU instructions per group at p = 11: 50% and 14% of the time on 5.4M pairs, 43% and
-// 13% at p = 12, one wave per SIMD), and by what the latencies leave exposed.  Against the block kernel (16 x 16 x 4 tiles, 16 targets x 2 directions per
-// workgroup): 5.4M pairs at p = 11 3.96 -> 1.65 ms with the sums, 584136 at p = 12 0.84 -> 0.325, 53352 at
-// p = 14 0.19 -> 0.077; the five levels of 100k points (p = 11) 1.39 -> 0.33 ms, of 300k on surfaces (p = 10)
-// 2.3 -> 0.52, of 150k at k = 0 (p = 7) 0.52 -> 0.136.  Errors against FP64 are those of the block kernel
-// (1.1e-7 to 1.6e-7 of the potential).
+// Bound by the issue of MFMA and VALU instructions, which do not overlap on this chip (1358 MFMAs of 8 cycles
+// and 744 VALU instructions per group at p = 11: 50% and 14% of the time on 5.4M pairs, 43% and 13% at p = 12,
+// one wave per SIMD), and by what the latencies leave exposed.  Against the block kernel (16 x 16 x 4 tiles,
+// 16 targets x 2 directions per workgroup): 5.4M pairs at p = 11 3.96 -> 1.65 ms with the sums, 584136 at p =
+// 12 0.84 -> 0.325, 53352 at p = 14 0.19 -> 0.077; the five levels of 100k points (p = 11) 1.39 -> 0.33 ms, of
+// 300k on surfaces (p = 10) 2.3 -> 0.52, of 150k at k = 0 (p = 7) 0.52 -> 0.136.  Errors against FP64 are
+// those of the block kernel (1.1e-7 to 1.6e-7 of the potential).
 #include <hip/hip_runtime.h>
 
 #include <string>

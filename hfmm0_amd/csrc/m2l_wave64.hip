@@ -24,9 +24,10 @@
 // Against the block kernel's 8 targets x 1 direction per workgroup: 584136 pairs at p = 14 1.95 ms
 // against 2.41, 53352 pairs at p = 10 0.13 + 0.01 ms against 0.29, the levels of 60k points on
 // surfaces (p = 12) 0.99 ms against 2.00, a batch of 16 problems of 2k to 20k points (p = 10) 1.4 ms
-// against 9.7.  (plan.cpp has the sizes and degrees at which a level takes this kernel.)  Where levels are irregular the gain is in the packing: pairs of a target
-// fill the columns whatever their azimuth, where the block kernel leaves a column empty for every
-// target without a source in the block's direction.
+// against 9.7.  (plan.cpp has the sizes and degrees at which a level takes this kernel.)  Where levels
+// are irregular the gain is in the packing: pairs of a target fill the columns whatever their azimuth,
+// where the block kernel leaves a column empty for every target without a source in the block's
+// direction.
 //
 // Source and target degrees may differ (M2M, L2L): P is the larger, the tables are padded with
 // zeros, absent source degrees enter as zeros and absent target degrees are not stored.
