@@ -336,6 +336,17 @@ void launch_m2l_wave64_batch(const M2LWaveArgs* d_args, const int2* work, int n,
 // the expansions of n_boxes consecutive boxes of degree p as (S_re, S_im, D_re, D_im) entries
 void launch_to_sd64(const double2* x, double4* sd, int64_t n_boxes, int p, hipStream_t s);
 
+// the same for runs of boxes of many plans: n entries (FP64) or pairs (FP32) of a run, work[i] = (run, chunk)
+struct SdRun {
+    const double2* x;
+    void* sd;
+    int64_t n;
+    int P1, pad;
+};
+constexpr int kSdChunk = 1024;
+void launch_to_sd64_batch(const SdRun* runs, const int2* work, int n, hipStream_t s);
+void launch_to_sd32_batch(const SdRun* runs, const int2* work, int n, hipStream_t s);
+
 // FP32 M2L with one wave per work item (m2l_wave32.hip), the lists as for FP64 with 32 pairs per
 // group and source offsets in pairs of (S, D) entries.  M2L alone: source and target degree are the
 // same, and the sums are stored (overwrite = 1), the first that a level's locals receive.  The operators are sequences of columns of four

@@ -672,39 +672,49 @@ void with_degree(int p, F&& f) {
     }
 }
 
-// expansions of a level's boxes (contiguous, (p+1)^2 each) as pairs of entries tri(n) + m in FP32:
-// Re S, Im D of both, then Im S, Re D of both; a box starts at a whole pair
-__global__ __launch_bounds__(256) void to_sd32_kernel(const double2* x, float4* sd, int64_t n, int P1) {
+// Pair i of the FP32 (S, D) form of consecutive boxes' expansions ((p+1)^2 each), entries tri(n) + m: Re S,
+// Im D of both, then Im S, Re D of both; a box starts at a whole pair
+__device__ __forceinline__ void to_sd32(const double2* x, float4* sd, int64_t i, int P1) {
     const int te = P1 * (P1 + 1) / 2, np = (te + 1) / 2;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-        const int64_t b = i / np;
-        const int e0 = 2 * (int)(i - b * np);
-        float4 re = make_float4(0, 0, 0, 0), im = re;
+    const int64_t b = i / np;
+    const int e0 = 2 * (int)(i - b * np);
+    float4 re = make_float4(0, 0, 0, 0), im = re;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int e = e0 + j;
-            if (e >= te) break;
-            int nn = (int)((sqrtf(8.0f * (float)e + 1.0f) - 1.0f) * 0.5f);   // the largest with tri(nn) <= e
-            if (tri(nn + 1) <= e) ++nn;
-            if (tri(nn) > e) --nn;
-            const int m = e - tri(nn);
-            const double2* xb = x + b * P1 * P1 + nn * nn + nn;
-            const double2 xp = xb[m];
-            double2 s = xp, d = make_double2(0.0, 0.0);
-            if (m > 0) {
-                double2 xm = xb[-m];
-                if (m & 1) xm = make_double2(-xm.x, -xm.y);
-                s = make_double2(xp.x + xm.x, xp.y + xm.y);
-                d = make_double2(xp.x - xm.x, xp.y - xm.y);
-            }
-            (j ? re.z : re.x) = (float)s.x;
-            (j ? re.w : re.y) = (float)d.y;
-            (j ? im.z : im.x) = (float)s.y;
-            (j ? im.w : im.y) = (float)d.x;
+    for (int j = 0; j < 2; ++j) {
+        const int e = e0 + j;
+        if (e >= te) break;
+        int nn = (int)((sqrtf(8.0f * (float)e + 1.0f) - 1.0f) * 0.5f);   // the largest with tri(nn) <= e
+        if (tri(nn + 1) <= e) ++nn;
+        if (tri(nn) > e) --nn;
+        const int m = e - tri(nn);
+        const double2* xb = x + b * P1 * P1 + nn * nn + nn;
+        const double2 xp = xb[m];
+        double2 s = xp, d = make_double2(0.0, 0.0);
+        if (m > 0) {
+            double2 xm = xb[-m];
+            if (m & 1) xm = make_double2(-xm.x, -xm.y);
+            s = make_double2(xp.x + xm.x, xp.y + xm.y);
+            d = make_double2(xp.x - xm.x, xp.y - xm.y);
         }
-        sd[2 * i] = re;
-        sd[2 * i + 1] = im;
+        (j ? re.z : re.x) = (float)s.x;
+        (j ? re.w : re.y) = (float)d.y;
+        (j ? im.z : im.x) = (float)s.y;
+        (j ? im.w : im.y) = (float)d.x;
     }
+    sd[2 * i] = re;
+    sd[2 * i + 1] = im;
+}
+
+__global__ __launch_bounds__(256) void to_sd32_kernel(const double2* x, float4* sd, int64_t n, int P1) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) to_sd32(x, sd, i, P1);
+}
+
+// work[i] = (run, chunk of kSdChunk pairs)
+__global__ __launch_bounds__(256) void to_sd32_batch_kernel(const SdRun* __restrict__ runs, const int2* __restrict__ work) {
+    const int2 wk = work[blockIdx.x];
+    const SdRun r = runs[wk.x];
+    const int64_t i0 = (int64_t)wk.y * kSdChunk, i1 = min(r.n, i0 + kSdChunk);
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += 256) to_sd32(r.x, (float4*)r.sd, i, r.P1);
 }
 
 }  // namespace
@@ -739,6 +749,12 @@ void launch_to_sd32(const double2* x, float4* sd, int64_t n_boxes, int p, hipStr
     hipLaunchKernelGGL(to_sd32_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 65536)), dim3(256), 0, s, x, sd,
                        n, p + 1);
     check_launch("to_sd32");
+}
+
+void launch_to_sd32_batch(const SdRun* runs, const int2* work, int n, hipStream_t s) {
+    if (n <= 0) return;
+    hipLaunchKernelGGL(to_sd32_batch_kernel, dim3(n), dim3(256), 0, s, runs, work);
+    check_launch("to_sd32 batch");
 }
 
 }  // namespace hfmm

@@ -417,27 +417,37 @@ void with_degree(int p, F&& f) {
     }
 }
 
-// expansions of a level's boxes (contiguous, (p+1)^2 each) as (S_re, S_im, D_re, D_im) per
-// entry tri(n) + m
-__global__ __launch_bounds__(256) void to_sd64_kernel(const double2* x, double4* sd, int64_t n, int P1) {
+// Entry i of the (S, D) form (S_re, S_im, D_re, D_im; tri(n) + m within a box) of consecutive boxes'
+// expansions ((p+1)^2 each)
+__device__ __forceinline__ void to_sd64(const double2* x, double4* sd, int64_t i, int P1) {
     const int te = P1 * (P1 + 1) / 2;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-        const int64_t b = i / te;
-        const int e = (int)(i - b * te);
-        int nn = (int)((sqrtf(8.0f * (float)e + 1.0f) - 1.0f) * 0.5f);   // the largest with tri(nn) <= e
-        if (tri(nn + 1) <= e) ++nn;
-        if (tri(nn) > e) --nn;
-        const int m = e - tri(nn);
-        const double2* xb = x + b * P1 * P1 + nn * nn + nn;
-        const double2 xp = xb[m];
-        double4 o = make_double4(xp.x, xp.y, 0.0, 0.0);
-        if (m > 0) {
-            double2 xm = xb[-m];
-            if (m & 1) xm = make_double2(-xm.x, -xm.y);
-            o = make_double4(xp.x + xm.x, xp.y + xm.y, xp.x - xm.x, xp.y - xm.y);
-        }
-        sd[i] = o;
+    const int64_t b = i / te;
+    const int e = (int)(i - b * te);
+    int nn = (int)((sqrtf(8.0f * (float)e + 1.0f) - 1.0f) * 0.5f);   // the largest with tri(nn) <= e
+    if (tri(nn + 1) <= e) ++nn;
+    if (tri(nn) > e) --nn;
+    const int m = e - tri(nn);
+    const double2* xb = x + b * P1 * P1 + nn * nn + nn;
+    const double2 xp = xb[m];
+    double4 o = make_double4(xp.x, xp.y, 0.0, 0.0);
+    if (m > 0) {
+        double2 xm = xb[-m];
+        if (m & 1) xm = make_double2(-xm.x, -xm.y);
+        o = make_double4(xp.x + xm.x, xp.y + xm.y, xp.x - xm.x, xp.y - xm.y);
     }
+    sd[i] = o;
+}
+
+__global__ __launch_bounds__(256) void to_sd64_kernel(const double2* x, double4* sd, int64_t n, int P1) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) to_sd64(x, sd, i, P1);
+}
+
+// work[i] = (run, chunk of kSdChunk entries)
+__global__ __launch_bounds__(256) void to_sd64_batch_kernel(const SdRun* __restrict__ runs, const int2* __restrict__ work) {
+    const int2 wk = work[blockIdx.x];
+    const SdRun r = runs[wk.x];
+    const int64_t i0 = (int64_t)wk.y * kSdChunk, i1 = min(r.n, i0 + kSdChunk);
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += 256) to_sd64(r.x, (double4*)r.sd, i, r.P1);
 }
 
 size_t lds_bytes(int p) { return (size_t)16 * (tri(p + 1) + 7) * sizeof(double2); }
@@ -471,6 +481,12 @@ void launch_to_sd64(const double2* x, double4* sd, int64_t n_boxes, int p, hipSt
     hipLaunchKernelGGL(to_sd64_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 65536)), dim3(256), 0, s, x, sd,
                        n, p + 1);
     check_launch("to_sd64");
+}
+
+void launch_to_sd64_batch(const SdRun* runs, const int2* work, int n, hipStream_t s) {
+    if (n <= 0) return;
+    hipLaunchKernelGGL(to_sd64_batch_kernel, dim3(n), dim3(256), 0, s, runs, work);
+    check_launch("to_sd64 batch");
 }
 
 }  // namespace hfmm

@@ -1740,14 +1740,19 @@ void level_to_sd(const hfmm_plan& P, int l, const double2* e, double4* sd, hipSt
     if (b1 > b0) launch_to_sd64(e + P.exp_off[b0], sd + P.sd_off[b0], b1 - b0, P.p_level[l], s);
 }
 
-// The multipoles of the levels whose M2L the wave kernels take, in (S, D) form (FP64 levels but those
-// of `done`): one launch per run of levels of one precision and table degree.  A launch per level made
-// the upward passes of 64 problems of 30 points, which are launches alone, 10% longer.
-void levels_to_sd(const hfmm_plan& P, const bool* done, hipStream_t s) {
+// Runs of levels of one precision and table degree whose M2L the wave kernels take, less the FP64
+// levels that M2M has in (S, D) form already.  A run is contiguous in both buffers: one launch.  (A launch per
+// level made the upward passes of 64 problems of 30 points, which are launches alone, 10% longer.)
+struct LevelRun {
+    int b0, n, p;
+    bool fp32;
+};
+std::vector<LevelRun> sd_runs(const hfmm_plan& P) {
     const Tree& t = P.tree;
     auto needed = [&](int l, bool fp32) {
-        return l <= P.depth && P.m2lc[l].use && P.m2lc[l].fp32 == fp32 && (fp32 || !done[l]);
+        return l <= P.depth && P.m2lc[l].use && P.m2lc[l].fp32 == fp32 && (fp32 || !P.m2mc[l - 1].use);
     };
+    std::vector<LevelRun> runs;
     for (int l = 2; l <= P.depth;) {
         const bool fp32 = P.m2lc[l].fp32;
         if (!needed(l, fp32)) {
@@ -1756,12 +1761,9 @@ void levels_to_sd(const hfmm_plan& P, const bool* done, hipStream_t s) {
         }
         const int b0 = t.level_start[l], p = P.p_level[l];
         while (needed(l, fp32) && P.p_level[l] == p) ++l;
-        const int n = t.level_start[l] - b0;
-        if (fp32)
-            launch_to_sd32(P.dM + P.exp_off[b0], P.dMs32 + 2 * P.sd32_off[b0], n, p, s);
-        else
-            launch_to_sd64(P.dM + P.exp_off[b0], P.dMs + P.sd_off[b0], n, p, s);
+        runs.push_back({b0, t.level_start[l] - b0, p, fp32});
     }
+    return runs;
 }
 
 int out_mode_of(const hfmm_plan& P, int q_type) {
@@ -1812,12 +1814,10 @@ void run_sequence(hfmm_plan& P, const void* q, int q_type, double2* out, hipStre
         launch_p2m(P.d_leafdesc, P.n_far_leaves, P.p2m_chunk, lv, P.dX, P.dY, P.dZ, P.d_q, P.k, P.p_leafmax, P.dM, s);
         mark(2);
         bool conv[kMaxLevels + 1] = {};   // levels whose multipoles are in FP32 already
-        bool conv_sd[kMaxLevels + 1] = {};   // ... in (S, D) form
         for (int L = P.depth - 1; L >= 2; --L) {
             if (P.m2mc[L].use) {
                 const M2LWaveLevel& B = P.m2mc[L];
                 level_to_sd(P, L + 1, P.dM, P.dMs, s);
-                conv_sd[L + 1] = true;
                 launch_wave(P, B, P.dMs, P.dM, 1, s);
             } else if (P.m2mb[L].use) {
                 const M2LBlockLevel& B = P.m2mb[L];
@@ -1835,7 +1835,13 @@ void run_sequence(hfmm_plan& P, const void* q, int q_type, double2* out, hipStre
                 launch_xlate(xargs(P, P.m2m[L], P.dM, P.dM, 0), P.m2m[L].n_targets, s);
         }
         mark(3);
-        levels_to_sd(P, conv_sd, s);
+        if (parts & kSeqM2LBlock)   // (a batch converts those of all its plans at once)
+            for (const LevelRun& r : sd_runs(P)) {
+                if (r.fp32)
+                    launch_to_sd32(P.dM + P.exp_off[r.b0], P.dMs32 + 2 * P.sd32_off[r.b0], r.n, r.p, s);
+                else
+                    launch_to_sd64(P.dM + P.exp_off[r.b0], P.dMs + P.sd_off[r.b0], r.n, r.p, s);
+            }
         // multipoles in FP32 for the FP32 block levels: every level not converted for an FP32
         // M2M (the converted ones need not be contiguous), one launch per run of levels
         bool any_fp32 = false;
@@ -2448,6 +2454,9 @@ struct hfmm_batch {
     };
     std::vector<M2LInstance> m2l_inst;
     std::vector<const M2LBlockArgs*> m2l_args;   // device descriptors per instance
+    const SdRun* sd_runs[2] = {};           // multipoles in (S, D) form, FP64 and FP32
+    const int2* sd_work[2] = {};
+    int sd_n[2] = {};
     const P2PArgs* d_p2p_args = nullptr;
     const NearItem* p2p_items[4] = {};     // per near-field leaf class (kP2PClass*)
     const int* p2p_prob[4] = {};
@@ -2544,6 +2553,23 @@ void build_persistent(hfmm_batch& B, void* const* out, int q_type) {
     using WaveKey = std::pair<bool, int>;   // FP32, degree
     std::map<WaveKey, std::vector<std::pair<hfmm_plan*, const M2LWaveLevel*>>> waves;
     std::map<WaveKey, int64_t> wave_groups;
+    for (int fp32 = 0; fp32 < 2; ++fp32) {
+        std::vector<SdRun> runs;
+        std::vector<int2> work;
+        for (const hfmm_plan* P : B.plans)
+            for (const LevelRun& r : sd_runs(*P)) {
+                if (r.fp32 != (bool)fp32) continue;
+                const int entries = (r.p + 1) * (r.p + 2) / 2;
+                const int64_t n = (int64_t)r.n * (fp32 ? (entries + 1) / 2 : entries);
+                for (int64_t c = 0; c * kSdChunk < n; ++c) work.push_back(make_int2((int)runs.size(), (int)c));
+                runs.push_back({P->dM + P->exp_off[r.b0],
+                                fp32 ? (void*)(P->dMs32 + 2 * P->sd32_off[r.b0]) : (void*)(P->dMs + P->sd_off[r.b0]), n,
+                                r.p + 1, 0});
+            }
+        B.sd_n[fp32] = (int)work.size();
+        B.sd_runs[fp32] = B.upload(runs);
+        B.sd_work[fp32] = B.upload(work);
+    }
     for (hfmm_plan* P : B.plans)
         for (const M2LWaveLevel& c : P->m2lc) {
             if (!c.use || !c.n_groups) continue;
@@ -2690,7 +2716,11 @@ void batch_sequence(hfmm_batch& B, const void* const* q, int q_type, void* const
     }
     mark(1);
     // the matrix-core M2L of every problem and level: persistent launches of the block
-    // kernel, the wave kernels' items
+    // kernel, the wave kernels' items.  The (S, D) form of all problems in one launch: every node of a
+    // captured graph costs some 10 us of a batch (64 problems of 30 points at p = 4: 2.2 ms with the block
+    // kernel, 2.8 with a conversion per problem).
+    launch_to_sd64_batch(B.sd_runs[0], B.sd_work[0], B.sd_n[0], s);
+    launch_to_sd32_batch(B.sd_runs[1], B.sd_work[1], B.sd_n[1], s);
     for (size_t j = 0; j < B.m2l_inst.size(); ++j) {
         const auto& in = B.m2l_inst[j];
         launch_m2l_block_persistent(B.m2l_args[j], in.q, in.grid, in.p, in.tb, in.g, in.fp32, in.shm, s);
